@@ -115,7 +115,9 @@ __device__ __forceinline__ double u01d(uint32_t hi, uint32_t lo)
 template <typename T> struct Prec;
 
 template <> struct Prec<float> {
-    __device__ static __forceinline__ float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
+    // start value of a sum of squares handed to sqrt_r2 / r_and_rinv
+    static constexpr float kR2Floor = 0.0f;
+    __device__ static __forceinline__ float sqrt_r2(float x) { return __builtin_amdgcn_sqrtf(x); }
     __device__ static __forceinline__ float rint_(float x) { return __builtin_rintf(x); }
     __device__ static __forceinline__ float floor_(float x) { return __builtin_floorf(x); }
     __device__ static __forceinline__ float rcp_(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -147,14 +149,45 @@ template <> struct Prec<float> {
 };
 
 template <> struct Prec<double> {
-    __device__ static __forceinline__ double sqrt_(double x) { return __builtin_sqrt(x); }
+    // Distances from squared distances: the general square root and divide of
+    // the compiler spend 18 and 11 vector instructions a pair on scaling,
+    // special cases and exact rounding; a squared distance needs none of the
+    // first two.  v_rsq_f64 (2^-24) and one coupled step give x^(1/2) and
+    // x^(-1/2) / 2 to 2^-46, the remainder x - g^2 (exact in an FMA) then
+    // x^(1/2) rounded as the general square root rounds it (but for results
+    // within 2^-92 of a tie), 8 instructions in all, and two more x^(-1/2)
+    // within an ulp.  Sums of squares start at kR2Floor, which no sum of a
+    // nonzero displacement notices: coincident particles get r = 2^-500 (the
+    // knot position of r = 0) and 1/r = infinity, and a NaN stays one.
+    static constexpr double kR2Floor = 0x1p-1000;
+    __device__ static __forceinline__ void rsq_step(double x, double* g, double* h)
+    {
+        const double y = __builtin_amdgcn_rsq(x);
+        *g = x * y;
+        *h = 0.5 * y;
+        const double e = __builtin_fma(-*h, *g, 0.5);
+        *g = __builtin_fma(*g, e, *g);
+        *h = __builtin_fma(*h, e, *h);
+        *g = __builtin_fma(__builtin_fma(-*g, *g, x), *h, *g);
+    }
+    __device__ static __forceinline__ double sqrt_r2(double x)
+    {
+        double g, h;
+        rsq_step(x, &g, &h);
+        return g;
+    }
     __device__ static __forceinline__ double rint_(double x) { return __builtin_rint(x); }
     __device__ static __forceinline__ double floor_(double x) { return __builtin_floor(x); }
     __device__ static __forceinline__ double rcp_(double x) { return 1.0 / x; }
     __device__ static __forceinline__ void r_and_rinv(double r2, double* r, double* rinv)
     {
-        *r = __builtin_sqrt(r2);
-        *rinv = 1.0 / *r;
+        double h;
+        rsq_step(r2, r, &h);
+        h += h;
+        h = __builtin_fma(h, __builtin_fma(-*r, h, 1.0), h);
+        // h is 2^500 here for coincident particles: infinity with its exponent raised
+        const int hi = __double2hiint(h);
+        *rinv = __hiloint2double(r2 <= 0x1p-990 ? 0x7ff00000 : hi, __double2loint(h));
     }
     __device__ static __forceinline__ void sincos_rev(double t, double* s, double* c)
     {

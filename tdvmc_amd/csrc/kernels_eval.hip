@@ -252,7 +252,7 @@ __device__ __forceinline__ void eval_pairs(const KSys& sy, const typename Coord<
 
             auto pair = [&]() {
                 T d[D];
-                T r2 = (T)0;
+                T r2 = Prec<T>::kR2Floor;
 #pragma unroll
                 for (int a = 0; a < D; a++) {
                     d[a] = C::diff(rn[a], cp[a]);
