@@ -501,9 +501,21 @@ static hipError_t launch_sweep_l(const KSys& sy, const KTables<T>& tb, const Swe
     if constexpr (!PER) {
         return hipErrorInvalidValue;   // k-space terms need the periodic box
     } else {
-        if (kpl <= 2) return launch_sweep_k<T, D, LPW, 2, PER>(sy, tb, a, st);
-        if (kpl <= 4) return launch_sweep_k<T, D, LPW, 4, PER>(sy, tb, a, st);
-        if (kpl <= 8) return launch_sweep_k<T, D, LPW, 8, PER>(sy, tb, a, st);
+        // a term past the lane's last costs what a real one does (31 issue
+        // slots of about 450 per trial in the FP32 form): every count has its
+        // kernel, but 7, which no default lane count leads to (258 terms of a
+        // 2-D system with 512 k on 64 lanes, 5 instead of 8: mixed sweep
+        // 35.2 -> 30.1 ms at 131072 walkers, N = 400)
+        switch (kpl) {
+        case 1: return launch_sweep_k<T, D, LPW, 1, PER>(sy, tb, a, st);
+        case 2: return launch_sweep_k<T, D, LPW, 2, PER>(sy, tb, a, st);
+        case 3: return launch_sweep_k<T, D, LPW, 3, PER>(sy, tb, a, st);
+        case 4: return launch_sweep_k<T, D, LPW, 4, PER>(sy, tb, a, st);
+        case 5: return launch_sweep_k<T, D, LPW, 5, PER>(sy, tb, a, st);
+        case 6: return launch_sweep_k<T, D, LPW, 6, PER>(sy, tb, a, st);
+        case 7:
+        case 8: return launch_sweep_k<T, D, LPW, 8, PER>(sy, tb, a, st);
+        }
         return hipErrorInvalidValue;
     }
 }
