@@ -463,10 +463,12 @@ int build_system(tdvmc_ctx* ctx)
     s.Kh = (int)ctx->kmap.size() / 2;
     ctx->kv_d.assign(4 * (size_t)std::max(s.Kh, 1), 0.0);
     ctx->kv_f.assign(4 * (size_t)std::max(s.Kh, 1), 0.0f);
+    s.kmax = 0;
     for (int k = 0; k < s.Kh; k++) {
         const auto& n = ns[ctx->kmap[2 * k]];
         double n2 = 0;
         for (int a = 0; a < s.D; a++) {
+            s.kmax = std::max(s.kmax, std::abs(n[a]));
             ctx->kv_d[4 * k + a] = n[a] * s.Linv;
             n2 += (double)n[a] * n[a];
         }

@@ -12,6 +12,7 @@ struct KSys {
     int N, D;
     int P_s, K, P;
     int Kh;                // k-space terms after pairing k with -k (see KTables)
+    int kmax;              // largest |component| of their integer vectors n
     int off_pair, off_k, one_body;
     int periodic;          // 1: minimum image in a box of length L
     int pot_type;          // 0 none, 1 square well, 2 Gaussian, 3 Lennard-Jones
@@ -189,10 +190,39 @@ template <> struct Prec<double> {
         const int hi = __double2hiint(h);
         *rinv = __hiloint2double(r2 <= 0x1p-990 ? 0x7ff00000 : hi, __double2loint(h));
     }
+    // Quarter turn q = rint(4 t), the remainder f = t - q / 4 in [-1/8, 1/8]
+    // (exact), the Taylor series of sin and cos in 2 pi f (truncated below
+    // 2^-54 of the result), then sine and cosine swapped and signed by q: about
+    // half of the instructions of the library's sincospi, which also treats
+    // arguments of any size.
     __device__ static __forceinline__ void sincos_rev(double t, double* s, double* c)
     {
         t = t - __builtin_rint(t);
-        sincospi(2.0 * t, s, c);
+        const double q = __builtin_rint(4.0 * t);
+        const double f = __builtin_fma(q, -0.25, t);
+        const double x = __builtin_fma(f, 0x1.921fb54442d18p+2, f * 0x1.1a62633145c07p-52);   // 2 pi in two parts
+        const double x2 = x * x;
+        double sp = -1.0 / 1307674368000.0;                                  // -1 / 15!
+        sp = __builtin_fma(sp, x2, 1.0 / 6227020800.0);
+        sp = __builtin_fma(sp, x2, -1.0 / 39916800.0);
+        sp = __builtin_fma(sp, x2, 1.0 / 362880.0);
+        sp = __builtin_fma(sp, x2, -1.0 / 5040.0);
+        sp = __builtin_fma(sp, x2, 1.0 / 120.0);
+        sp = __builtin_fma(sp, x2, -1.0 / 6.0);
+        sp = __builtin_fma(sp * x2, x, x);
+        double cp = 1.0 / 20922789888000.0;                                  // 1 / 16!
+        cp = __builtin_fma(cp, x2, -1.0 / 87178291200.0);
+        cp = __builtin_fma(cp, x2, 1.0 / 479001600.0);
+        cp = __builtin_fma(cp, x2, -1.0 / 3628800.0);
+        cp = __builtin_fma(cp, x2, 1.0 / 40320.0);
+        cp = __builtin_fma(cp, x2, -1.0 / 720.0);
+        cp = __builtin_fma(cp, x2, 1.0 / 24.0);
+        cp = __builtin_fma(cp, x2, -0.5);
+        cp = __builtin_fma(cp, x2, 1.0);
+        const int k = (int)q;                                                // -2 .. 2
+        const double a = (k & 1) ? cp : sp, b = (k & 1) ? sp : cp;
+        *s = __longlong_as_double(__double_as_longlong(a) ^ ((long long)(k & 2) << 62));
+        *c = __longlong_as_double(__double_as_longlong(b) ^ ((long long)((k + 1) & 2) << 62));
     }
     __device__ static __forceinline__ void sincos_small(double t, double* s, double* c) { sincos_rev(t, s, c); }
     __device__ static __forceinline__ double fract_(double x) { return x - __builtin_floor(x); }

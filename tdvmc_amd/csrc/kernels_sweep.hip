@@ -38,6 +38,8 @@ constexpr int kThreads = 256;
 
 template <typename T>
 struct Vec4 { T x, y, z, w; };
+template <typename T>
+struct alignas(2 * sizeof(T)) Vec2 { T x, y; };
 
 template <int LPW, typename T>
 __device__ __forceinline__ T bcast(T v, int src)
@@ -117,15 +119,15 @@ __device__ __forceinline__ T pair_u(T r, T rc, T hinv, int Ps, const Vec4<T>* sp
 }
 
 // u(r) on non-uniform knots (periodic box): cell c = min((int)(r cin), ncell-1)
-// gives the interval (j, or j + 1 past the cell's knot b) and its left knot;
+// (rows past the P_s interval rows) gives the interval (j, or j + 1 past the cell's knot b) and its left knot;
 // the piece is a cubic in s = (r - g) unitR (real length).  Row P_s - 1 of
 // spl is the constant outer-pair value beyond rc.
 template <typename T>
-__device__ __forceinline__ T pair_u_nu(T r, T cin, int cmax, T unitR, const Vec4<T>* cells, const Vec4<T>* spl)
+__device__ __forceinline__ T pair_u_nu(T r, T cin, int cmax, T unitR, int Ps, const Vec4<T>* spl)
 {
     int c = (int)(r * cin);
     c = c < cmax ? c : cmax;
-    const Vec4<T> e = cells[c];
+    const Vec4<T> e = spl[Ps + c];
     const bool right = r > e.x;
     const int j = (int)e.y + (right ? 1 : 0);
     const T s = (r - (right ? e.w : e.z)) * unitR;
@@ -146,9 +148,38 @@ __host__ __device__ inline int sweep_table_len(const KSys& sy)
     return j > sy.P_s - 1 ? j : sy.P_s - 1;
 }
 
+// Phase factors of the FP64 form: e^{ik.r} = prod_a e^{2 pi i n_a x_a}, so the
+// group tabulates e^{2 pi i m x_a}, |m| <= kmax, of two positions (a trial's
+// old and new one, or two particles while rho_k is built) in LDS, one sine and
+// cosine per lane for the 2 D kmax factors, and a k-space term takes them from
+// there with D - 1 complex products.  Two sincos per term, lane and trial took
+// 237 of about 720 vector instructions of a trial (N = 343, 128 terms, 64
+// lanes) and set the time in 2-D.  16384 walkers, 64 lanes: 7.48 -> 6.33 ms
+// (3-D, N = 343, 128 terms), 18.0 -> 8.50 ms (2-D, N = 400, 258 terms).  In 1-D
+// kmax is the number of terms and nothing is shared: each term keeps its own
+// sincos there, as where the tables would not fit the LDS or the group.
+constexpr size_t kLdsMax = 160 * 1024;
+// LDS of one workgroup without the phase tables: spline rows and coordinates
+template <typename T>
+__host__ __device__ inline size_t sweep_base_lds(const KSys& sy, int lpw)
+{
+    // coordinates: uint32 fractions (FP32, periodic) or T
+    const size_t cs = (sizeof(T) == 4 && sy.periodic) ? sizeof(uint32_t) : sizeof(T);
+    return sizeof(T) * 4 * (size_t)sweep_table_len(sy) + ((cs * (kThreads / lpw) * sy.N * sy.D + 15) & ~(size_t)15);
+}
+// entries of a walker's table: [axis][m + kmax][position], (cos, sin) each
+__host__ __device__ inline int sweep_phase_len(const KSys& sy) { return sy.D * (2 * sy.kmax + 1) * 2; }
+template <typename T>
+__host__ __device__ inline bool sweep_phase_table(const KSys& sy, int lpw)
+{
+    if (sizeof(T) == 4 || sy.D < 2 || sy.Kh == 0 || 2 * sy.D * sy.kmax > 64) return false;   // 64: factors per group
+    return sweep_base_lds<T>(sy, lpw) + (kThreads / lpw) * (size_t)sweep_phase_len(sy) * 2 * sizeof(T) <= kLdsMax;
+}
+
 // One workgroup's share of the sweep: walkers blk * WPB .. (blk + 1) * WPB - 1
-// of the system described by (sy, tb, a).
-template <typename T, int D, int LPW, int KPL, bool PER, bool NU = false>
+// of the system described by (sy, tb, a).  TAB: k-space terms from the phase
+// table (sweep_phase_table).
+template <typename T, int D, int LPW, int KPL, bool PER, bool NU = false, bool TAB = false>
 __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb, const SweepArgs& a, int64_t blk)
 {
     using C = Coord<T, PER>;
@@ -162,11 +193,12 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
     const int64_t w = blk * WPB + grp;
 
     extern __shared__ __align__(16) unsigned char smem[];
-    Vec4<T>* spl = reinterpret_cast<Vec4<T>*>(smem);                      // NT x (A0..A3) of Re u
-    Vec4<T>* kvl = spl + NT;                                               // K x (n/L, |k|^2)
-    T* all = reinterpret_cast<T*>(kvl + K);                                // K x Re alpha
-    S* posb = reinterpret_cast<S*>(all + ((K + 3) & ~3));                  // WPB x N x D (particle-major)
+    Vec4<T>* spl = reinterpret_cast<Vec4<T>*>(smem);                       // NT x (A0..A3) of Re u
+    S* posb = reinterpret_cast<S*>(spl + NT);                                                    // WPB x N x D (particle-major)
     S* pos = posb + (size_t)grp * N * D;
+    const int km = sy.kmax, prow = 2 * km + 1;                             // TAB: rows per axis
+    Vec2<T>* ptab = reinterpret_cast<Vec2<T>*>(smem + sweep_base_lds<T>(sy, LPW)) +
+                    (size_t)grp * sweep_phase_len(sy);                     // TAB: [D][prow][2]
 
     const T u_out = (T)tb.uR[sy.outer_idx];
     // real length per coordinate-difference unit
@@ -176,36 +208,20 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
         // P_s rows (the last one the outer constant), then the cells in
         // coordinate-difference units
         for (int i = tid; i < Ps; i += kThreads) {
-            spl[i].x = tb.spl[i * 8 + 0];
-            spl[i].y = tb.spl[i * 8 + 1];
-            spl[i].z = tb.spl[i * 8 + 2];
-            spl[i].w = tb.spl[i * 8 + 3];
+            const T* q = tb.spl + 8 * i;
+            spl[i] = Vec4<T>{q[0], q[1], q[2], q[3]};
         }
         for (int i = tid; i < sy.ncell; i += kThreads) {
             const double* e = tb.nucell + 4 * i;
-            spl[Ps + i].x = (T)(e[0] / unit_len);
-            spl[Ps + i].y = (T)e[1];
-            spl[Ps + i].z = (T)(e[2] / unit_len);
-            spl[Ps + i].w = (T)(e[3] / unit_len);
+            spl[Ps + i] = Vec4<T>{(T)(e[0] / unit_len), (T)e[1], (T)(e[2] / unit_len), (T)(e[3] / unit_len)};
         }
     }
     for (int i = NU ? NT : tid; i < NT; i += kThreads) {
-        if (i < Ps - 1) {
-            spl[i].x = tb.spl[i * 8 + 0];
-            spl[i].y = tb.spl[i * 8 + 1];
-            spl[i].z = tb.spl[i * 8 + 2];
-            spl[i].w = tb.spl[i * 8 + 3];
-        } else {
-            spl[i].x = u_out;
-            spl[i].y = spl[i].z = spl[i].w = (T)0;
-        }
-    }
-    for (int i = tid; i < K; i += kThreads) {
-        kvl[i].x = tb.kv[i * 4 + 0];
-        kvl[i].y = tb.kv[i * 4 + 1];
-        kvl[i].z = tb.kv[i * 4 + 2];
-        kvl[i].w = tb.kv[i * 4 + 3];
-        all[i] = tb.alpha[2 * i];
+        const T* q = tb.spl + 8 * i;
+        if (i < Ps - 1)
+            spl[i] = Vec4<T>{q[0], q[1], q[2], q[3]};
+        else
+            spl[i] = Vec4<T>{u_out, (T)0, (T)0, (T)0};
     }
     // lengths in box units when periodic (scale = 1/L), unscaled otherwise;
     // diff() and raw() return multiples of C::kUnit of that unit
@@ -219,10 +235,9 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
 
     const T hinv = (T)(sy.hinv / scale * C::kUnit), rc = (T)(sy.rc * scale / C::kUnit);
     const T cin = (T)(sy.cinv * unit_len), unitR = (T)unit_len;
-    const Vec4<T>* cells = spl + Ps;
     auto uof = [&](T r) -> T {
         if constexpr (NU)
-            return pair_u_nu<T>(r, cin, sy.ncell - 1, unitR, cells, spl);
+            return pair_u_nu<T>(r, cin, sy.ncell - 1, unitR, Ps, spl);
         else
             return pair_u<T, PER>(r, rc, hinv, Ps, spl, u_out);
     };
@@ -230,25 +245,110 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
     // one-body factor on raw coordinates: -ob sum raw^2
     const T ob = sy.one_body ? (T)(tb.uR[0] / (scale * scale) * C::kUnit * C::kUnit) : (T)0;
 
-    // this lane's k-vectors (revolutions per raw coordinate unit) and
-    // amplitudes, and twice their rho_k (sR + i sI = 2 rho_k: scaling by 2 is
-    // exact, and it saves a multiply per k and trial)
-    T sR[KPL > 0 ? KPL : 1], sI[KPL > 0 ? KPL : 1];
-    T qx[KPL > 0 ? KPL : 1], qy[KPL > 0 ? KPL : 1], qz[KPL > 0 ? KPL : 1], qa[KPL > 0 ? KPL : 1];
+    // this lane's k-vectors and amplitudes, and twice their rho_k (sR + i sI =
+    // 2 rho_k: scaling by 2 is exact, and it saves a multiply per k and trial)
+    constexpr int KP = KPL > 0 ? KPL : 1;
+    T sR[KP], sI[KP], qa[KP];
+    // TAB: the lane's rows in the phase table; otherwise revolutions per raw
+    // coordinate unit
+    T qx[KP], qy[KP], qz[KP];
+    int rx[KP], ry[KP], rz[KP];
+    // periodic: kv L is the integer lattice vector n (rounded to remove the
+    // storage error of n / L)
+    auto lattice = [&](T v) { return PER ? rint((double)v / scale) : (double)v; };
 #pragma unroll
     for (int m = 0; m < KPL; m++) {
         sR[m] = sI[m] = (T)0;
         const int k = gl + m * LPW;
         qx[m] = qy[m] = qz[m] = qa[m] = (T)0;   // lanes past K: zero amplitude, no effect
+        rx[m] = ry[m] = rz[m] = 2 * km;
         if (k < K) {
-            // periodic: kv L is the integer lattice vector n (rounded to
-            // remove the storage error of n / L)
-            const Vec4<T> q = kvl[k];
-            auto qs = [&](T v) { return (T)((PER ? rint((double)v / scale) : (double)v) * C::kUnit); };
-            qx[m] = qs(q.x);
-            qy[m] = qs(q.y);
-            qz[m] = qs(q.z);
-            qa[m] = all[k];
+            const T* q = tb.kv + 4 * k;
+            qa[m] = tb.alpha[2 * k];
+            if constexpr (TAB) {
+                rx[m] = 2 * (km + (int)lattice(q[0]));
+                ry[m] = 2 * (prow + km + (int)lattice(q[1]));
+                if (D > 2) rz[m] = 2 * (2 * prow + km + (int)lattice(q[2]));
+            } else {
+                qx[m] = (T)(lattice(q[0]) * C::kUnit);
+                qy[m] = (T)(lattice(q[1]) * C::kUnit);
+                qz[m] = (T)(lattice(q[2]) * C::kUnit);
+            }
+        }
+    }
+    // TAB: lane gl computes the factors e = gl + j LPW of (position, axis, m =
+    // 1 .. kmax): the coordinate's axis, the power, whether the position's
+    // displacement is added (as a 0 / 1 weight per axis), the rows of m and -m
+    constexpr int NE = TAB ? 64 / LPW : 1;
+    T ew[NE][3], em[NE];
+    int ea[NE], eq[NE], eplus[NE], eminus[NE];
+    const int ne = 2 * D * km;
+    if constexpr (TAB) {
+#pragma unroll
+        for (int j = 0; j < NE; j++) {
+            const int e = gl + j * LPW;
+            const bool on = e < ne;
+            const int q = on ? e / (D * km) : 0, f = on ? e - q * (D * km) : 0;
+            ea[j] = km ? f / km : 0;
+            eq[j] = q;
+            const int m = on ? f - ea[j] * km + 1 : 0;   // 0: an idle lane, writes the entry 1 of m = 0
+            em[j] = (T)m;
+            eplus[j] = 2 * (ea[j] * prow + km + m) + q;
+            eminus[j] = 2 * (ea[j] * prow + km - m) + q;
+#pragma unroll
+            for (int c = 0; c < 3; c++) ew[j][c] = (q == 1 && ea[j] == c) ? (T)1 : (T)0;
+        }
+        for (int e = gl; e < 2 * D; e += LPW) ptab[2 * ((e >> 1) * prow + km) + (e & 1)] = Vec2<T>{(T)1, (T)0};
+    }
+    // factor e^{2 pi i m x} into both rows, |x| <= 3/2; the phase is reduced
+    // before it is rounded
+    auto put = [&](int j, T x) {
+        const T t = em[j] * x;
+        T sn, cs;
+        Prec<T>::sincos_rev(__builtin_fma(em[j], x, -Prec<T>::rint_(t)), &sn, &cs);
+        ptab[eplus[j]] = Vec2<T>{cs, sn};
+        ptab[eminus[j]] = Vec2<T>{cs, -sn};
+    };
+    // e^{ik.r} of this lane's term m at position q
+    auto take = [&](int m, int q, T* re, T* im) {
+        Vec2<T> z = ptab[rx[m] + q];
+        const Vec2<T> y = ptab[ry[m] + q];
+        z = Vec2<T>{z.x * y.x - z.y * y.y, z.x * y.y + z.y * y.x};
+        if (D > 2) {
+            const Vec2<T> v = ptab[rz[m] + q];
+            z = Vec2<T>{z.x * v.x - z.y * v.y, z.x * v.y + z.y * v.x};
+        }
+        *re = z.x;
+        *im = z.y;
+    };
+    auto lds_order = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    if constexpr (TAB) {
+        // rho_k of the walker, two particles per pass
+        for (int n = 0; n < N; n += 2) {
+            lds_order();
+#pragma unroll
+            for (int j = 0; j < NE; j++)
+                if (gl + j * LPW < ne) put(j, pos[min(n + eq[j], N - 1) * D + ea[j]]);
+            lds_order();
+            const T w1 = n + 1 < N ? (T)1 : (T)0;
+#pragma unroll
+            for (int m = 0; m < KPL; m++) {
+                T c0, s0, c1, s1;
+                take(m, 0, &c0, &s0);
+                take(m, 1, &c1, &s1);
+                sR[m] += c0 + w1 * c1;
+                sI[m] += s0 + w1 * s1;
+            }
+        }
+        lds_order();
+    } else {
+#pragma unroll
+        for (int m = 0; m < KPL; m++) {
+            if (gl + m * LPW >= K) continue;
             for (int n = 0; n < N; n++) {
                 T ph = qx[m] * C::raw(pos[n * D]);
                 if (D > 1) ph += qy[m] * C::raw(pos[n * D + 1]);
@@ -258,9 +358,12 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
                 sR[m] += c;
                 sI[m] += s;
             }
-            sR[m] *= (T)2;
-            sI[m] *= (T)2;
         }
+    }
+#pragma unroll
+    for (int m = 0; m < KPL; m++) {
+        sR[m] *= (T)2;
+        sI[m] *= (T)2;
     }
     // u at distance 0: the moved particle meets itself in the partner loop
     const T u_zero = uof((T)0);
@@ -321,10 +424,26 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
             const int p = bcast_i<LPW>(pm, tt);
             S* const pp = pos + __umul24((uint32_t)p, (uint32_t)D);   // the moved particle's slot
             S old[D], nw[D];
+            Inc dz[D];
 #pragma unroll
             for (int c = 0; c < D; c++) {
                 old[c] = pp[c];
-                nw[c] = C::add(old[c], bcast<LPW>(dl[c], tt));
+                dz[c] = bcast<LPW>(dl[c], tt);
+                nw[c] = C::add(old[c], dz[c]);
+            }
+            if constexpr (TAB) {
+                // phase factors of the old and the new position (read after the
+                // partner loop); a whole box added or taken off leaves them alone
+#pragma unroll
+                for (int j = 0; j < NE; j++) {
+                    if (gl + j * LPW < ne) {
+                        T x = pp[ea[j]];
+#pragma unroll
+                        for (int c = 0; c < D; c++) x = __builtin_fma(ew[j][c], dz[c], x);
+                        put(j, x);
+                    }
+                }
+                lds_order();
             }
             const T lu = bcast<LPW>(logu, tt);
             const T us = bcast<LPW>(uself, tt);
@@ -359,19 +478,24 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
             T dR[KPL > 0 ? KPL : 1], dI[KPL > 0 ? KPL : 1];
 #pragma unroll
             for (int m = 0; m < KPL; m++) {
-                // |phase| <= sum |n_a| / 2 revolutions: no range reduction needed
-                T po = qx[m] * oc[0], pn = qx[m] * ncd[0];
-                if (D > 1) {
-                    po += qy[m] * oc[1];
-                    pn += qy[m] * ncd[1];
-                }
-                if (D > 2) {
-                    po += qz[m] * oc[2];
-                    pn += qz[m] * ncd[2];
-                }
                 T so, co, sn, cn;
-                Prec<T>::sincos_small(po, &so, &co);
-                Prec<T>::sincos_small(pn, &sn, &cn);
+                if constexpr (TAB) {
+                    take(m, 0, &co, &so);
+                    take(m, 1, &cn, &sn);
+                } else {
+                    // |phase| <= sum |n_a| / 2 revolutions: no range reduction needed
+                    T po = qx[m] * oc[0], pn = qx[m] * ncd[0];
+                    if (D > 1) {
+                        po += qy[m] * oc[1];
+                        pn += qy[m] * ncd[1];
+                    }
+                    if (D > 2) {
+                        po += qz[m] * oc[2];
+                        pn += qz[m] * ncd[2];
+                    }
+                    Prec<T>::sincos_small(po, &so, &co);
+                    Prec<T>::sincos_small(pn, &sn, &cn);
+                }
                 dR[m] = cn - co;
                 dI[m] = sn - so;
                 // |rho + d|^2 - |rho|^2 = 2 Re(conj(rho) d) + |d|^2 = Re((2 rho + d) conj(d))
@@ -403,9 +527,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
                 nacc++;
             }
             // the moved particle's LDS slot is read by every lane of the group next trial
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            lds_order();
         }
     }
 
@@ -424,17 +546,18 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
     if (gl == 0 && a.acc) a.acc[w] += nacc;
 }
 
-// FP64: scheduled for 4 wavefronts per SIMD: the LDS of the larger systems
-// allows no more, and a scheduler that aims at 5 serialises the old and the
-// new pair term to save the registers (N = 343: 7.6 against 7.5 ms).
-constexpr int sweep_least_waves(bool fp64) { return fp64 ? 4 : 1; }
+// FP64: scheduled for 4 wavefronts per SIMD (3 with many k-space terms, whose
+// sums and rows fill the registers): the LDS of the larger systems allows no
+// more, and a scheduler that aims at 5 serialises the old and the new pair
+// term to save the registers (N = 343: 7.6 against 7.5 ms).
+constexpr int sweep_least_waves(bool fp64, int kpl) { return !fp64 ? 1 : (kpl > 2 ? 3 : 4); }
 constexpr int sweep_most_waves(bool fp64) { return fp64 ? 4 : 8; }
-template <typename T, int D, int LPW, int KPL, bool PER, bool NU>
+template <typename T, int D, int LPW, int KPL, bool PER, bool NU, bool TAB>
 __global__ __launch_bounds__(kThreads)
-    __attribute__((amdgpu_waves_per_eu(sweep_least_waves(sizeof(T) == 8), sweep_most_waves(sizeof(T) == 8))))
+    __attribute__((amdgpu_waves_per_eu(sweep_least_waves(sizeof(T) == 8, KPL), sweep_most_waves(sizeof(T) == 8))))
     void sweep_kernel(KSys sy, KTables<T> tb, SweepArgs a)
 {
-    sweep_body<T, D, LPW, KPL, PER, NU>(sy, tb, a, blockIdx.x);
+    sweep_body<T, D, LPW, KPL, PER, NU, TAB>(sy, tb, a, blockIdx.x);
 }
 
 // Batch of independent systems in one launch: workgroup b belongs to system
@@ -450,7 +573,14 @@ __global__ __launch_bounds__(kThreads) void sweep_batch_kernel(SweepBatch<T> bt)
         else
             hi = mid;
     }
-    sweep_body<T, D, LPW, KPL, PER>(bt.sys[lo], bt.tab[lo], bt.args[lo], (int64_t)blockIdx.x - bt.block_start[lo]);
+    const int64_t blk = (int64_t)blockIdx.x - bt.block_start[lo];
+    if constexpr (sizeof(T) == 8 && KPL > 0 && D > 1) {
+        if (sweep_phase_table<T>(bt.sys[lo], LPW)) {
+            sweep_body<T, D, LPW, KPL, PER, false, true>(bt.sys[lo], bt.tab[lo], bt.args[lo], blk);
+            return;
+        }
+    }
+    sweep_body<T, D, LPW, KPL, PER>(bt.sys[lo], bt.tab[lo], bt.args[lo], blk);
 }
 
 // Default lanes per walker without tuning: 32 from N = 24 on (two walkers
@@ -470,11 +600,8 @@ template <typename T>
 size_t sweep_lds_bytes(const KSys& sy, int lpw)
 {
     if (lpw <= 0) lpw = pick_lpw(sy.N, sy.Kh);
-    const size_t wpb = kThreads / lpw;
-    // coordinates: uint32 fractions (FP32, periodic) or T
-    const size_t cs = (sizeof(T) == 4 && sy.periodic) ? sizeof(uint32_t) : sizeof(T);
-    return sizeof(T) * (4 * (size_t)sweep_table_len(sy) + 4 * (size_t)sy.Kh + (((size_t)sy.Kh + 3) & ~(size_t)3)) +
-           cs * wpb * sy.N * sy.D;
+    const size_t base = sweep_base_lds<T>(sy, lpw);
+    return sweep_phase_table<T>(sy, lpw) ? base + (kThreads / lpw) * (size_t)sweep_phase_len(sy) * 2 * sizeof(T) : base;
 }
 
 template <typename T, int D, int LPW, int KPL, bool PER>
@@ -482,7 +609,11 @@ static hipError_t launch_sweep_k(const KSys& sy, const KTables<T>& tb, const Swe
 {
     const size_t lds = sweep_lds_bytes<T>(sy, LPW);
     if (sy.nu && (!PER || !tb.nucell)) return hipErrorInvalidValue;
-    auto kern = sy.nu ? sweep_kernel<T, D, LPW, KPL, PER, PER> : sweep_kernel<T, D, LPW, KPL, PER, false>;
+    auto kern = sy.nu ? sweep_kernel<T, D, LPW, KPL, PER, PER, false> : sweep_kernel<T, D, LPW, KPL, PER, false, false>;
+    if constexpr (sizeof(T) == 8 && KPL > 0 && D > 1) {
+        if (sweep_phase_table<T>(sy, LPW))
+            kern = sy.nu ? sweep_kernel<T, D, LPW, KPL, PER, PER, true> : sweep_kernel<T, D, LPW, KPL, PER, false, true>;
+    }
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
