@@ -48,6 +48,7 @@ struct DevTables {
     T* kv = nullptr;
     T* alpha = nullptr;
     T* kag = nullptr;
+    T* kagr = nullptr;   // FP64 only
     bool dirty = true;
 };
 
@@ -105,7 +106,10 @@ struct tdvmc_ctx {
     std::vector<float> kv_f;          // [Kh][4] representatives
     std::vector<double> kv_d;
     std::vector<int> kmap;            // [Kh][2] parameter slots of k and -k
+    std::vector<int> kpos, krun;      // run order of the k-space terms (KTables)
     int* dKmap = nullptr;
+    int* dKpos = nullptr;
+    int* dKrun = nullptr;
 
     int64_t cap_samples = 0;
     double* dSamp = nullptr;          // [spw][W][N][D] sample configurations kept for reuse (spw > 1)
@@ -239,6 +243,40 @@ std::vector<std::vector<int>> shortest_lattice_vectors(int D, int K)
             vs.resize(K);
             return vs;
         }
+    }
+}
+
+// Run order of the vectors n[0..K): grouped by all components but the last,
+// each component in the order 0, 1, 2, ..., -1, -2, ... (outwards from 0, so
+// that a power of e^{2 pi i x} follows from the one before it); a run is a
+// stretch along the last component in steps of dir = +1 or -1.
+void kspace_runs(const std::vector<std::vector<int>>& n, int D, std::vector<int>* kpos, std::vector<int>* krun)
+{
+    const int K = (int)n.size();
+    std::vector<int> order(K);
+    for (int k = 0; k < K; k++) order[k] = k;
+    auto rank = [](int v) { return v >= 0 ? v : (1 << 20) - v; };
+    std::sort(order.begin(), order.end(), [&](int a, int b) {
+        for (int c = 0; c < D; c++)
+            if (n[a][c] != n[b][c]) return rank(n[a][c]) < rank(n[b][c]);
+        return false;
+    });
+    kpos->assign(K, 0);
+    krun->clear();
+    for (int i = 0; i < K; i++) {
+        const auto& v = n[order[i]];
+        (*kpos)[order[i]] = i;
+        bool same = !krun->empty();
+        int* r = same ? krun->data() + krun->size() - 8 : nullptr;
+        for (int c = 0; same && c < D - 1; c++) same = r[c] == v[c];
+        const int dir = v[D - 1] >= 0 ? 1 : -1;
+        if (same && r[5] == dir && v[D - 1] == r[D - 1] + dir * r[4]) {
+            r[4]++;
+            continue;
+        }
+        int h[8] = {0, 0, 0, i, 1, dir, 0, 0};
+        for (int c = 0; c < D; c++) h[c] = v[c];
+        krun->insert(krun->end(), h, h + 8);
     }
 }
 
@@ -463,6 +501,12 @@ int build_system(tdvmc_ctx* ctx)
     s.Kh = (int)ctx->kmap.size() / 2;
     ctx->kv_d.assign(4 * (size_t)std::max(s.Kh, 1), 0.0);
     ctx->kv_f.assign(4 * (size_t)std::max(s.Kh, 1), 0.0f);
+    {
+        std::vector<std::vector<int>> rep;
+        for (int k = 0; k < s.Kh; k++) rep.push_back(ns[ctx->kmap[2 * k]]);
+        kspace_runs(rep, s.D, &ctx->kpos, &ctx->krun);
+        s.nrun = (int)ctx->krun.size() / 8;
+    }
     s.kmax = 0;
     for (int k = 0; k < s.Kh; k++) {
         const auto& n = ns[ctx->kmap[2 * k]];
@@ -532,6 +576,9 @@ KTables<T> tables_of(tdvmc_ctx* ctx, DevTables<T>& t)
     k.alpha = t.alpha;
     k.kag = t.kag;
     k.kmap = ctx->dKmap;
+    k.kagr = t.kagr;
+    k.kpos = ctx->dKpos;
+    k.krun = ctx->dKrun;
     k.uR = ctx->dUR;
     k.uI = ctx->dUI;
     k.nucell = ctx->dNuCell;
@@ -543,8 +590,8 @@ template <typename T>
 int ensure_tables(tdvmc_ctx* ctx, DevTables<T>& t, bool force)
 {
     if (!t.dirty && !force) return TDVMC_OK;
-    HIPC(launch_prep_tables<T>(ctx->sy, ctx->dUR, ctx->dUI, ctx->dKmap, t.kv, t.spl, t.dspl, t.alpha, t.kag,
-                               ctx->dNuBeta, ctx->stream));
+    HIPC(launch_prep_tables<T>(ctx->sy, ctx->dUR, ctx->dUI, ctx->dKmap, ctx->dKpos, t.kv, t.spl, t.dspl,
+                               t.alpha, t.kag, t.kagr, ctx->dNuBeta, ctx->stream));
     t.dirty = false;
     return TDVMC_OK;
 }
@@ -1204,6 +1251,15 @@ int alloc_ctx(tdvmc_ctx* ctx)
     HIPC(dalloc(&ctx->dKmap, ctx->kmap.size()));
     HIPC(hipMemcpyAsync(ctx->dKmap, ctx->kmap.data(), ctx->kmap.size() * sizeof(int), hipMemcpyHostToDevice,
                         ctx->stream));
+    if (ctx->sy.Kh > 0) {
+        HIPC(dalloc(&ctx->dKpos, ctx->kpos.size()));
+        HIPC(dalloc(&ctx->dKrun, ctx->krun.size()));
+        HIPC(dalloc(&ctx->td.kagr, 8 * (size_t)K));
+        HIPC(hipMemcpyAsync(ctx->dKpos, ctx->kpos.data(), ctx->kpos.size() * sizeof(int), hipMemcpyHostToDevice,
+                            ctx->stream));
+        HIPC(hipMemcpyAsync(ctx->dKrun, ctx->krun.data(), ctx->krun.size() * sizeof(int), hipMemcpyHostToDevice,
+                            ctx->stream));
+    }
     HIPC(dalloc(&ctx->tf.spl, (size_t)Ps * 8));
     if (ctx->sy.nu) {
         HIPC(dalloc(&ctx->dNuCell, ctx->knots.cells.size()));
@@ -1273,6 +1329,8 @@ void release(tdvmc_ctx* ctx)
     dfree(ctx->dMomOut);
     dfree(ctx->dMeanCols);
     dfree(ctx->dKmap);
+    dfree(ctx->dKpos);
+    dfree(ctx->dKrun);
     dfree(ctx->tf.dspl);
     dfree(ctx->td.dspl);
     dfree(ctx->tf.kv);
@@ -1282,6 +1340,7 @@ void release(tdvmc_ctx* ctx)
     dfree(ctx->td.kv);
     dfree(ctx->td.alpha);
     dfree(ctx->td.kag);
+    dfree(ctx->td.kagr);
     dfree(ctx->dO64);
     dfree(ctx->dO32);
     dfree(ctx->dER);
@@ -1445,12 +1504,10 @@ int batch_upload(tdvmc_batch* b, int64_t n_moves, uint64_t seed, bool want_rho)
         sy[s] = c->sy;
         tf[s] = tables_of(c, c->tf);
         td[s] = tables_of(c, c->td);
-        bpf[s] = BatchParams<float>{c->sy, c->dUR, c->dUI, c->dKmap, c->tf.kv, c->tf.spl, c->tf.dspl, c->tf.alpha,
-                                    c->tf.kag, c->dX,
-                                    b->xoff[s]};
-        bpd[s] = BatchParams<double>{c->sy, c->dUR, c->dUI, c->dKmap, c->td.kv, c->td.spl, c->td.dspl, c->td.alpha,
-                                     c->td.kag, c->dX,
-                                     b->xoff[s]};
+        bpf[s] = BatchParams<float>{c->sy, c->dUR, c->dUI, c->dKmap, c->dKpos, c->tf.kv, c->tf.spl, c->tf.dspl,
+                                    c->tf.alpha, c->tf.kag, c->tf.kagr, c->dX, b->xoff[s]};
+        bpd[s] = BatchParams<double>{c->sy, c->dUR, c->dUI, c->dKmap, c->dKpos, c->td.kv, c->td.spl, c->td.dspl,
+                                     c->td.alpha, c->td.kag, c->td.kagr, c->dX, b->xoff[s]};
         const int lanes = batch_sys_lanes(b, s);
         const int wpb = sweep_walkers_per_block(lanes);
         sstart[s] = sb;

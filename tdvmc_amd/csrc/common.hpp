@@ -13,6 +13,7 @@ struct KSys {
     int P_s, K, P;
     int Kh;                // k-space terms after pairing k with -k (see KTables)
     int kmax;              // largest |component| of their integer vectors n
+    int nrun;              // runs of the k-space terms (KTables::krun)
     int off_pair, off_k, one_body;
     int periodic;          // 1: minimum image in a box of length L
     int pot_type;          // 0 none, 1 square well, 2 Gaussian, 3 Lennard-Jones
@@ -56,7 +57,11 @@ struct KTables {
     const T* kv;      // [Kh][4]: n/L of the representative (phase in revolutions = kv . r), |k|^2
     const T* alpha;   // [Kh][2]: (Re, Im) of alpha_k (+ alpha_{-k} when paired)
     const T* kag;     // [Kh][8]: Re alpha_k times (kv, |k|^2), then Im alpha_k times the same
+    const T* kagr;    // the same in run order (FP64; null otherwise)
     const int* kmap;  // [Kh][2]: parameter slots (relative to off_k) of k and of -k (-1: unpaired)
+    const int* kpos;  // [Kh]: place of term k in the run order below
+    const int* krun;  // [nrun][8]: terms start .. start + count - 1 of that order have the integer vectors n,
+                      //   n + dir e, n + 2 dir e, ... along the last axis: (n_0, n_1, n_2, start, count, dir, 0, 0)
     const double* uR; // [P + 1] parameters (FP64 master copy), then phi R
     const double* uI; // [P + 1] parameters, then phi I
     // non-uniform knots only (null otherwise); lengths in real units

@@ -10,8 +10,9 @@ namespace tdvmc {
 
 // ---- parameter-derived tables (kernels_misc.hip)
 template <typename T>
-hipError_t launch_prep_tables(const KSys& sy, const double* uR, const double* uI, const int* kmap, const T* kv, T* spl,
-                              T* dspl, T* alpha, T* kag, const double* nubeta, hipStream_t st);
+hipError_t launch_prep_tables(const KSys& sy, const double* uR, const double* uI, const int* kmap, const int* kpos,
+                              const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr, const double* nubeta,
+                              hipStream_t st);
 
 // ---- evaluation (kernels_eval.hip); grad/lap non-null selects the per-particle variant
 // LDS of one walker with wpw wavefronts (single contexts: 4)
@@ -139,11 +140,13 @@ struct BatchParams {
     double* uR;                // [P + 1] this system's parameters, then phi R (device)
     double* uI;
     const int* kmap;
+    const int* kpos;           // place of each k-space term in kagr
     const T* kv;
     T* spl;
     T* dspl;
     T* alpha;
     T* kag;
+    T* kagr;                   // or null
     double* xsys;              // [2P+2] this system's packed parameters
     int64_t xoff;              // offset of this system in the concatenated vector
 };

@@ -27,6 +27,8 @@
 // times faster than FP32 ones on this part, and FP64 sums keep O_k and the
 // gradients accurate in the mixed form.
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -574,6 +576,237 @@ __device__ __forceinline__ void eval_kgrad(const KSys& sy, const KTables<T>& tb,
     }
 }
 
+// Phase factors of the FP64 form.  A sincos is 35-odd FP64 instructions and
+// was three quarters of a (particle, k) term; e^{ik.r} = prod_a e_a^{n_a},
+// e_a = e^{2 pi i x_a}, leaves 4 for the term that follows another along the
+// last axis.  16384 walkers, whole measurement: N = 343, 128 terms (rho_k
+// handed over) 3.23 -> 2.97 ms; 2-D, N = 400, 258 terms 6.86 -> 5.73 ms.
+// Below kRunTerms terms per wavefront the D sincos of the particle and the
+// chain of a run's dependent products cost more than they save: the direct
+// form runs there (N = 25, 16 terms, 4 a wavefront: 61 against 65 us).
+constexpr int kRunTerms = 8;
+struct Cplx {
+    double x, y;
+};
+__device__ __forceinline__ Cplx cmul(Cplx a, Cplx b)
+{
+    return Cplx{__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x)};
+}
+// e^{2 pi i n x}, the phase reduced before it is rounded (|x| <= 1/2)
+__device__ __forceinline__ Cplx phase(int n, double x)
+{
+    Cplx z;
+    Prec<double>::sincos_rev(__builtin_fma((double)n, x, -__builtin_rint((double)n * x)), &z.y, &z.x);
+    return z;
+}
+// e^n for a wave-uniform n, e = e^{2 pi i x}: products where they are fewer
+// instructions than a sincos
+__device__ __forceinline__ Cplx phase_power(int n, Cplx e, double x)
+{
+    const int m = abs(n);
+    if (m > 8) return phase(n, x);
+    if (m == 0) return Cplx{1.0, 0.0};
+    const Cplx f{e.x, n < 0 ? -e.y : e.y};
+    Cplx z = f;
+    for (int i = 1; i < m; i++) z = cmul(z, f);
+    return z;
+}
+
+// eval_kgrad of the FP64 form: the terms in run order (KTables::krun), rho
+// stored in that order.  Every lane (particle) keeps the phase factors of
+// the run's leading components and steps along the last axis; which factor
+// follows from which is the same for the whole wave.
+template <int D, bool PP, bool CPLX, int NW>
+__device__ __forceinline__ void eval_kgrad_runs(const KSys& sy, const KTables<double>& tb, const double* pos,
+                                                const double* rho, double* gsum, double* lsum, int wave, int lane,
+                                                double& lap_tot_R, double& lap_tot_I)
+{
+    const int N = sy.N, K = sy.Kh;
+    const int kchunk = (K + NW - 1) / NW;
+    const int k_lo = wave * kchunk, k_hi = min(K, (wave + 1) * kchunk);
+    if (k_lo >= k_hi) return;
+    typedef const __attribute__((address_space(4))) double* CDP;
+    typedef const __attribute__((address_space(4))) int* CIP;
+    const CDP kag = (CDP)tb.kagr;
+    const CIP runs = (CIP)tb.krun;
+    double cR = 0.0, cI = 0.0;   // the constant part of the Laplacian
+    for (int k = k_lo; k < k_hi; k++) {
+        cR += kag[8 * k + 3];
+        if (CPLX) cI += kag[8 * k + 7];
+    }
+    int r0 = 0, r1 = sy.nrun;    // the last run that starts at or before k_lo
+    while (r1 - r0 > 1) {
+        const int mid = (r0 + r1) >> 1;
+        if (runs[8 * mid + 3] <= k_lo)
+            r0 = mid;
+        else
+            r1 = mid;
+    }
+    for (int rb = 0; rb < N; rb += 64) {
+        const int n = min(rb + lane, N - 1);
+        double x[D];
+        Cplx e[D];
+#pragma unroll
+        for (int a = 0; a < D; a++) {
+            x[a] = pos[a * N + n];
+            e[a] = phase(1, x[a]);
+        }
+        // lead: prod over the leading components but the last of them, then all of them
+        Cplx px{1.0, 0.0}, pre{1.0, 0.0}, z{1.0, 0.0};
+        int cx = 0, cy = 0;
+        double gR[D], gI[D];
+#pragma unroll
+        for (int a = 0; a < D; a++) gR[a] = gI[a] = 0.0;
+        double lR = 0.0, lI = 0.0;   // - sum alpha |k|^2 Re(e^{ikr} conj rho)
+        int k = k_lo;
+        for (int r = r0; k < k_hi; r++) {
+            const CIP h = runs + 8 * r;
+            const int start = h[3], end = min(k_hi, start + h[4]), dir = h[5];
+            // leading components: one step of the first moves px, of the second pre
+            if constexpr (D >= 2) {
+                const int nx = h[0];
+                bool moved = k == k_lo;
+                if (moved || nx != cx) {
+                    px = (!moved && (nx == cx + 1 || nx == cx - 1)) ? cmul(px, Cplx{e[0].x, nx > cx ? e[0].y : -e[0].y})
+                                                                   : phase_power(nx, e[0], x[0]);
+                    cx = nx;
+                    moved = true;
+                }
+                if constexpr (D == 2) {
+                    pre = px;
+                } else {
+                    const int ny = h[1];
+                    if (moved)
+                        pre = ny == 0 ? px : cmul(px, phase_power(ny, e[1], x[1]));
+                    else if (ny == cy + 1 || ny == cy - 1)
+                        pre = cmul(pre, Cplx{e[1].x, ny > cy ? e[1].y : -e[1].y});
+                    else if (ny != cy)
+                        pre = cmul(px, phase_power(ny, e[1], x[1]));
+                    cy = ny;
+                }
+            }
+            const int nl = h[D - 1] + dir * (k - start);
+            const Cplx step{e[D - 1].x, dir > 0 ? e[D - 1].y : -e[D - 1].y};
+            if (nl == 0)
+                z = pre;
+            else
+                z = D == 1 ? phase_power(nl, e[D - 1], x[D - 1]) : cmul(pre, phase_power(nl, e[D - 1], x[D - 1]));
+            while (true) {
+                const CDP ka = kag + 8 * k;
+                const double rr = rho[2 * k], ri = rho[2 * k + 1];
+                const double re = z.x * rr + z.y * ri;    // Re(e^{ikr} conj(rho))
+                const double im = z.y * rr - z.x * ri;    // Im(e^{ikr} conj(rho))
+#pragma unroll
+                for (int a = 0; a < D; a++) gR[a] += im * ka[a];
+                lR -= re * ka[3];
+                if constexpr (CPLX) {
+#pragma unroll
+                    for (int a = 0; a < D; a++) gI[a] += im * ka[4 + a];
+                    lI -= re * ka[7];
+                }
+                if (++k >= end) break;
+                z = cmul(z, step);
+            }
+        }
+        if (rb + lane >= N) continue;
+#pragma unroll
+        for (int a = 0; a < D; a++) {
+            lds_add(gsum + a * N + n, gR[a] * (-2.0 * 6.283185307179586));
+            if (CPLX) lds_add(gsum + (D + a) * N + n, gI[a] * (-2.0 * 6.283185307179586));
+        }
+        const double lapR = 2.0 * (cR + lR), lapI = 2.0 * (cI + lI);
+        if (PP) {
+            lds_add(lsum + n, lapR);
+            if (CPLX) lds_add(lsum + N + n, lapI);
+        } else {
+            lap_tot_R += lapR;
+            if (CPLX) lap_tot_I += lapI;
+        }
+    }
+}
+
+// rho_k of one walker in the FP64 form, 2-D and 3-D: the factors e_a^m of a
+// group of particles go to an LDS table [particle][axis][m + kmax], and a
+// thread multiplies D of them per particle for its term; the particles are
+// split over G threads per term where there are more threads than terms.
+// scratch: `bytes` of LDS that nothing else holds yet.  Returns false, with
+// nothing done, where the table does not fit.
+template <int D, int NT>
+__device__ __forceinline__ bool eval_rho_table(const KSys& sy, const KTables<double>& tb, const double* pos,
+                                               double* rho, double* scratch, size_t bytes, int tid,
+                                               bool run_order)
+{
+    const int N = sy.N, K = sy.Kh, km = sy.kmax, prow = 2 * km + 1;
+    constexpr int KR = NT == 256 ? 2 : (NT == 128 ? 3 : 5);   // terms per thread
+    int G = max(1, NT / K);
+    const size_t row = sizeof(Cplx) * D * prow;
+    while (G > 1 && sizeof(Cplx) * G * K + row > bytes) G--;
+    const size_t parts = G > 1 ? sizeof(Cplx) * G * K : 0;
+    if (parts + row > bytes || K > KR * NT) return false;
+    const int nb = (int)min((size_t)64, (bytes - parts) / row);   // particles per pass
+    Cplx* part = reinterpret_cast<Cplx*>(scratch);
+    Cplx* tab = part + parts / sizeof(Cplx);
+    int q[KR][D];
+    Cplx acc[KR];
+    const int g = G > 1 ? tid / K : 0;
+    const bool on = G == 1 || tid < G * K;
+#pragma unroll
+    for (int j = 0; j < KR; j++) {
+        const int k = G > 1 ? tid - g * K : tid + j * NT;
+        acc[j] = Cplx{0.0, 0.0};
+#pragma unroll
+        for (int a = 0; a < D; a++)
+            q[j][a] = a * prow + km + (on && k < K ? (int)rint(tb.kv[4 * k + a] * sy.L) : 0);
+    }
+    for (int c0 = 0; c0 < N; c0 += nb) {
+        const int nc = min(nb, N - c0);
+        __syncthreads();   // the previous pass has read the table
+        for (int f = tid; f < nc * D * (km + 1); f += NT) {
+            const int i = f / (D * (km + 1)), u = f - i * (D * (km + 1)), a = u / (km + 1), m = u - a * (km + 1);
+            const Cplx z = phase(m, pos[a * N + c0 + i]);
+            Cplx* t = tab + (i * D + a) * prow + km;
+            t[m] = z;
+            if (m > 0) t[-m] = Cplx{z.x, -z.y};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KR; j++) {
+            if (G > 1 ? (j > 0 || !on) : tid + j * NT >= K) break;
+            for (int i = g; i < nc; i += G) {
+                const Cplx* t = tab + i * (D * prow);
+                Cplx z = t[q[j][0]];
+#pragma unroll
+                for (int a = 1; a < D; a++) z = cmul(z, t[q[j][a]]);
+                acc[j].x += z.x;
+                acc[j].y += z.y;
+            }
+        }
+    }
+    if (G > 1) {
+        if (on) part[tid] = acc[0];   // [G][K]
+        __syncthreads();
+        if (tid < K) {
+            Cplx v = part[tid];
+            for (int h = 1; h < G; h++) {
+                v.x += part[h * K + tid].x;
+                v.y += part[h * K + tid].y;
+            }
+            acc[0] = v;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < KR; j++) {
+        const int k = tid + j * NT;
+        if (k < K) {
+            const int at = run_order ? tb.kpos[k] : k;
+            rho[2 * at] = acc[j].x;
+            rho[2 * at + 1] = acc[j].y;
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
 // Pairs and the k-space gradient for one value of CPLX, the potential type
 // resolved to a template argument.
 template <typename T, int D, bool PP, bool PER, bool CPLX, int NW>
@@ -704,9 +937,23 @@ __device__ __forceinline__ void eval_body(const KSys& sy, const KTables<T>& tb, 
     // ------------------------------------------------------------ rho_k
     // phase in revolutions = kq . raw coordinate, |phase| <= sum_a |n_a| / 2
     double ex_k = 0.0;
+    const bool use_runs = sizeof(T) == 8 && K >= kRunTerms * WPW;   // rho in run order, for eval_kgrad_runs
+    bool ready = false;                                              // rho holds every term
+    if constexpr (sizeof(T) == 8 && D > 1 && PER) {
+        if (K > 0 && !rho_in) {
+            // the histogram and the gradient sums lend their LDS
+            const int nd = Ps * 4 * hc + N * (cplx ? 2 : 1) * D;
+            ready = eval_rho_table<D, NT>(sy, tb, pos, rho, hist, sizeof(double) * nd, tid, use_runs);
+            for (int i = tid; ready && i < nd; i += NT) hist[i] = 0.0;
+        }
+    }
     for (int k = tid; k < K; k += NT) {
+        const int at = use_runs ? tb.kpos[k] : k;
         T re = (T)0, im = (T)0;
-        if (rho_in) {
+        if (ready) {
+            re = rho[2 * at];
+            im = rho[2 * at + 1];
+        } else if (rho_in) {
             re = rho_in[((size_t)w * K + k) * 2];
             im = rho_in[((size_t)w * K + k) * 2 + 1];
         } else {
@@ -723,8 +970,10 @@ __device__ __forceinline__ void eval_body(const KSys& sy, const KTables<T>& tb, 
                 im += sn;
             }
         }
-        rho[2 * k] = re;
-        rho[2 * k + 1] = im;
+        if (!ready) {
+            rho[2 * at] = re;
+            rho[2 * at + 1] = im;
+        }
         // O = |rho_k|^2 for k and for -k (rho_{-k} = conj rho_k)
         const double ok = (double)re * (double)re + (double)im * (double)im;
         const int m0 = tb.kmap[2 * k], m1 = tb.kmap[2 * k + 1];
@@ -740,16 +989,24 @@ __device__ __forceinline__ void eval_body(const KSys& sy, const KTables<T>& tb, 
 
     // ------------------------------------------------------------ pairs, k-space gradient / Laplacian
     double vpot = 0.0, lap_tot_R = 0.0, lap_tot_I = 0.0;
+    auto kgrad = [&](auto c) {
+        constexpr bool CP = decltype(c)::value;
+        if constexpr (sizeof(T) == 8) {
+            if (use_runs) {
+                eval_kgrad_runs<D, PP, CP, WPW>(sy, tb, pos, rho, gsum, lsum, wave, lane, lap_tot_R, lap_tot_I);
+                return;
+            }
+        }
+        eval_kgrad<T, D, PP, PER, CP, WPW>(sy, tb, pos, rho, kq, gsum, lsum, wave, lane, lap_tot_R, lap_tot_I);
+    };
     if (PP || cplx) {
         eval_forces<T, D, PP, PER, true, WPW>(sy, tb, pos, dsp, hist, gsum, lsum, wave, lane, vpot, lap_tot_R,
                                               lap_tot_I);
-        if (K > 0)
-            eval_kgrad<T, D, PP, PER, true, WPW>(sy, tb, pos, rho, kq, gsum, lsum, wave, lane, lap_tot_R, lap_tot_I);
+        if (K > 0) kgrad(std::integral_constant<bool, true>());
     } else if constexpr (!PP) {
         eval_forces<T, D, PP, PER, false, WPW>(sy, tb, pos, dsp, hist, gsum, lsum, wave, lane, vpot, lap_tot_R,
                                                lap_tot_I);
-        if (K > 0)
-            eval_kgrad<T, D, PP, PER, false, WPW>(sy, tb, pos, rho, kq, gsum, lsum, wave, lane, lap_tot_R, lap_tot_I);
+        if (K > 0) kgrad(std::integral_constant<bool, false>());
     }
     __syncthreads();
 

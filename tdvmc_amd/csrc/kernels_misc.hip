@@ -69,8 +69,8 @@ __device__ void prep_nu_interval(const KSys& sy, const double* uR, const double*
 
 template <typename T>
 __device__ void prep_tables_body(const KSys& sy, const double* __restrict__ uR, const double* __restrict__ uI,
-                                 const int* __restrict__ kmap, const T* __restrict__ kv, T* __restrict__ spl,
-                                 T* __restrict__ dspl, T* __restrict__ alpha, T* __restrict__ kag,
+                                 const int* __restrict__ kmap, const int* __restrict__ kpos,
+                                 const T* __restrict__ kv, T* __restrict__ spl, T* __restrict__ dspl, T* __restrict__ alpha, T* __restrict__ kag, T* __restrict__ kagr,
                                  const double* __restrict__ nubeta, int j0, int jstep)
 {
     const int Ps = sy.P_s;
@@ -119,9 +119,15 @@ __device__ void prep_tables_body(const KSys& sy, const double* __restrict__ uR, 
             alpha[2 * k] = (T)aR;
             alpha[2 * k + 1] = (T)aI;
             // amplitude times (n / L, |k|^2) for the k-space gradient and Laplacian
+            T* kr = kagr ? kagr + 8 * kpos[k] : nullptr;
             for (int m = 0; m < 4; m++) {
-                kag[8 * k + m] = (T)(aR * (double)kv[4 * k + m]);
-                kag[8 * k + 4 + m] = (T)(aI * (double)kv[4 * k + m]);
+                const T vR = (T)(aR * (double)kv[4 * k + m]), vI = (T)(aI * (double)kv[4 * k + m]);
+                kag[8 * k + m] = vR;
+                kag[8 * k + 4 + m] = vI;
+                if (kr) {
+                    kr[m] = vR;
+                    kr[4 + m] = vI;
+                }
             }
         }
     }
@@ -129,11 +135,11 @@ __device__ void prep_tables_body(const KSys& sy, const double* __restrict__ uR, 
 
 template <typename T>
 __global__ void prep_tables_kernel(KSys sy, const double* __restrict__ uR, const double* __restrict__ uI,
-                                   const int* __restrict__ kmap, const T* __restrict__ kv, T* __restrict__ spl,
-                                   T* __restrict__ dspl, T* __restrict__ alpha, T* __restrict__ kag,
+                                   const int* __restrict__ kmap, const int* __restrict__ kpos,
+                                   const T* __restrict__ kv, T* __restrict__ spl, T* __restrict__ dspl, T* __restrict__ alpha, T* __restrict__ kag, T* __restrict__ kagr,
                                    const double* __restrict__ nubeta)
 {
-    prep_tables_body(sy, uR, uI, kmap, kv, spl, dspl, alpha, kag, nubeta, threadIdx.x + blockIdx.x * blockDim.x,
+    prep_tables_body(sy, uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta, threadIdx.x + blockIdx.x * blockDim.x,
                      blockDim.x * gridDim.x);
 }
 
@@ -142,7 +148,7 @@ template <typename T>
 __global__ void prep_tables_batch_kernel(const BatchParams<T>* __restrict__ bp)
 {
     const BatchParams<T> b = bp[blockIdx.x];
-    prep_tables_body(b.sy, b.uR, b.uI, b.kmap, b.kv, b.spl, b.dspl, b.alpha, b.kag, nullptr, threadIdx.x,
+    prep_tables_body(b.sy, b.uR, b.uI, b.kmap, b.kpos, b.kv, b.spl, b.dspl, b.alpha, b.kag, b.kagr, nullptr, threadIdx.x,
                      blockDim.x);
 }
 
@@ -376,20 +382,23 @@ hipError_t launch_adjoint_outer(const double* outer, const double* gbar, int64_t
 }
 
 template <typename T>
-hipError_t launch_prep_tables(const KSys& sy, const double* uR, const double* uI, const int* kmap, const T* kv, T* spl,
-                              T* dspl, T* alpha, T* kag, const double* nubeta, hipStream_t st)
+hipError_t launch_prep_tables(const KSys& sy, const double* uR, const double* uI, const int* kmap, const int* kpos,
+                              const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr, const double* nubeta,
+                              hipStream_t st)
 {
     if (sy.nu && !nubeta) return hipErrorInvalidValue;
     const int n = sy.P_s - 1 + sy.Kh;
     const int blocks = (n + 255) / 256;
-    hipLaunchKernelGGL(prep_tables_kernel<T>, dim3(blocks), dim3(256), 0, st, sy, uR, uI, kmap, kv, spl, dspl, alpha,
-                       kag, nubeta);
+    hipLaunchKernelGGL(prep_tables_kernel<T>, dim3(blocks), dim3(256), 0, st, sy, uR, uI, kmap, kpos, kv, spl, dspl,
+                       alpha, kag, kagr, nubeta);
     return hipGetLastError();
 }
-template hipError_t launch_prep_tables<float>(const KSys&, const double*, const double*, const int*, const float*,
-                                              float*, float*, float*, float*, const double*, hipStream_t);
-template hipError_t launch_prep_tables<double>(const KSys&, const double*, const double*, const int*, const double*,
-                                               double*, double*, double*, double*, const double*, hipStream_t);
+template hipError_t launch_prep_tables<float>(const KSys&, const double*, const double*, const int*, const int*,
+                                              const float*, float*, float*, float*, float*, float*, const double*,
+                                              hipStream_t);
+template hipError_t launch_prep_tables<double>(const KSys&, const double*, const double*, const int*, const int*,
+                                               const double*, double*, double*, double*, double*, double*, const double*,
+                                               hipStream_t);
 
 hipError_t launch_axpy_params(int P, const double* x0, const double* xdot, double c, double* y, hipStream_t st)
 {
