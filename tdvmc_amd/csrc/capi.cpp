@@ -586,11 +586,12 @@ KTables<T> tables_of(tdvmc_ctx* ctx, DevTables<T>& t)
     return k;
 }
 
+// packed: device parameters [2P + 2] to take (null: dUR, dUI), which then are in force
 template <typename T>
-int ensure_tables(tdvmc_ctx* ctx, DevTables<T>& t, bool force)
+int ensure_tables(tdvmc_ctx* ctx, DevTables<T>& t, bool force, const double* packed = nullptr)
 {
     if (!t.dirty && !force) return TDVMC_OK;
-    HIPC(launch_prep_tables<T>(ctx->sy, ctx->dUR, ctx->dUI, ctx->dKmap, ctx->dKpos, t.kv, t.spl, t.dspl,
+    HIPC(launch_prep_tables<T>(ctx->sy, packed, ctx->dUR, ctx->dUI, ctx->dKmap, ctx->dKpos, t.kv, t.spl, t.dspl,
                                t.alpha, t.kag, t.kagr, ctx->dNuBeta, ctx->stream));
     t.dirty = false;
     return TDVMC_OK;
@@ -1032,19 +1033,17 @@ int enqueue_reuse_samples(tdvmc_ctx* ctx, int prec)
     return enqueue_moments(ctx, prec, (int64_t)ctx->spw * ctx->W);
 }
 
-int enqueue_prep(tdvmc_ctx* ctx, int prec)
+int enqueue_prep(tdvmc_ctx* ctx, int prec, const double* x)
 {
-    if (prec == TDVMC_MIXED) return ensure_tables(ctx, ctx->tf, true);
-    return ensure_tables(ctx, ctx->td, true);
+    if (prec == TDVMC_MIXED) return ensure_tables(ctx, ctx->tf, true, x);
+    return ensure_tables(ctx, ctx->td, true, x);
 }
 
 // f(x): parameters x (packed, device) -> xdot.  reuse: evaluate the kept
 // samples instead of sampling; keep: keep this stage's samples for reuse
 int enqueue_rhs(tdvmc_ctx* ctx, int prec, const double* x, double* xdot, bool reuse = false, bool keep = false)
 {
-    const int P = P_of(ctx);
-    HIPC(launch_unpack_params(P, x, ctx->dUR, ctx->dUI, ctx->stream));
-    int rc = enqueue_prep(ctx, prec);
+    int rc = enqueue_prep(ctx, prec, x);
     if (rc) return rc;
     rc = reuse ? enqueue_reuse_samples(ctx, prec) : enqueue_stage_samples(ctx, prec, ctx->seed, keep);
     if (rc) return rc;
@@ -1622,13 +1621,15 @@ int batch_measure_launch(tdvmc_batch* b, int prec)
     return TDVMC_OK;
 }
 
-int batch_prep(tdvmc_batch* b, int prec)
+int batch_prep(tdvmc_batch* b, int prec, const double* x = nullptr)
 {
     const int n = (int)b->sys.size();
+    int ps = 0;
+    for (const auto* c : b->sys) ps = std::max(ps, c->sy.P_s);
     if (prec == TDVMC_MIXED)
-        BHIPC(launch_prep_tables_batch<float>(b->dBpF, n, b->stream));
+        BHIPC(launch_prep_tables_batch<float>(b->dBpF, n, ps, x, b->stream));
     else
-        BHIPC(launch_prep_tables_batch<double>(b->dBpD, n, b->stream));
+        BHIPC(launch_prep_tables_batch<double>(b->dBpD, n, ps, x, b->stream));
     for (auto* c : b->sys) c->tf.dirty = c->td.dirty = true;
     return TDVMC_OK;
 }
@@ -1639,8 +1640,7 @@ int batch_prep(tdvmc_batch* b, int prec)
 int batch_rhs(tdvmc_batch* b, int prec, const double* x, int k, bool reuse = false)
 {
     const int n = (int)b->sys.size();
-    BHIPC(launch_unpack_batch<double>(b->dBpD, n, x, b->stream));
-    int rc = batch_prep(b, prec);
+    int rc = batch_prep(b, prec, x);
     if (rc) return rc;
     if (!reuse) {
         rc = batch_sweep_launch(b, prec);

@@ -9,10 +9,11 @@
 namespace tdvmc {
 
 // ---- parameter-derived tables (kernels_misc.hip)
+// packed: parameters [2P + 2] to take (and to copy to uR, uI first), or null: uR, uI as they are
 template <typename T>
-hipError_t launch_prep_tables(const KSys& sy, const double* uR, const double* uI, const int* kmap, const int* kpos,
-                              const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr, const double* nubeta,
-                              hipStream_t st);
+hipError_t launch_prep_tables(const KSys& sy, const double* packed, double* uR, double* uI, const int* kmap,
+                              const int* kpos, const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr,
+                              const double* nubeta, hipStream_t st);
 
 // ---- evaluation (kernels_eval.hip); grad/lap non-null selects the per-particle variant
 // LDS of one walker with wpw wavefronts (single contexts: 4)
@@ -151,7 +152,8 @@ struct BatchParams {
     int64_t xoff;              // offset of this system in the concatenated vector
 };
 template <typename T>
-hipError_t launch_prep_tables_batch(const BatchParams<T>* bp_dev, int n, hipStream_t st);
+// Ps_max: the largest P_s; x: concatenated packed parameters to take (and to copy to the systems' uR, uI), or null
+hipError_t launch_prep_tables_batch(const BatchParams<T>* bp_dev, int n, int Ps_max, const double* x, hipStream_t st);
 template <typename T>
 hipError_t launch_unpack_batch(const BatchParams<T>* bp_dev, int n, const double* x, hipStream_t st);
 template <typename T>

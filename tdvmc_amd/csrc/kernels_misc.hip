@@ -34,87 +34,107 @@ __device__ double spline_coeff(const KSys& sy, const double* u, int s)
 // in s directly (u' = A1 + 2 A2 s + 3 A3 s^2, u'' = 2 A2 + 6 A3 s).  Row P_s-1
 // of spl holds the constant beyond rc, row P_s-1 of dspl u'(rc), u''(rc).
 template <typename T>
-__device__ void prep_nu_interval(const KSys& sy, const double* uR, const double* uI, const double* beta, T* spl,
-                                 T* dspl, int j)
+__device__ void prep_nu_interval(const KSys& sy, const double* u, const double* beta, T* spl, T* dspl, int j, int part)
 {
     const int Ps = sy.P_s;
-    for (int part = 0; part < 2; part++) {
-        const double* u = (part == 0 ? uR : uI) + sy.off_pair;
-        double A[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int m = 0; m < 4; m++) {
-            const double c = spline_coeff(sy, u, j + m);
-            for (int p = 0; p < 4; p++) A[p] += c * beta[(j * 4 + m) * 4 + p];
-        }
-        for (int p = 0; p < 4; p++) spl[j * 8 + part * 4 + p] = (T)A[p];
-        T* dr = dspl + j * kDsplStride + part * 4;
-        dr[0] = (T)A[1];
-        dr[1] = (T)(2.0 * A[2]);
-        dr[2] = (T)(3.0 * A[3]);
-        dr[3] = (T)(6.0 * A[3]);
-        if (j == Ps - 2) {
-            // r = rc: the last interval at its end, s = g_{P-1} - g_{P-2}; beyond
-            // rc the outer-pair value
-            T* de = dspl + (Ps - 1) * kDsplStride + part * 4;
-            const double hl = sy.hlast;
-            de[0] = (T)(A[1] + hl * (2.0 * A[2] + hl * 3.0 * A[3]));
-            de[1] = (T)(2.0 * A[2] + 6.0 * A[3] * hl);
-            de[2] = (T)0;
-            de[3] = (T)0;
-            T* so = spl + (Ps - 1) * 8 + part * 4;
-            so[0] = (T)u[Ps - 1];
-            so[1] = so[2] = so[3] = (T)0;
-        }
+    double A[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int m = 0; m < 4; m++) {
+        const double c = spline_coeff(sy, u, j + m);
+        for (int p = 0; p < 4; p++) A[p] += c * beta[(j * 4 + m) * 4 + p];
+    }
+    for (int p = 0; p < 4; p++) spl[j * 8 + part * 4 + p] = (T)A[p];
+    T* dr = dspl + j * kDsplStride + part * 4;
+    dr[0] = (T)A[1];
+    dr[1] = (T)(2.0 * A[2]);
+    dr[2] = (T)(3.0 * A[3]);
+    dr[3] = (T)(6.0 * A[3]);
+    if (j == Ps - 2) {
+        // r = rc: the last interval at its end, s = g_{P-1} - g_{P-2}; beyond
+        // rc the outer-pair value
+        T* de = dspl + (Ps - 1) * kDsplStride + part * 4;
+        const double hl = sy.hlast;
+        de[0] = (T)(A[1] + hl * (2.0 * A[2] + hl * 3.0 * A[3]));
+        de[1] = (T)(2.0 * A[2] + 6.0 * A[3] * hl);
+        de[2] = (T)0;
+        de[3] = (T)0;
+        T* so = spl + (Ps - 1) * 8 + part * 4;
+        so[0] = (T)u[Ps - 1];
+        so[1] = so[2] = so[3] = (T)0;
     }
 }
 
 template <typename T>
-__device__ void prep_tables_body(const KSys& sy, const double* __restrict__ uR, const double* __restrict__ uI,
-                                 const int* __restrict__ kmap, const int* __restrict__ kpos,
-                                 const T* __restrict__ kv, T* __restrict__ spl, T* __restrict__ dspl, T* __restrict__ alpha, T* __restrict__ kag, T* __restrict__ kagr,
-                                 const double* __restrict__ nubeta, int j0, int jstep)
+__device__ void prep_interval(const KSys& sy, const double* u, T* spl, T* dspl, int j, int part)
 {
     const int Ps = sy.P_s;
-    for (int j = j0; j < Ps - 1 + sy.Kh; j += jstep) {
-        if (j < Ps - 1 && sy.nu) {
-            prep_nu_interval(sy, uR, uI, nubeta, spl, dspl, j);
-        } else if (j < Ps - 1) {
-            for (int part = 0; part < 2; part++) {
-                const double* u = (part == 0 ? uR : uI) + sy.off_pair;
-                const double c0 = spline_coeff(sy, u, j), c1 = spline_coeff(sy, u, j + 1);
-                const double c2 = spline_coeff(sy, u, j + 2), c3 = spline_coeff(sy, u, j + 3);
-                // u(t) on knot interval j for the four uniform cubic B-spline pieces
-                const double A1 = (c2 - c0) / 2.0, A2 = (c0 - 2.0 * c1 + c2) / 2.0;
-                const double A3 = (-c0 + 3.0 * c1 - 3.0 * c2 + c3) / 6.0;
-                spl[j * 8 + part * 4 + 0] = (T)((c0 + 4.0 * c1 + c2) / 6.0);
-                spl[j * 8 + part * 4 + 1] = (T)A1;
-                spl[j * 8 + part * 4 + 2] = (T)A2;
-                spl[j * 8 + part * 4 + 3] = (T)A3;
-                // derivatives per unit length, t = (r - knot_j) / h:
-                // u' = d1 + t (d2 + t d3), u'' = hinv (d2 + t e3)
-                const double hi = sy.hinv;
-                T* dr = dspl + j * kDsplStride + part * 4;
-                dr[0] = (T)(A1 * hi);
-                dr[1] = (T)(2.0 * A2 * hi);
-                dr[2] = (T)(3.0 * A3 * hi);
-                dr[3] = (T)(6.0 * A3 * hi);
-                if (j == Ps - 2) {
-                    // extra row for r = rc exactly (interval P_s-1, t = 0): the
-                    // values of interval P_s-2 at t = 1
-                    T* de = dspl + (Ps - 1) * kDsplStride + part * 4;
-                    de[0] = (T)((A1 + 2.0 * A2 + 3.0 * A3) * hi);
-                    de[1] = (T)((2.0 * A2 + 6.0 * A3) * hi);
-                    de[2] = (T)0;
-                    de[3] = (T)0;
-                }
-            }
+    const double c0 = spline_coeff(sy, u, j), c1 = spline_coeff(sy, u, j + 1);
+    const double c2 = spline_coeff(sy, u, j + 2), c3 = spline_coeff(sy, u, j + 3);
+    // u(t) on knot interval j for the four uniform cubic B-spline pieces
+    const double A1 = (c2 - c0) / 2.0, A2 = (c0 - 2.0 * c1 + c2) / 2.0;
+    const double A3 = (-c0 + 3.0 * c1 - 3.0 * c2 + c3) / 6.0;
+    spl[j * 8 + part * 4 + 0] = (T)((c0 + 4.0 * c1 + c2) / 6.0);
+    spl[j * 8 + part * 4 + 1] = (T)A1;
+    spl[j * 8 + part * 4 + 2] = (T)A2;
+    spl[j * 8 + part * 4 + 3] = (T)A3;
+    // derivatives per unit length, t = (r - knot_j) / h:
+    // u' = d1 + t (d2 + t d3), u'' = hinv (d2 + t e3)
+    const double hi = sy.hinv;
+    T* dr = dspl + j * kDsplStride + part * 4;
+    dr[0] = (T)(A1 * hi);
+    dr[1] = (T)(2.0 * A2 * hi);
+    dr[2] = (T)(3.0 * A3 * hi);
+    dr[3] = (T)(6.0 * A3 * hi);
+    if (j == Ps - 2) {
+        // extra row for r = rc exactly (interval P_s-1, t = 0): the
+        // values of interval P_s-2 at t = 1
+        T* de = dspl + (Ps - 1) * kDsplStride + part * 4;
+        de[0] = (T)((A1 + 2.0 * A2 + 3.0 * A3) * hi);
+        de[1] = (T)((2.0 * A2 + 6.0 * A3) * hi);
+        de[2] = (T)0;
+        de[3] = (T)0;
+    }
+}
+
+// One item per (knot interval, real or imaginary part) and per k-space term.
+// The workgroup stages the pair parameters in LDS first: read one by one where
+// an interval needs them they were 24 dependent loads of memory that the
+// solve, on another XCD, had just written (10 to 60 us a launch).
+// packed: parameters [2P + 2] to take instead of uR, uI, and to copy there.
+template <typename T>
+__device__ void prep_tables_body(const KSys& sy, const double* __restrict__ packed, double* __restrict__ uR,
+                                 double* __restrict__ uI, const int* __restrict__ kmap, const int* __restrict__ kpos,
+                                 const T* __restrict__ kv, T* __restrict__ spl, T* __restrict__ dspl,
+                                 T* __restrict__ alpha, T* __restrict__ kag, T* __restrict__ kagr,
+                                 const double* __restrict__ nubeta, double* sh, int block, int nblocks)
+{
+    const int Ps = sy.P_s, P = sy.P, tid = threadIdx.x, nt = blockDim.x;
+    const double* sR = packed ? packed : uR;
+    const double* sI = packed ? packed + P : uI;
+    for (int i = tid; i < 2 * Ps; i += nt) sh[i] = (i < Ps ? sR + sy.off_pair : sI + sy.off_pair - Ps)[i];
+    if (packed) {
+        // slot P: phi R, phi I (packed at 2P, 2P + 1)
+        for (int i = block * nt + tid; i <= P; i += nblocks * nt) {
+            uR[i] = i < P ? packed[i] : packed[2 * P];
+            uI[i] = i < P ? packed[P + i] : packed[2 * P + 1];
+        }
+    }
+    __syncthreads();
+    const int n = 2 * (Ps - 1);
+    for (int e = block * nt + tid; e < n + sy.Kh; e += nblocks * nt) {
+        if (e < n) {
+            const int part = e >= Ps - 1, j = part ? e - (Ps - 1) : e;
+            if (sy.nu)
+                prep_nu_interval(sy, sh + part * Ps, nubeta, spl, dspl, j, part);
+            else
+                prep_interval(sy, sh + part * Ps, spl, dspl, j, part);
         } else {
             // amplitude of |rho_k|^2: alpha_k, plus alpha_{-k} when -k is in the set
-            const int k = j - (Ps - 1);
+            const int k = e - n;
             const int m0 = kmap[2 * k], m1 = kmap[2 * k + 1];
-            double aR = uR[sy.off_k + m0], aI = uI[sy.off_k + m0];
+            double aR = sR[sy.off_k + m0], aI = sI[sy.off_k + m0];
             if (m1 >= 0) {
-                aR += uR[sy.off_k + m1];
-                aI += uI[sy.off_k + m1];
+                aR += sR[sy.off_k + m1];
+                aI += sI[sy.off_k + m1];
             }
             alpha[2 * k] = (T)aR;
             alpha[2 * k + 1] = (T)aI;
@@ -134,22 +154,29 @@ __device__ void prep_tables_body(const KSys& sy, const double* __restrict__ uR, 
 }
 
 template <typename T>
-__global__ void prep_tables_kernel(KSys sy, const double* __restrict__ uR, const double* __restrict__ uI,
-                                   const int* __restrict__ kmap, const int* __restrict__ kpos,
-                                   const T* __restrict__ kv, T* __restrict__ spl, T* __restrict__ dspl, T* __restrict__ alpha, T* __restrict__ kag, T* __restrict__ kagr,
-                                   const double* __restrict__ nubeta)
+__global__ __launch_bounds__(64) void prep_tables_kernel(KSys sy, const double* __restrict__ packed,
+                                                         double* __restrict__ uR, double* __restrict__ uI,
+                                                         const int* __restrict__ kmap, const int* __restrict__ kpos,
+                                                         const T* __restrict__ kv, T* __restrict__ spl,
+                                                         T* __restrict__ dspl, T* __restrict__ alpha,
+                                                         T* __restrict__ kag, T* __restrict__ kagr,
+                                                         const double* __restrict__ nubeta)
 {
-    prep_tables_body(sy, uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta, threadIdx.x + blockIdx.x * blockDim.x,
-                     blockDim.x * gridDim.x);
+    extern __shared__ __align__(16) unsigned char smem[];
+    prep_tables_body(sy, packed, uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta,
+                     reinterpret_cast<double*>(smem), blockIdx.x, gridDim.x);
 }
 
-// ---- batches of systems: one workgroup per system
+// ---- batches of systems: one workgroup per system; x: concatenated packed
+// parameters to take (null: the systems' uR, uI)
 template <typename T>
-__global__ void prep_tables_batch_kernel(const BatchParams<T>* __restrict__ bp)
+__global__ __launch_bounds__(256) void prep_tables_batch_kernel(const BatchParams<T>* __restrict__ bp,
+                                                                const double* __restrict__ x)
 {
+    extern __shared__ __align__(16) unsigned char smem[];
     const BatchParams<T> b = bp[blockIdx.x];
-    prep_tables_body(b.sy, b.uR, b.uI, b.kmap, b.kpos, b.kv, b.spl, b.dspl, b.alpha, b.kag, b.kagr, nullptr, threadIdx.x,
-                     blockDim.x);
+    prep_tables_body(b.sy, x ? x + b.xoff : nullptr, b.uR, b.uI, b.kmap, b.kpos, b.kv, b.spl, b.dspl, b.alpha, b.kag,
+                     b.kagr, nullptr, reinterpret_cast<double*>(smem), 0, 1);
 }
 
 // x (concatenated packed parameters) -> per-system uR, uI
@@ -382,23 +409,22 @@ hipError_t launch_adjoint_outer(const double* outer, const double* gbar, int64_t
 }
 
 template <typename T>
-hipError_t launch_prep_tables(const KSys& sy, const double* uR, const double* uI, const int* kmap, const int* kpos,
-                              const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr, const double* nubeta,
-                              hipStream_t st)
+hipError_t launch_prep_tables(const KSys& sy, const double* packed, double* uR, double* uI, const int* kmap,
+                              const int* kpos, const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr,
+                              const double* nubeta, hipStream_t st)
 {
     if (sy.nu && !nubeta) return hipErrorInvalidValue;
-    const int n = sy.P_s - 1 + sy.Kh;
-    const int blocks = (n + 255) / 256;
-    hipLaunchKernelGGL(prep_tables_kernel<T>, dim3(blocks), dim3(256), 0, st, sy, uR, uI, kmap, kpos, kv, spl, dspl,
-                       alpha, kag, kagr, nubeta);
+    const int n = 2 * (sy.P_s - 1) + sy.Kh;
+    hipLaunchKernelGGL(prep_tables_kernel<T>, dim3((n + 63) / 64), dim3(64), 2 * sy.P_s * sizeof(double), st, sy, packed,
+                       uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta);
     return hipGetLastError();
 }
-template hipError_t launch_prep_tables<float>(const KSys&, const double*, const double*, const int*, const int*,
+template hipError_t launch_prep_tables<float>(const KSys&, const double*, double*, double*, const int*, const int*,
                                               const float*, float*, float*, float*, float*, float*, const double*,
                                               hipStream_t);
-template hipError_t launch_prep_tables<double>(const KSys&, const double*, const double*, const int*, const int*,
-                                               const double*, double*, double*, double*, double*, double*, const double*,
-                                               hipStream_t);
+template hipError_t launch_prep_tables<double>(const KSys&, const double*, double*, double*, const int*, const int*,
+                                               const double*, double*, double*, double*, double*, double*,
+                                               const double*, hipStream_t);
 
 hipError_t launch_axpy_params(int P, const double* x0, const double* xdot, double c, double* y, hipStream_t st)
 {
@@ -430,10 +456,10 @@ hipError_t launch_unpack_params(int P, const double* packed, double* uR, double*
 }
 
 template <typename T>
-hipError_t launch_prep_tables_batch(const BatchParams<T>* bp_dev, int n, hipStream_t st)
+hipError_t launch_prep_tables_batch(const BatchParams<T>* bp_dev, int n, int Ps_max, const double* x, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(prep_tables_batch_kernel<T>, dim3(n), dim3(256), 0, st, bp_dev);
+    hipLaunchKernelGGL(prep_tables_batch_kernel<T>, dim3(n), dim3(256), 2 * Ps_max * sizeof(double), st, bp_dev, x);
     return hipGetLastError();
 }
 template <typename T>
@@ -450,8 +476,10 @@ hipError_t launch_gather_batch(const BatchParams<T>* bp_dev, int n, double* x, i
     hipLaunchKernelGGL(gather_batch_kernel<T>, dim3(n), dim3(256), 0, st, bp_dev, x, to_batch);
     return hipGetLastError();
 }
-template hipError_t launch_prep_tables_batch<float>(const BatchParams<float>*, int, hipStream_t);
-template hipError_t launch_prep_tables_batch<double>(const BatchParams<double>*, int, hipStream_t);
+template hipError_t launch_prep_tables_batch<float>(const BatchParams<float>*, int, int, const double*,
+                                                    hipStream_t);
+template hipError_t launch_prep_tables_batch<double>(const BatchParams<double>*, int, int, const double*,
+                                                     hipStream_t);
 template hipError_t launch_unpack_batch<double>(const BatchParams<double>*, int, const double*, hipStream_t);
 template hipError_t launch_gather_batch<double>(const BatchParams<double>*, int, double*, int, hipStream_t);
 

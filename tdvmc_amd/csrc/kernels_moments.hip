@@ -252,11 +252,20 @@ __global__ __launch_bounds__(64) void gemm64_kernel(const double* __restrict__ x
     const double* A = xt + (size_t)I * ksteps * 64;
     const double* B = xt + (size_t)J * ksteps * 64;
     double4v acc = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t s = s0; s < s1; s++) {
-        const double a = A[s * 64 + lane];
-        const double b = B[s * 64 + lane];
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+    // 8 k-steps' operands in flight: one step at a time the products waited
+    // for memory
+    int64_t s = s0;
+    for (; s + 8 <= s1; s += 8) {
+        double a[8], b[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            a[q] = A[(s + q) * 64 + lane];
+            b[q] = B[(s + q) * 64 + lane];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[q], acc, 0, 0, 0);
     }
+    for (; s < s1; s++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[s * 64 + lane], B[s * 64 + lane], acc, 0, 0, 0);
     // D[i][j]: j = lane % 16, i = 4 v + lane / 16
     double* out = partial + (((size_t)g * ntiles + t) * 256);
 #pragma unroll
@@ -315,40 +324,179 @@ __global__ __launch_bounds__(64) void gemm_bf16x6_kernel(const __bf16* __restric
     for (int v = 0; v < 16; v++) out[(8 * (v / 4) + 4 * (lane / 32) + (v % 4)) * 32 + (lane % 32)] = acc64[v];
 }
 
-// ---- pass 4: sum slices, scale 1/W, scatter to S (both triangles) and F
-__global__ void reduce_tiles_kernel(const double* __restrict__ partial, int ntiles, int nb, int tile, int groups,
-                                    int P, int64_t W, const int* __restrict__ outmap, int P_full,
-                                    double* __restrict__ S, double* __restrict__ F)
+// s = cov(computed columns i, j), i <= j, to every full index: S (both
+// triangles) for two operators, F for an operator and an energy
+__device__ __forceinline__ void store_cov(double s, int i, int j, int P, const int* __restrict__ outmap, int P_full,
+                                          double* __restrict__ S, double* __restrict__ F)
+{
+    // full indices of computed columns i and j (one, or two for a folded group)
+    int fi[2] = {i, -1}, fj[2] = {j, -1};
+    if (outmap) {
+        if (i < P) fi[0] = outmap[2 * i], fi[1] = outmap[2 * i + 1];
+        if (j < P) fj[0] = outmap[2 * j], fj[1] = outmap[2 * j + 1];
+    }
+    if (i < P && j < P) {
+        for (int a = 0; a < 2; a++)
+            for (int b = 0; b < 2; b++)
+                if (fi[a] >= 0 && fj[b] >= 0) {
+                    S[(size_t)fi[a] * P_full + fj[b]] = s;
+                    S[(size_t)fj[b] * P_full + fi[a]] = s;
+                }
+    } else if (i < P && (j == P || j == P + 1)) {
+        for (int a = 0; a < 2; a++)
+            if (fi[a] >= 0) F[(size_t)(j - P) * P_full + fi[a]] = s;
+    }
+}
+
+// ---- pass 4: sum slices, scale 1/W, scatter to S (both triangles) and F.
+// One tile element per thread, its slices loaded 16 at a time and added in
+// order: with 4 elements per thread and one load at a time the latency of 128
+// loads was 18 to 37 us (W = 8192 .. 131072).
+__global__ __launch_bounds__(256) void reduce_tiles_kernel(const double* __restrict__ partial, int ntiles, int nb,
+                                                           int tile, int groups, int P, int64_t W,
+                                                           const int* __restrict__ outmap, int P_full,
+                                                           double* __restrict__ S, double* __restrict__ F)
 {
     const int t = blockIdx.x;
     int I, J;
     tile_of(t, nb, &I, &J);
     const int tt = tile * tile;
-    const double inv = 1.0 / (double)W;
-    for (int e = threadIdx.x; e < tt; e += blockDim.x) {
-        // diagonal tiles: take the upper element for both triangles
-        if (I == J && e / tile > e % tile) continue;
+    const int e = blockIdx.y * 256 + threadIdx.x;   // tt is a multiple of 256
+    // diagonal tiles: take the upper element for both triangles
+    if (I == J && e / tile > e % tile) return;
+    const double* p = partial + (size_t)t * tt + e;
+    const size_t stride = (size_t)ntiles * tt;
+    double s = 0.0;
+#pragma unroll 16
+    for (int g = 0; g < groups; g++) s += p[g * stride];
+    s *= 1.0 / (double)W;
+    store_cov(s, I * tile + e / tile, J * tile + e % tile, P, outmap, P_full, S, F);
+}
+
+// ---- few columns, few walkers (FP64): two launches instead of five.
+// Workgroup c centres a chunk of kSmallRows walkers on the chunk's own means
+// in LDS and forms its products on FP64 MFMA; the second kernel combines the
+// chunks by the parallel-variance formula, sum_c (M_c + n_c d_c d_c^T) with
+// d_c = mean_c - mean, so nothing is subtracted that is larger than the
+// spread of the samples.
+constexpr int kSmallRows = 64, kSmallCols = 64, kSmallChunks = 512;
+
+inline bool moments_small(int64_t W, int P, int mode)
+{
+    // sums, means, packing, products and reduction are a launch each, 41 to
+    // 62 us together at these sizes whatever the work; the two launches take
+    // 12 us (16 columns, 1024 walkers) to 25 us (34 columns, 16384 walkers).
+    // More columns or chunks would outgrow the LDS of the combination.
+    return mode == 0 && P + 2 <= kSmallCols && W <= (int64_t)kSmallRows * kSmallChunks;
+}
+inline int small_chunks(int64_t W) { return (int)ceil_div(W, kSmallRows); }
+
+template <typename TO>
+__global__ __launch_bounds__(256) void small_partial_kernel(const TO* __restrict__ O, const double* __restrict__ ER,
+                                                            const double* __restrict__ EI, int64_t W, int P, ColSrc cs,
+                                                            int nb, double* __restrict__ mean, double* __restrict__ part)
+{
+    // rows 16 doubles apart from a multiple of 32 banks' width: the 4 rows of
+    // an MFMA operand sit in different banks
+    constexpr int LD = kSmallCols + 4;
+    __shared__ double X[kSmallRows * LD];
+    __shared__ double m[4][kSmallCols];
+    const int tid = threadIdx.x, Pa = P + 2, Pp = nb * 16;
+    const int64_t w0 = (int64_t)blockIdx.x * kSmallRows;
+    const int n = (int)min((int64_t)kSmallRows, W - w0);
+    const int c = tid & 63, q = tid >> 6;   // this thread's column and rows q, q + 4, ...
+    const int oc = c < P ? cs(c) : 0;
+    double v[kSmallRows / 4];
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < kSmallRows / 4; i++) {
+        const int64_t w = w0 + q + 4 * i;
+        v[i] = 0.0;
+        if (q + 4 * i < n && c < Pa) v[i] = c < P ? (double)O[w * cs.ld + oc] : (c == P ? ER[w] : EI[w]);
+    }
+#pragma unroll
+    for (int i = 0; i < kSmallRows / 4; i++) s += v[i];
+    m[q][c] = s;
+    __syncthreads();
+    const double mc = (((m[0][c] + m[1][c]) + m[2][c]) + m[3][c]) / (double)n;
+    if (q == 0 && c < Pa) mean[(size_t)blockIdx.x * Pa + c] = mc;
+#pragma unroll
+    for (int i = 0; i < kSmallRows / 4; i++)
+        if (c < Pp) X[(q + 4 * i) * LD + c] = (q + 4 * i < n && c < Pa) ? v[i] - mc : 0.0;
+    __syncthreads();
+    const int lane = tid & 63, pp = lane & 15, kk = lane >> 4;
+    const int ntiles = nb * (nb + 1) / 2;
+    for (int t = q; t < ntiles; t += 4) {
+        int I, J;
+        tile_of(t, nb, &I, &J);
+        double4v acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < kSmallRows; k += 4)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(X[(k + kk) * LD + 16 * I + pp], X[(k + kk) * LD + 16 * J + pp], acc,
+                                                       0, 0, 0);
+        double* out = part + ((size_t)blockIdx.x * ntiles + t) * 256;
+#pragma unroll
+        for (int u = 0; u < 4; u++) out[(4 * u + kk) * 16 + pp] = acc[u];
+    }
+}
+
+__global__ __launch_bounds__(1024) void small_combine_kernel(const double* __restrict__ cmean,
+                                                             const double* __restrict__ part, int chunks, int64_t W,
+                                                             int P, int nb, const int* __restrict__ outmap, int P_full,
+                                                             double* __restrict__ mean, double* __restrict__ S,
+                                                             double* __restrict__ F)
+{
+    __shared__ double cm[kSmallChunks * 32];   // chunk means of the tile's 16 + 16 columns
+    __shared__ double red[1024];
+    __shared__ double mt[32];
+    const int t = blockIdx.x, tid = threadIdx.x, Pa = P + 2, ntiles = gridDim.x;
+    int I, J;
+    tile_of(t, nb, &I, &J);
+    auto rows = [&](int k) { return (double)min((int64_t)kSmallRows, W - (int64_t)k * kSmallRows); };
+    // total means of the 32 columns: 32 strided sums each, then a fixed tree
+    {
+        const int u = tid & 31, col = u < 16 ? 16 * I + u : 16 * J + u - 16;
         double s = 0.0;
-        for (int g = 0; g < groups; g++) s += partial[((size_t)g * ntiles + t) * tt + e];
-        s *= inv;
-        const int i = I * tile + e / tile, j = J * tile + e % tile;
-        // full indices of computed columns i and j (one, or two for a folded group)
-        int fi[2] = {i, -1}, fj[2] = {j, -1};
-        if (outmap) {
-            if (i < P) fi[0] = outmap[2 * i], fi[1] = outmap[2 * i + 1];
-            if (j < P) fj[0] = outmap[2 * j], fj[1] = outmap[2 * j + 1];
+#pragma unroll 4
+        for (int k = tid >> 5; k < chunks; k += 32) {
+            const double v = col < Pa ? cmean[(size_t)k * Pa + col] : 0.0;
+            cm[k * 32 + u] = v;
+            s += rows(k) * v;
         }
-        if (i < P && j < P) {
-            for (int a = 0; a < 2; a++)
-                for (int b = 0; b < 2; b++)
-                    if (fi[a] >= 0 && fj[b] >= 0) {
-                        S[(size_t)fi[a] * P_full + fj[b]] = s;
-                        S[(size_t)fj[b] * P_full + fi[a]] = s;
-                    }
-        } else if (i < P && (j == P || j == P + 1)) {
-            for (int a = 0; a < 2; a++)
-                if (fi[a] >= 0) F[(size_t)(j - P) * P_full + fi[a]] = s;
+        red[tid] = s;
+        __syncthreads();
+        for (int o = 16; o > 0; o >>= 1) {
+            if ((tid >> 5) < o) red[tid] += red[tid + 32 * o];
+            __syncthreads();
         }
+        if (tid < 32) {
+            const double m = red[tid] / (double)W;
+            mt[tid] = m;
+            // the diagonal tiles hold every column once
+            if (I == J && tid < 16 && col < Pa) {
+                if (col >= P)
+                    mean[P_full + (col - P)] = m;
+                else if (!outmap)
+                    mean[col] = m;
+                else
+                    for (int k = 0; k < 2; k++)
+                        if (outmap[2 * col + k] >= 0) mean[outmap[2 * col + k]] = m;
+            }
+        }
+        __syncthreads();
+    }
+    // element (i, j) of the tile: chunks tid / 256, + 4, ..., then the four sums
+    const int e = tid & 255, i = e >> 4, j = e & 15;
+    const double mi = mt[i], mj = mt[16 + j];
+    double s = 0.0;
+#pragma unroll 8
+    for (int k = tid >> 8; k < chunks; k += 4)
+        s += part[((size_t)k * ntiles + t) * 256 + e] + rows(k) * (cm[k * 32 + i] - mi) * (cm[k * 32 + 16 + j] - mj);
+    red[tid] = s;
+    __syncthreads();
+    if (tid < 256 && !(I == J && i > j)) {
+        s = ((red[e] + red[256 + e]) + red[512 + e]) + red[768 + e];
+        store_cov(s * (1.0 / (double)W), 16 * I + i, 16 * J + j, P, outmap, P_full, S, F);
     }
 }
 
@@ -363,6 +511,8 @@ void moments_work_bytes(int64_t W, int P, int mode, size_t* xt, size_t* partial,
         *xt = (size_t)g.Wp * g.Pp * kSplit * sizeof(__bf16);
     *partial = (size_t)g.groups * g.ntiles * g.tile * g.tile * sizeof(double);
     *colsum = (size_t)g.chunks * g.Pa * sizeof(double);
+    // (a chunk of the small form is a column-sum chunk: kSmallRows == kChunkRows)
+    if (moments_small(W, P, mode)) *partial = (size_t)small_chunks(W) * g.ntiles * 256 * sizeof(double);
 }
 
 template <typename TO>
@@ -381,6 +531,14 @@ hipError_t launch_moments(const TO* O, const double* ER, const double* EI, int64
     moments_work_bytes(W, Pc, mode, &xb, &pb, &cb);
     if (wk.xt_bytes < xb || wk.partial_bytes < pb || wk.colsum_bytes < cb) return hipErrorInvalidValue;
 
+    if (moments_small(W, Pc, mode)) {
+        const int chunks = small_chunks(W);
+        hipLaunchKernelGGL(small_partial_kernel<TO>, dim3(chunks), dim3(256), 0, st, O, ER, EI, W, Pc, cs, g.nb, wk.colsum,
+                           wk.partial);
+        hipLaunchKernelGGL(small_combine_kernel, dim3(g.ntiles), dim3(1024), 0, st, wk.colsum, wk.partial, chunks, W, Pc,
+                           g.nb, wk.outmap, P, mean, S, F);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(colsum_kernel<TO>, dim3((unsigned)ceil_div(g.Pa, kColBlock), g.chunks), dim3(kColBlock), 0, st,
                        O, ER, EI, W, Pc, cs, g.chunks, wk.colsum);
     hipLaunchKernelGGL(colmean_kernel, dim3((unsigned)g.Pa), dim3(256), 0, st, wk.colsum, g.chunks, g.Pa, W, mc,
@@ -402,7 +560,7 @@ hipError_t launch_moments(const TO* O, const double* ER, const double* EI, int64
         hipLaunchKernelGGL(gemm_bf16x6_kernel, dim3(g.ntiles * g.groups), dim3(64), 0, st,
                            static_cast<const __bf16*>(wk.xt), g.ksteps, g.nb, g.groups, wk.partial);
     }
-    hipLaunchKernelGGL(reduce_tiles_kernel, dim3(g.ntiles), dim3(256), 0, st, wk.partial, g.ntiles, g.nb, g.tile,
+    hipLaunchKernelGGL(reduce_tiles_kernel, dim3(g.ntiles, g.tile * g.tile / 256), dim3(256), 0, st, wk.partial, g.ntiles, g.nb, g.tile,
                        g.groups, Pc, W, wk.outmap, P, S, F);
     return hipGetLastError();
 }
