@@ -26,6 +26,8 @@ SOURCES = [
     "writer.cpp",
     "knots.cpp",
     "kernels_eval.hip",
+    "kernels_eval_fp64.hip",
+    "kernels_eval_batch.hip",
     "kernels_sweep.hip",
     "kernels_moments.hip",
     "kernels_solve.hip",

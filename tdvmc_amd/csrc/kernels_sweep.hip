@@ -604,6 +604,24 @@ size_t sweep_lds_bytes(const KSys& sy, int lpw)
     return sweep_phase_table<T>(sy, lpw) ? base + (kThreads / lpw) * (size_t)sweep_phase_len(sy) * 2 * sizeof(T) : base;
 }
 
+// Default lanes per walker of a single system.  Mixed form: pick_lpw (its FP32
+// sums, and with them rare decisions, depend on the lane count).  FP64: the
+// fewest lanes, which share a trial's overhead among the most walkers, that
+// still leave two wavefronts for every SIMD and the LDS room for three
+// workgroups per CU.  Sweep in us with 16 / 32 / 64 lanes: N = 64, 16384 / 2048
+// / 512 walkers 209 / 233 / 264, 82 / 55 / 49, 77 / 51 / 35; N = 100 (2-D), 8192
+// / 1024 walkers 251 / 259 / 278, 154 / 104 / 66; N = 125, 60 k, 8192 walkers
+// (2, 5 and 8 workgroups by LDS) 561 / 510 / 614; N = 343, 256 k, 512 walkers
+// 3147 / 1294 / 769.
+template <typename T>
+static int default_lanes(const KSys& sy, int64_t W)
+{
+    if (sizeof(T) == 4) return pick_lpw(sy.N, sy.Kh);
+    for (int l = 16; l < 64; l *= 2)
+        if (sy.Kh <= 8 * l && W * l >= 64 * 2048 && sweep_lds_bytes<T>(sy, l) <= kLdsMax / 3) return l;
+    return 64;
+}
+
 template <typename T, int D, int LPW, int KPL, bool PER>
 static hipError_t launch_sweep_k(const KSys& sy, const KTables<T>& tb, const SweepArgs& a, hipStream_t st)
 {
@@ -654,7 +672,7 @@ static hipError_t launch_sweep_l(const KSys& sy, const KTables<T>& tb, const Swe
 template <typename T, int D>
 static hipError_t launch_sweep_d(const KSys& sy, const KTables<T>& tb, const SweepArgs& a, hipStream_t st)
 {
-    const int lpw = a.lanes_per_walker > 0 ? a.lanes_per_walker : pick_lpw(sy.N, sy.Kh);
+    const int lpw = a.lanes_per_walker > 0 ? a.lanes_per_walker : default_lanes<T>(sy, a.W);
     const bool per = sy.periodic != 0;
     switch (lpw) {
     case 16: return per ? launch_sweep_l<T, D, 16, true>(sy, tb, a, st) : launch_sweep_l<T, D, 16, false>(sy, tb, a, st);
