@@ -161,6 +161,9 @@ struct tdvmc_ctx {
         std::vector<double> scale, centres, kgrid;
         int* dVec = nullptr;                  // [V][4]
         int* dOff = nullptr;                  // [nshell + 1]
+        int npair = 0;
+        int* dPairs = nullptr;                // [npair][2]
+        double* dThr = nullptr;               // [count + 1]
         double* dScale = nullptr;             // [count]
         unsigned long long* dTot = nullptr;   // [count]
         double* dSkAcc = nullptr;             // [nshell]
@@ -856,6 +859,48 @@ int enqueue_solve(tdvmc_ctx* ctx, double* xdot)
 constexpr int kObsShells = 50;
 constexpr int kObsMaxBins = 8192;
 
+// Segments per row of g(r)'s pair loop: enough work items for the workgroup's
+// 256 threads twice, and the count whose last round of items and last partner
+// of a segment are fullest (N = 343: 8 segments keep 95 % of the lanes busy, the
+// 2 that 512 items need 89 %).
+int gr_segments(int N)
+{
+    const int M = N / 2;   // partners of a row
+    const int least = std::max(1, std::min(M, (512 + N - 1) / N));
+    int best = least;
+    double eff = 0.0;
+    for (int s = least; s <= std::min(M, least + 10); s++) {
+        const double items = (double)N * s;
+        const double e = items / (256.0 * std::ceil(items / 256.0)) * M / (s * std::ceil((double)M / s));
+        if (e > eff + 0.01) {
+            eff = e;
+            best = s;
+        }
+    }
+    return best;
+}
+
+// Bin b of g(r) holds the squared distances s with thr[b] <= s < thr[b + 1]:
+// thr[b] is the smallest s whose floor(sqrt(s) / spacing) reaches b, thr[count]
+// the smallest that r < gmax or the bin count leaves out (both are monotone in
+// s, each operation being rounded to nearest).
+std::vector<double> gr_thresholds(double gmax, double spacing, int count)
+{
+    std::vector<double> thr(count + 1, 0.0);
+    for (int b = 1; b <= count; b++) {
+        auto reached = [&](double s) {
+            const double r = std::sqrt(s);
+            return std::floor(r / spacing) >= b || (b == count && !(r < gmax));
+        };
+        double s = b * spacing;
+        s *= s;
+        while (!reached(s)) s = std::nextafter(s, 1e300);
+        while (reached(std::nextafter(s, 0.0))) s = std::nextafter(s, 0.0);
+        thr[b] = s;
+    }
+    return thr;
+}
+
 int ensure_obs(tdvmc_ctx* ctx)
 {
     auto& o = ctx->obs;
@@ -928,6 +973,22 @@ int ensure_obs(tdvmc_ctx* ctx)
         ctx->err = "too many S(k) wave vectors";
         return TDVMC_ERR_BAD_CONFIG;
     }
+    // distinct leading components (all but the last) of the vectors
+    std::vector<int> pairs;
+    for (int v = 0; D > 1 && v < o.V; v++) {
+        const int x = vec[4 * v], y = D > 2 ? vec[4 * v + 1] : 0;
+        size_t p = 0;
+        while (p < pairs.size() && (pairs[p] != x || pairs[p + 1] != y)) p += 2;
+        if (p == pairs.size()) pairs.insert(pairs.end(), {x, y});
+        vec[4 * v + 3] = (int)(p / 2);
+    }
+    o.npair = (int)pairs.size() / 2;
+    const std::vector<double> thr = gr_thresholds(o.gmax, o.spacing, o.count);
+    HIPC(dalloc(&o.dPairs, pairs.size()));
+    HIPC(dalloc(&o.dThr, thr.size()));
+    if (!pairs.empty())
+        HIPC(hipMemcpyAsync(o.dPairs, pairs.data(), pairs.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+    HIPC(hipMemcpyAsync(o.dThr, thr.data(), thr.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     HIPC(dalloc(&o.dVec, vec.size()));
     HIPC(dalloc(&o.dOff, off.size()));
     HIPC(dalloc(&o.dScale, (size_t)o.count));
@@ -950,7 +1011,11 @@ int enqueue_obs(tdvmc_ctx* ctx, int prec, const double* dR, int64_t W, double* g
     const bool f32 = prec == TDVMC_MIXED;
     const size_t cx = f32 ? 2 * sizeof(float) : 2 * sizeof(double);
     const int chunk = (int)std::min<size_t>(64, std::max<size_t>(1, 24576 / ((size_t)D * (o.nmax + 1) * cx)));
-    const size_t lds = obs_lds_bytes(N, D, o.V, chunk, o.nmax, o.count, f32);
+    // FP64 in 2-D and 3-D: the matrix-product form where its LDS fits (and the
+    // squared distances fit an FP32 guess)
+    const size_t mfma = f32 || o.gmax < 1e-12 || o.gmax > 1e12 ? 0 : obs_mfma_lds_bytes(N, D, chunk, o.nmax, o.count, o.npair);
+    const bool use_mfma = mfma > 0 && mfma <= 65536;
+    const size_t lds = use_mfma ? mfma : obs_lds_bytes(N, D, o.V, chunk, o.nmax, o.count, f32);
     if (lds > 65536) {
         ctx->err = "g(r) / S(k) need " + std::to_string(lds) + " bytes of LDS per walker (at most 65536)";
         return TDVMC_ERR_BAD_ARG;
@@ -968,18 +1033,23 @@ int enqueue_obs(tdvmc_ctx* ctx, int prec, const double* dR, int64_t W, double* g
     a.gr_tot = o.dTot;
     a.gr_w = gr_w;
     a.kvec = o.dVec;
+    a.pairs = o.dPairs;
+    a.npair = o.npair;
+    a.thr = o.dThr;
     a.shell_off = o.dOff;
     a.V = o.V;
     a.nshell = o.nshell;
     a.nmax = o.nmax;
     a.chunk = chunk;
-    a.gr_segs = std::max(1, std::min((N - 1) / 2 + 1, (512 + N - 1) / N));
+    a.gr_segs = gr_segments(N);
     a.sk_w = sk_w;
     hipEvent_t ev{};
     int rc = prof_begin(ctx, "observables", &ev);
     if (rc) return rc;
     if (f32) {
         HIPC(launch_obs<float>(a, D, lds, ctx->stream));
+    } else if (use_mfma) {
+        HIPC(launch_obs_mfma(a, D, lds, ctx->stream));
     } else {
         HIPC(launch_obs<double>(a, D, lds, ctx->stream));
     }
@@ -1298,6 +1368,8 @@ void release(tdvmc_ctx* ctx)
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     dfree(ctx->obs.dVec);
     dfree(ctx->obs.dOff);
+    dfree(ctx->obs.dPairs);
+    dfree(ctx->obs.dThr);
     dfree(ctx->obs.dScale);
     dfree(ctx->obs.dTot);
     dfree(ctx->obs.dSkAcc);

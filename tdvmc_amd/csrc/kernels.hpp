@@ -219,7 +219,11 @@ struct ObsArgs {
     const double* scale;            // [count] (D / (N-1)) / scaling[bin]
     unsigned long long* gr_tot;     // [count] pair counts summed over walkers (atomics)
     double* gr_w;                   // [W][count] per-walker g(r), or null
-    const int* kvec;                // [V][4] integer wave vectors n (components 0..D-1)
+    const int* kvec;                // [V][4] integer wave vectors n (components 0..D-1), then the
+                                    //   leading components' place in pairs (D > 1)
+    const int* pairs;               // [npair][2] distinct leading components (D > 1; the second 0 in 2-D)
+    int npair;
+    const double* thr;              // [count + 1] smallest squared distance of each bin, then of none
     const int* shell_off;           // [nshell + 1] first vector of each shell
     int V, nshell, nmax;            // vectors, shells, largest component
     int chunk;                      // particles per LDS phase table
@@ -227,6 +231,10 @@ struct ObsArgs {
     double* sk_w;                   // [W][nshell] per-walker S(k)
 };
 size_t obs_lds_bytes(int N, int D, int V, int chunk, int nmax, int count, bool fp32);
+// FP64 in 2-D and 3-D: S(k) as a matrix product, bins from thresholds; its LDS,
+// or 0 where it does not take the shape
+size_t obs_mfma_lds_bytes(int N, int D, int chunk, int nmax, int count, int npair);
+hipError_t launch_obs_mfma(const ObsArgs& a, int D, size_t lds, hipStream_t st);
 template <typename T>
 hipError_t launch_obs(const ObsArgs& a, int D, size_t lds, hipStream_t st);
 // acc[s] += sum_w sk_w[w][s] (fixed order)
