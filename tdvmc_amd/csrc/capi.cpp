@@ -54,6 +54,8 @@ struct DevTables {
 
 }  // namespace
 
+struct tdvmc_batch;
+
 struct tdvmc_ctx {
     Config cfg;
     KSys sy{};
@@ -124,6 +126,12 @@ struct tdvmc_ctx {
     double* dMean = nullptr;
     double* dS = nullptr;
     double* dF = nullptr;
+    // kept by the host-pointer entry points between calls (Arena)
+    double* ws_dev = nullptr;
+    double* ws_pin = nullptr;
+    size_t ws_dev_cap = 0, ws_pin_cap = 0;   // doubles
+    tdvmc_batch* batch = nullptr;            // the batch this context is a member of
+    bool params_in_batch = false;            // the parameters are those of the batch's last step (and host_params_stale)
     MomentsWork mw{};
     int64_t mw_samples = 0;
 
@@ -210,6 +218,109 @@ void dfree(T*& p)
     if (p) (void)hipFree(p);
     p = nullptr;
 }
+
+// Device memory of one host-pointer call, carved from the context's workspace
+// (up to kWsDevice bytes, kept for the next call) or, beyond that, from one
+// allocation given back at the end.  Arrays small enough (kWsPinned bytes in
+// all) travel through a pinned buffer, the results in one copy: an
+// allocation and release per array and a copy per result were most of a small
+// call (16 configurations of 64 particles: 107 us, 15 of them in the kernel).
+constexpr size_t kWsDevice = (size_t)64 << 20, kWsPinned = (size_t)1 << 20;
+class Arena {
+public:
+    explicit Arena(tdvmc_ctx* c) : ctx(c) {}
+    ~Arena()
+    {
+        // nothing may still use the memory (a call that ended early)
+        if (base && !done) (void)hipStreamSynchronize(ctx->stream);
+        if (own) (void)hipFree(base);
+    }
+    // offsets (in doubles, 256-byte aligned) of the arrays, before start()
+    size_t take(size_t n)
+    {
+        const size_t at = total;
+        total += (n + 31) & ~(size_t)31;
+        return at;
+    }
+    // `back`: the first double of the part that finish() brings back
+    hipError_t start(size_t back)
+    {
+        from = back;
+        hipError_t e = hipSuccess;
+        if (total * sizeof(double) <= kWsDevice) {
+            if (ctx->ws_dev_cap < total) {
+                ctx->ws_dev_cap = 0;
+                e = dalloc(&ctx->ws_dev, total);
+                if (e != hipSuccess) return e;
+                ctx->ws_dev_cap = total;
+            }
+            base = ctx->ws_dev;
+        } else {
+            e = hipMalloc(reinterpret_cast<void**>(&base), total * sizeof(double));
+            if (e != hipSuccess) {
+                base = nullptr;
+                return e;
+            }
+            own = true;
+        }
+        pinned = total * sizeof(double) <= kWsPinned;
+        if (pinned && ctx->ws_pin_cap < total) {
+            if (ctx->ws_pin) (void)hipHostFree(ctx->ws_pin);
+            ctx->ws_pin = nullptr;
+            ctx->ws_pin_cap = 0;
+            e = hipHostMalloc(reinterpret_cast<void**>(&ctx->ws_pin), total * sizeof(double), hipHostMallocDefault);
+            if (e != hipSuccess) return e;
+            ctx->ws_pin_cap = total;
+        }
+        return hipSuccess;
+    }
+    double* at(size_t off) const { return base + off; }
+    hipError_t send(size_t off, const double* src, size_t n)
+    {
+        if (pinned) {
+            std::memcpy(ctx->ws_pin + off, src, n * sizeof(double));
+            src = ctx->ws_pin + off;
+        }
+        return hipMemcpyAsync(base + off, src, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
+    }
+    // dst (null: not wanted) receives n doubles from off at finish()
+    void want(double* dst, size_t off, size_t n)
+    {
+        if (dst) wanted.push_back({dst, off, n});
+    }
+    hipError_t finish()
+    {
+        hipError_t e = hipSuccess;
+        if (pinned) {
+            size_t end = from;
+            for (const auto& w : wanted) end = std::max(end, w.off + w.n);
+            if (end > from)
+                e = hipMemcpyAsync(ctx->ws_pin + from, base + from, (end - from) * sizeof(double), hipMemcpyDeviceToHost,
+                                   ctx->stream);
+        } else {
+            for (const auto& w : wanted)
+                if (e == hipSuccess)
+                    e = hipMemcpyAsync(w.dst, base + w.off, w.n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
+        }
+        const hipError_t s = hipStreamSynchronize(ctx->stream);
+        if (e == hipSuccess) e = s;
+        done = true;
+        if (pinned && e == hipSuccess)
+            for (const auto& w : wanted) std::memcpy(w.dst, ctx->ws_pin + w.off, w.n * sizeof(double));
+        return e;
+    }
+
+private:
+    struct Want {
+        double* dst;
+        size_t off, n;
+    };
+    tdvmc_ctx* ctx;
+    double* base = nullptr;
+    size_t total = 0, from = 0;
+    bool own = false, pinned = false, done = false;
+    std::vector<Want> wanted;
+};
 
 // K shortest non-zero integer vectors ordered by (|n|^2, lexicographic n);
 // both n and -n are kept.
@@ -551,12 +662,16 @@ int upload_params(tdvmc_ctx* ctx)
     HIPC(launch_unpack_params(P, ctx->dX, ctx->dUR, ctx->dUI, ctx->stream));
     ctx->tf.dirty = ctx->td.dirty = true;
     ctx->host_params_stale = false;
+    ctx->params_in_batch = false;
     return TDVMC_OK;
 }
+
+int batch_pull_params(tdvmc_ctx* ctx);
 
 int pull_params(tdvmc_ctx* ctx)
 {
     if (!ctx->host_params_stale) return TDVMC_OK;
+    if (ctx->batch && ctx->params_in_batch) return batch_pull_params(ctx);
     const int P = P_of(ctx);
     std::vector<double> packed(2 * P + 2);
     HIPC(hipMemcpyAsync(packed.data(), ctx->dX, packed.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1418,6 +1533,9 @@ void release(tdvmc_ctx* ctx)
     dfree(ctx->dEI);
     dfree(ctx->dExpo);
     dfree(ctx->dOther);
+    dfree(ctx->ws_dev);
+    if (ctx->ws_pin) (void)hipHostFree(ctx->ws_pin);
+    ctx->ws_pin = nullptr;
     dfree(ctx->dMean);
     dfree(ctx->dS);
     dfree(ctx->dF);
@@ -1469,6 +1587,9 @@ struct tdvmc_batch {
     size_t mom_lds = 0;
     SolveArgs* dSolve[4] = {nullptr, nullptr, nullptr, nullptr};
     double* dX = nullptr;
+    std::vector<double> hx;           // host copy of dX (valid until the next step; read under hx_mu)
+    bool hx_valid = false;
+    std::mutex hx_mu;
     double* dXtmp = nullptr;
     double* dK[4] = {nullptr, nullptr, nullptr, nullptr};
     uint32_t* dEpoch = nullptr;
@@ -1759,6 +1880,35 @@ int batch_step_enqueue(tdvmc_batch* b, int prec, int ode, double dt)
     }
     BHIPC(launch_gather_batch<double>(b->dBpD, n, b->dX, 0, b->stream));
     BHIPC(launch_unpack_batch<double>(b->dBpD, n, b->dX, b->stream));
+    return TDVMC_OK;
+}
+
+// A member's parameters after the last batched step, from a host copy of the
+// whole batch's that the first member asked for brings (64 copies of one
+// system each took 0.8 ms).  Members may be asked from several threads.
+int batch_pull_params(tdvmc_ctx* c)
+{
+    tdvmc_batch* b = c->batch;
+    std::lock_guard<std::mutex> lock(b->hx_mu);
+    if (!b->hx_valid) {
+        b->hx.resize((size_t)b->xtotal);
+        hipError_t e = hipMemcpyAsync(b->hx.data(), b->dX, b->hx.size() * sizeof(double), hipMemcpyDeviceToHost, b->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+        if (e != hipSuccess) {
+            c->err = std::string("batch parameters: ") + hipGetErrorString(e);
+            return TDVMC_ERR_HIP;
+        }
+        b->hx_valid = true;
+    }
+    size_t s = 0;
+    while (b->sys[s] != c) s++;
+    const double* p = b->hx.data() + b->xoff[s];
+    const int P = c->sy.P;
+    std::copy(p, p + P, c->uR.begin());
+    std::copy(p + P, p + 2 * P, c->uI.begin());
+    c->phiR = p[2 * P];
+    c->phiI = p[2 * P + 1];
+    c->host_params_stale = false;
     return TDVMC_OK;
 }
 
@@ -2304,56 +2454,36 @@ int eval_configs_host(tdvmc_ctx* ctx, const double* R, int64_t W, int precision,
     if (rc) return rc;
     const int N = ctx->sy.N, D = ctx->sy.D, P = P_of(ctx), S = ctx->sy.P_s + 2;
     const bool pp = grad != nullptr || lap != nullptr;
-    double *dR = nullptr, *dEx = nullptr, *dER = nullptr, *dEI = nullptr, *dO = nullptr, *dG = nullptr,
-           *dL = nullptr, *dOt = nullptr, *dB = nullptr;
-    auto cleanup = [&]() {
-        dfree(dR); dfree(dEx); dfree(dER); dfree(dEI); dfree(dO); dfree(dG); dfree(dL); dfree(dOt); dfree(dB);
-    };
-    auto hipc = [&](hipError_t e, const char* what) {
-        if (e != hipSuccess) {
-            ctx->err = std::string(what) + ": " + hipGetErrorString(e);
-            return false;
-        }
-        return true;
-    };
-    bool ok = hipc(dalloc(&dR, (size_t)W * N * D), "hipMalloc") && hipc(dalloc(&dEx, (size_t)W), "hipMalloc") &&
-              hipc(dalloc(&dER, (size_t)W), "hipMalloc") && hipc(dalloc(&dEI, (size_t)W), "hipMalloc") &&
-              hipc(dalloc(&dO, (size_t)W * P), "hipMalloc") && hipc(dalloc(&dOt, (size_t)W * 9), "hipMalloc");
-    if (ok && pp) ok = hipc(dalloc(&dG, (size_t)W * N * D * 2), "hipMalloc") && hipc(dalloc(&dL, (size_t)W * N * 2), "hipMalloc");
-    if (ok && bsum) ok = hipc(dalloc(&dB, (size_t)W * S), "hipMalloc");
-    if (ok) ok = hipc(hipMemcpyAsync(dR, R, (size_t)W * N * D * sizeof(double), hipMemcpyHostToDevice, ctx->stream), "hipMemcpy");
-    if (ok) {
-        rc = prec == TDVMC_MIXED ? ensure_tables(ctx, ctx->tf, false) : ensure_tables(ctx, ctx->td, false);
-        if (rc) {
-            cleanup();
-            return rc;
-        }
-        hipEvent_t ev{};
-        prof_begin(ctx, "eval", &ev);
-        if (prec == TDVMC_MIXED)
-            ok = hipc((launch_eval<float, double>(ctx->sy, tables_of(ctx, ctx->tf), dR, W, dEx, dER, dEI, dO, dOt, dG,
-                                                  dL, nullptr, nullptr, ctx->stream, dB)), "eval kernel");
-        else
-            ok = hipc((launch_eval<double, double>(ctx->sy, tables_of(ctx, ctx->td), dR, W, dEx, dER, dEI, dO, dOt,
-                                                   dG, dL, nullptr, nullptr, ctx->stream, dB)), "eval kernel");
-        prof_end(ctx, "eval", ev);
-    }
-    auto down = [&](double* h, double* d, size_t n) {
-        if (ok && h) ok = hipc(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpy");
-    };
-    down(expo, dEx, (size_t)W);
-    down(ER, dER, (size_t)W);
-    down(EI, dEI, (size_t)W);
-    down(O, dO, (size_t)W * P);
-    down(other, dOt, (size_t)W * 9);
+    const size_t n = (size_t)W * N * D;
+    Arena ar(ctx);
+    const size_t oR = ar.take(n), oEx = ar.take(W), oER = ar.take(W), oEI = ar.take(W), oOt = ar.take((size_t)W * 9),
+                 oO = ar.take((size_t)W * P), oB = ar.take(bsum ? (size_t)W * S : 0), oG = ar.take(pp ? 2 * n : 0),
+                 oL = ar.take(pp ? (size_t)W * N * 2 : 0);
+    HIPC(ar.start(oEx));
+    HIPC(ar.send(oR, R, n));
+    rc = prec == TDVMC_MIXED ? ensure_tables(ctx, ctx->tf, false) : ensure_tables(ctx, ctx->td, false);
+    if (rc) return rc;
+    hipEvent_t ev{};
+    prof_begin(ctx, "eval", &ev);
+    double *dG = pp ? ar.at(oG) : nullptr, *dL = pp ? ar.at(oL) : nullptr, *dB = bsum ? ar.at(oB) : nullptr;
+    if (prec == TDVMC_MIXED)
+        HIPC((launch_eval<float, double>(ctx->sy, tables_of(ctx, ctx->tf), ar.at(oR), W, ar.at(oEx), ar.at(oER),
+                                         ar.at(oEI), ar.at(oO), ar.at(oOt), dG, dL, nullptr, nullptr, ctx->stream, dB)));
+    else
+        HIPC((launch_eval<double, double>(ctx->sy, tables_of(ctx, ctx->td), ar.at(oR), W, ar.at(oEx), ar.at(oER),
+                                          ar.at(oEI), ar.at(oO), ar.at(oOt), dG, dL, nullptr, nullptr, ctx->stream, dB)));
+    prof_end(ctx, "eval", ev);
+    ar.want(expo, oEx, W);
+    ar.want(ER, oER, W);
+    ar.want(EI, oEI, W);
+    ar.want(other, oOt, (size_t)W * 9);
+    ar.want(O, oO, (size_t)W * P);
+    ar.want(bsum, oB, (size_t)W * S);
     if (pp) {
-        down(grad, dG, (size_t)W * N * D * 2);
-        down(lap, dL, (size_t)W * N * 2);
+        ar.want(grad, oG, 2 * n);
+        ar.want(lap, oL, (size_t)W * N * 2);
     }
-    down(bsum, dB, (size_t)W * S);
-    if (ok) ok = hipc(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    cleanup();
-    if (!ok) return TDVMC_ERR_HIP;
+    HIPC(ar.finish());
     return prof_flush(ctx);
 }
 
@@ -2410,36 +2540,17 @@ int tdvmc_observables_configs(tdvmc_ctx* ctx, const double* R, int64_t W, int pr
     if (rc) return rc;
     const auto& o = ctx->obs;
     const int N = ctx->sy.N, D = ctx->sy.D;
-    double *dR = nullptr, *dG = nullptr, *dS = nullptr;
-    auto cleanup = [&]() {
-        dfree(dR);
-        dfree(dG);
-        dfree(dS);
-    };
-    auto fail = [&](hipError_t e, const char* what) {
-        if (e == hipSuccess) return false;
-        ctx->err = std::string(what) + ": " + hipGetErrorString(e);
-        cleanup();
-        return true;
-    };
-    if (fail(dalloc(&dR, (size_t)W * N * D), "hipMalloc") || fail(dalloc(&dS, (size_t)W * o.nshell), "hipMalloc") ||
-        (gr && fail(dalloc(&dG, (size_t)W * o.count), "hipMalloc")) ||
-        fail(hipMemcpyAsync(dR, R, (size_t)W * N * D * sizeof(double), hipMemcpyHostToDevice, ctx->stream),
-             "hipMemcpy"))
-        return TDVMC_ERR_HIP;
+    const size_t n = (size_t)W * N * D;
+    Arena ar(ctx);
+    const size_t oR = ar.take(n), oS = ar.take((size_t)W * o.nshell), oG = ar.take(gr ? (size_t)W * o.count : 0);
+    HIPC(ar.start(oS));
+    HIPC(ar.send(oR, R, n));
     rc = clear_obs(ctx);
-    if (!rc) rc = enqueue_obs(ctx, prec, dR, W, dG, dS);
-    if (rc) {
-        cleanup();
-        return rc;
-    }
-    if ((gr && fail(hipMemcpyAsync(gr, dG, (size_t)W * o.count * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-                    "hipMemcpy")) ||
-        (sk && fail(hipMemcpyAsync(sk, dS, (size_t)W * o.nshell * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-                    "hipMemcpy")) ||
-        fail(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize"))
-        return TDVMC_ERR_HIP;
-    cleanup();
+    if (!rc) rc = enqueue_obs(ctx, prec, ar.at(oR), W, gr ? ar.at(oG) : nullptr, ar.at(oS));
+    if (rc) return rc;
+    ar.want(sk, oS, (size_t)W * o.nshell);
+    ar.want(gr, oG, (size_t)W * o.count);
+    HIPC(ar.finish());
     return prof_flush(ctx);
 }
 
@@ -2494,39 +2605,24 @@ int tdvmc_moments(tdvmc_ctx* ctx, const double* O, const double* ER, const doubl
     CHECK_ARG(O && ER && EI && W >= 1 && P >= 1, "bad moments arguments");
     int prec, rc = resolve_precision(ctx, precision, &prec);
     if (rc) return rc;
-    double *dO = nullptr, *dE = nullptr, *dM = nullptr, *dS = nullptr, *dF = nullptr, *dPart = nullptr, *dCol = nullptr;
-    void* dXt = nullptr;
     size_t xb, pb, cb;
     moments_work_bytes(W, P, prec == TDVMC_MIXED ? 1 : 0, &xb, &pb, &cb);
-    hipError_t e = hipSuccess;
-    auto step = [&](hipError_t x) {
-        if (e == hipSuccess) e = x;
-    };
-    step(dalloc(&dO, (size_t)W * P));
-    step(dalloc(&dE, 2 * (size_t)W));
-    step(dalloc(&dM, (size_t)P + 2));
-    step(dalloc(&dS, (size_t)P * P));
-    step(dalloc(&dF, 2 * (size_t)P));
-    step(dalloc(&dPart, (pb + 7) / 8));
-    step(dalloc(&dCol, (cb + 7) / 8));
-    if (e == hipSuccess) e = hipMalloc(&dXt, xb);
-    step(hipMemcpyAsync(dO, O, (size_t)W * P * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    step(hipMemcpyAsync(dE, ER, (size_t)W * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    step(hipMemcpyAsync(dE + W, EI, (size_t)W * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    if (e == hipSuccess) {
-        MomentsWork wk{dXt, dPart, dCol, xb, pb, cb};
-        e = launch_moments<double>(dO, dE, dE + W, W, P, prec == TDVMC_MIXED ? 1 : 0, wk, dM, dS, dF, ctx->stream);
-    }
-    if (mean) step(hipMemcpyAsync(mean, dM, ((size_t)P + 2) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    if (S) step(hipMemcpyAsync(S, dS, (size_t)P * P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    if (F) step(hipMemcpyAsync(F, dF, 2 * (size_t)P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    step(hipStreamSynchronize(ctx->stream));
-    dfree(dO); dfree(dE); dfree(dM); dfree(dS); dfree(dF); dfree(dPart); dfree(dCol);
-    if (dXt) (void)hipFree(dXt);
-    if (e != hipSuccess) {
-        ctx->err = std::string("moments: ") + hipGetErrorString(e);
-        return TDVMC_ERR_HIP;
-    }
+    const size_t p = (size_t)P;
+    Arena ar(ctx);
+    const size_t oO = ar.take((size_t)W * P), oER = ar.take(W), oEI = ar.take(W), oX = ar.take((xb + 7) / 8),
+                 oP = ar.take((pb + 7) / 8), oC = ar.take((cb + 7) / 8), oM = ar.take(p + 2), oS = ar.take(p * p),
+                 oF = ar.take(2 * p);
+    HIPC(ar.start(oM));
+    HIPC(ar.send(oO, O, (size_t)W * P));
+    HIPC(ar.send(oER, ER, W));
+    HIPC(ar.send(oEI, EI, W));
+    MomentsWork wk{ar.at(oX), ar.at(oP), ar.at(oC), xb, pb, cb};
+    HIPC(launch_moments<double>(ar.at(oO), ar.at(oER), ar.at(oEI), W, P, prec == TDVMC_MIXED ? 1 : 0, wk, ar.at(oM),
+                                ar.at(oS), ar.at(oF), ctx->stream));
+    ar.want(mean, oM, p + 2);
+    ar.want(S, oS, p * p);
+    ar.want(F, oF, 2 * p);
+    HIPC(ar.finish());
     return TDVMC_OK;
 }
 
@@ -2538,37 +2634,29 @@ int tdvmc_solve(tdvmc_ctx* ctx, const double* mean, const double* S, const doubl
     CHECK_ARG(solver_type == 0 || solver_type == 1, "solver type must be 0 or 1");
     CHECK_ARG(P <= solve_max_params(solver_type),
               "P = " + std::to_string(P) + " exceeds the solver's limit of " + std::to_string(solve_max_params(solver_type)));
-    double *dM = nullptr, *dS = nullptr, *dF = nullptr, *dW = nullptr, *dX = nullptr;
-    int* dSt = nullptr;
-    hipError_t e = hipSuccess;
-    auto step = [&](hipError_t x) {
-        if (e == hipSuccess) e = x;
-    };
-    step(dalloc(&dM, (size_t)P + 2));
-    step(dalloc(&dS, (size_t)P * P));
-    step(dalloc(&dF, 2 * (size_t)P));
-    step(dalloc(&dW, (size_t)P * P + 4 * (size_t)P));
-    step(dalloc(&dX, 2 * (size_t)P + 2));
-    step(dalloc(&dSt, 1));
-    step(hipMemcpyAsync(dM, mean, ((size_t)P + 2) * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    step(hipMemcpyAsync(dS, S, (size_t)P * P * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    step(hipMemcpyAsync(dF, F, 2 * (size_t)P * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    int bad = 0;
-    if (e == hipSuccess) e = launch_fill_u32(reinterpret_cast<uint32_t*>(dSt), 0u, 1, ctx->stream);
-    if (e == hipSuccess) {
+    const size_t p = (size_t)P;
+    Arena ar(ctx);
+    const size_t oM = ar.take(p + 2), oS = ar.take(p * p), oF = ar.take(2 * p), oW = ar.take(p * p + 4 * p),
+                 oX = ar.take(2 * p + 2), oSt = ar.take(1);
+    HIPC(ar.start(oX));
+    HIPC(ar.send(oM, mean, p + 2));
+    HIPC(ar.send(oS, S, p * p));
+    HIPC(ar.send(oF, F, 2 * p));
+    int* dSt = reinterpret_cast<int*>(ar.at(oSt));
+    HIPC(launch_fill_u32(reinterpret_cast<uint32_t*>(dSt), 0u, 2, ctx->stream));
+    {
         // type 1 regularises only together with the scaling (src/TDVMC.cpp:1766-1771)
         const double e_eff = solver_type == 1 ? (precondition ? 0.002 : 0.0) : eps;
-        SolveArgs a{P, imag_time, precondition, e_eff, dM, dS, dF, dW, dX, dSt, solver_type == 1 ? 1 : 0};
-        e = launch_solve(a, ctx->stream);
+        SolveArgs a{P, imag_time, precondition, e_eff, ar.at(oM), ar.at(oS), ar.at(oF), ar.at(oW), ar.at(oX), dSt,
+                    solver_type == 1 ? 1 : 0};
+        HIPC(launch_solve(a, ctx->stream));
     }
-    step(hipMemcpyAsync(xdot, dX, (2 * (size_t)P + 2) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    step(hipMemcpyAsync(&bad, dSt, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    step(hipStreamSynchronize(ctx->stream));
-    dfree(dM); dfree(dS); dfree(dF); dfree(dW); dfree(dX); dfree(dSt);
-    if (e != hipSuccess) {
-        ctx->err = std::string("solve: ") + hipGetErrorString(e);
-        return TDVMC_ERR_HIP;
-    }
+    double status = 0.0;   // the bits of the pivot count
+    ar.want(xdot, oX, 2 * p + 2);
+    ar.want(&status, oSt, 1);
+    HIPC(ar.finish());
+    int bad = 0;
+    std::memcpy(&bad, &status, sizeof(int));
     if (n_bad) *n_bad = bad;
     if (bad > 0) {
         ctx->err = "non-positive pivot in the Cholesky factorisation";
@@ -2667,6 +2755,7 @@ int tdvmc_tdvp_step(tdvmc_ctx* ctx, double dt, int ode_type, int precision, int 
     }
     ctx->tf.dirty = ctx->td.dirty = true;
     ctx->host_params_stale = true;
+    ctx->params_in_batch = false;
     rc = prof_flush(ctx);
     if (rc) return rc;
     if (ctx->accept_check) {
@@ -2711,52 +2800,30 @@ int tdvmc_adjoint(tdvmc_ctx* ctx, const double* R, int64_t W, const double* gbar
     int prec, rc = resolve_precision(ctx, precision, &prec);
     if (rc) return rc;
     const int N = ctx->sy.N, D = ctx->sy.D, P = P_of(ctx);
-    double *dRin = nullptr, *dEx = nullptr, *dER = nullptr, *dEI = nullptr, *dO = nullptr, *dG = nullptr,
-           *dL = nullptr, *dGb = nullptr, *dOutR = nullptr, *dOutA = nullptr, *dOuter = nullptr;
-    hipError_t e = hipSuccess;
-    auto step = [&](hipError_t x) {
-        if (e == hipSuccess) e = x;
-    };
-    step(dalloc(&dRin, (size_t)W * N * D));
-    step(dalloc(&dEx, (size_t)W));
-    step(dalloc(&dER, (size_t)W));
-    step(dalloc(&dEI, (size_t)W));
-    step(dalloc(&dO, (size_t)W * P));
-    step(dalloc(&dG, (size_t)W * N * D * 2));
-    step(dalloc(&dL, (size_t)W * N * 2));
-    step(dalloc(&dGb, (size_t)W));
-    step(dalloc(&dOutR, (size_t)W * N * D));
-    step(dalloc(&dOutA, (size_t)P));
-    step(dalloc(&dOuter, (size_t)W));
-    step(hipMemcpyAsync(dRin, R, (size_t)W * N * D * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    step(hipMemcpyAsync(dGb, gbar, (size_t)W * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    if (e == hipSuccess) {
-        rc = prec == TDVMC_MIXED ? ensure_tables(ctx, ctx->tf, false) : ensure_tables(ctx, ctx->td, false);
-        if (rc == TDVMC_OK) {
-            if (prec == TDVMC_MIXED)
-                e = launch_eval<float, double>(ctx->sy, tables_of(ctx, ctx->tf), dRin, W, dEx, dER, dEI, dO, nullptr,
-                                               dG, dL, dOuter, nullptr, ctx->stream);
-            else
-                e = launch_eval<double, double>(ctx->sy, tables_of(ctx, ctx->td), dRin, W, dEx, dER, dEI, dO, nullptr,
-                                                dG, dL, dOuter, nullptr, ctx->stream);
-        }
-    }
-    if (e == hipSuccess && rc == TDVMC_OK) {
-        e = launch_adjoint_scale(dG, dGb, W, N * D, dOutR, ctx->stream);
-        if (e == hipSuccess) e = launch_adjoint_reduce(dO, dGb, W, P, dOutA, ctx->stream);
-        if (e == hipSuccess) e = launch_adjoint_outer(dOuter, dGb, W, ctx->sy.outer_idx, dOutA, ctx->stream);
-    }
-    if (dR) step(hipMemcpyAsync(dR, dOutR, (size_t)W * N * D * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    if (dalpha) step(hipMemcpyAsync(dalpha, dOutA, (size_t)P * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    step(hipStreamSynchronize(ctx->stream));
-    dfree(dRin); dfree(dEx); dfree(dER); dfree(dEI); dfree(dO); dfree(dG); dfree(dL); dfree(dGb); dfree(dOutR);
-    dfree(dOutA);
-    dfree(dOuter);
+    const size_t n = (size_t)W * N * D;
+    Arena ar(ctx);
+    const size_t oR = ar.take(n), oGb = ar.take(W), oEx = ar.take(W), oER = ar.take(W), oEI = ar.take(W),
+                 oO = ar.take((size_t)W * P), oG = ar.take(2 * n), oL = ar.take((size_t)W * N * 2), oOuter = ar.take(W),
+                 oOutA = ar.take(P), oOutR = ar.take(n);
+    HIPC(ar.start(oOutA));
+    HIPC(ar.send(oR, R, n));
+    HIPC(ar.send(oGb, gbar, W));
+    rc = prec == TDVMC_MIXED ? ensure_tables(ctx, ctx->tf, false) : ensure_tables(ctx, ctx->td, false);
     if (rc) return rc;
-    if (e != hipSuccess) {
-        ctx->err = std::string("adjoint: ") + hipGetErrorString(e);
-        return TDVMC_ERR_HIP;
-    }
+    if (prec == TDVMC_MIXED)
+        HIPC((launch_eval<float, double>(ctx->sy, tables_of(ctx, ctx->tf), ar.at(oR), W, ar.at(oEx), ar.at(oER),
+                                         ar.at(oEI), ar.at(oO), nullptr, ar.at(oG), ar.at(oL), ar.at(oOuter), nullptr,
+                                         ctx->stream)));
+    else
+        HIPC((launch_eval<double, double>(ctx->sy, tables_of(ctx, ctx->td), ar.at(oR), W, ar.at(oEx), ar.at(oER),
+                                          ar.at(oEI), ar.at(oO), nullptr, ar.at(oG), ar.at(oL), ar.at(oOuter), nullptr,
+                                          ctx->stream)));
+    HIPC(launch_adjoint_scale(ar.at(oG), ar.at(oGb), W, N * D, ar.at(oOutR), ctx->stream));
+    HIPC(launch_adjoint_reduce(ar.at(oO), ar.at(oGb), W, P, ar.at(oOutA), ctx->stream));
+    HIPC(launch_adjoint_outer(ar.at(oOuter), ar.at(oGb), W, ctx->sy.outer_idx, ar.at(oOutA), ctx->stream));
+    ar.want(dR, oOutR, n);
+    ar.want(dalpha, oOutA, P);
+    HIPC(ar.finish());
     return TDVMC_OK;
 }
 
@@ -2966,6 +3033,7 @@ int tdvmc_batch_create(const char* const* configs, int n_systems, tdvmc_batch** 
         const int rc = tdvmc_create(configs[s], &c);
         if (rc) return fail(rc, "system " + std::to_string(s) + ": " + g_create_error);
         b->sys.push_back(c);
+        c->batch = b;
         if (s == 0) {
             b->D = c->sy.D;
             b->periodic = c->sy.periodic;
@@ -3195,6 +3263,7 @@ int tdvmc_batch_tdvp_step(tdvmc_batch* b, double dt, int ode_type, int precision
     // parameters set through the member contexts live in their packed vectors,
     // which the step gathers first
     if ((rc = batch_sync_members(b))) return rc;
+    b->hx_valid = false;
     // descriptors current with the members (a direct sweep or measurement, a
     // new walker count or a quench since the last step); drops a captured
     // step whose launch shapes no longer fit
@@ -3225,6 +3294,7 @@ int tdvmc_batch_tdvp_step(tdvmc_batch* b, double dt, int ode_type, int precision
     for (auto* c : b->sys) {
         c->tf.dirty = c->td.dirty = true;
         c->host_params_stale = true;
+        c->params_in_batch = true;
         c->time += dt;
         c->step += 1;
         c->trials_total += fresh_stages(ode) * c->therm_moves * c->W;
