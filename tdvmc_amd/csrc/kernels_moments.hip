@@ -380,6 +380,7 @@ __global__ __launch_bounds__(256) void reduce_tiles_kernel(const double* __restr
 // d_c = mean_c - mean, so nothing is subtracted that is larger than the
 // spread of the samples.
 constexpr int kSmallRows = 64, kSmallCols = 64, kSmallChunks = 512;
+static_assert(kSmallRows == kChunkRows && kSmallChunks <= kMaxChunks, "chunk means fit the column sums' buffer");
 
 inline bool moments_small(int64_t W, int P, int mode)
 {
@@ -511,8 +512,9 @@ void moments_work_bytes(int64_t W, int P, int mode, size_t* xt, size_t* partial,
         *xt = (size_t)g.Wp * g.Pp * kSplit * sizeof(__bf16);
     *partial = (size_t)g.groups * g.ntiles * g.tile * g.tile * sizeof(double);
     *colsum = (size_t)g.chunks * g.Pa * sizeof(double);
-    // (a chunk of the small form is a column-sum chunk: kSmallRows == kChunkRows)
-    if (moments_small(W, P, mode)) *partial = (size_t)small_chunks(W) * g.ntiles * 256 * sizeof(double);
+    // (the small form keeps its chunks' means where the column sums go, a chunk
+    // being a column-sum chunk, and their tiles, 32 nb (nb + 1) / 2 bytes a sample
+    // against 128 nb packed, where the packed operands go)
 }
 
 template <typename TO>
@@ -533,10 +535,11 @@ hipError_t launch_moments(const TO* O, const double* ER, const double* EI, int64
 
     if (moments_small(W, Pc, mode)) {
         const int chunks = small_chunks(W);
+        double* tiles = static_cast<double*>(wk.xt);
         hipLaunchKernelGGL(small_partial_kernel<TO>, dim3(chunks), dim3(256), 0, st, O, ER, EI, W, Pc, cs, g.nb, wk.colsum,
-                           wk.partial);
-        hipLaunchKernelGGL(small_combine_kernel, dim3(g.ntiles), dim3(1024), 0, st, wk.colsum, wk.partial, chunks, W, Pc,
-                           g.nb, wk.outmap, P, mean, S, F);
+                           tiles);
+        hipLaunchKernelGGL(small_combine_kernel, dim3(g.ntiles), dim3(1024), 0, st, wk.colsum, tiles, chunks, W, Pc, g.nb,
+                           wk.outmap, P, mean, S, F);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(colsum_kernel<TO>, dim3((unsigned)ceil_div(g.Pa, kColBlock), g.chunks), dim3(kColBlock), 0, st,
