@@ -1469,7 +1469,7 @@ int alloc_ctx(tdvmc_ctx* ctx)
     HIPC(dalloc(&ctx->dMean, P + 2));
     HIPC(dalloc(&ctx->dS, (size_t)P * P));
     HIPC(dalloc(&ctx->dF, 2 * (size_t)P));
-    HIPC(dalloc(&ctx->dWork, (size_t)P * P + 4 * (size_t)P));
+    HIPC(dalloc(&ctx->dWork, solve_work_doubles(P)));
     HIPC(dalloc(&ctx->dStatus, 1));
     int rc = upload_params(ctx);
     if (rc) return rc;
@@ -2636,7 +2636,7 @@ int tdvmc_solve(tdvmc_ctx* ctx, const double* mean, const double* S, const doubl
               "P = " + std::to_string(P) + " exceeds the solver's limit of " + std::to_string(solve_max_params(solver_type)));
     const size_t p = (size_t)P;
     Arena ar(ctx);
-    const size_t oM = ar.take(p + 2), oS = ar.take(p * p), oF = ar.take(2 * p), oW = ar.take(p * p + 4 * p),
+    const size_t oM = ar.take(p + 2), oS = ar.take(p * p), oF = ar.take(2 * p), oW = ar.take(solve_work_doubles(P)),
                  oX = ar.take(2 * p + 2), oSt = ar.take(1);
     HIPC(ar.start(oX));
     HIPC(ar.send(oM, mean, p + 2));

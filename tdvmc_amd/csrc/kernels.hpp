@@ -122,14 +122,20 @@ struct SolveArgs {
     const double* mean;        // [P+2]
     const double* S;           // [P][P]
     const double* F;           // [2][P]
-    double* work;              // [P][P] scratch (factor), + 4P
+    double* work;              // solve_work_doubles(P) of scratch (factor and four vectors)
     double* xdot;              // [2P+2] out: alpha-dot R, alpha-dot I, phi-dot R, phi-dot I
     int* status;               // [1] count of non-positive pivots (added to)
     int mean_sub;              // 1: subtract the mean of each solution vector (solver type 1)
 };
+// the factor in whole tiles of 16, four vectors
+inline size_t solve_work_doubles(int P)
+{
+    const size_t LD = ((size_t)P + 15) / 16 * 16;
+    return LD * LD + 4 * LD;
+}
 hipError_t launch_solve(const SolveArgs& a, hipStream_t st);
 // largest P the solve kernels take: Cholesky (solver type 0; LDS panel of
-// NB = 16 columns) or full-pivot QR (type 1)
+// 16 columns) or full-pivot QR (type 1)
 int solve_max_params(int solver_type);
 // one workgroup per system; args_dev [n] in device memory
 hipError_t launch_solve_batch(const SolveArgs* args_dev, int n, int P_max, hipStream_t st);

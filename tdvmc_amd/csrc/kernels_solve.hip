@@ -9,22 +9,18 @@
 // (phi-dot, computed on the scaled solution before the scaling is undone, as
 // in :1749-1758).  Solver type 1 is the full-pivot QR kernel further down.
 //
-// Blocked right-looking Cholesky: the rows below each NB-column diagonal
-// block are staged in LDS (row-major at a padded stride).  One wavefront
-// factors the NB x NB diagonal block (wave-level ordering, no workgroup
-// barrier), one thread per row solves the rows below it against that block,
-// the panel is written back, and the trailing lower triangle is updated by
-// all 1024 threads in 16 x 16 tiles on FP64 MFMA (a rank-NB update with the
-// panel read from LDS; every tile's loads are issued before its stores).  The
-// triangular solves are blocked the same way: each NB x NB diagonal block is
-// staged in LDS and solved by one wavefront with v_readlane exchanges, the
-// rest of the right-hand side is updated by the whole workgroup.  The factor
-// lives column-major in the work buffer (L2-resident for the sizes the LDS
-// panel allows), with 1 / L[c][c] on its diagonal so that the solves only
-// multiply.  NB is 16 for P <= 340 (shorter serial chains in the diagonal
-// blocks and row solves) and 32 above (fewer panels and barriers).
+// Blocked right-looking Cholesky in columns of kNB = 16: one wavefront factors
+// the 16 x 16 diagonal block in registers, one thread per row solves the rows
+// below it against that block in LDS (row-major at a padded stride), and the
+// trailing lower triangle is updated in 16 x 16 tiles on FP64 MFMA.  The factor
+// lives in the work buffer, with 1 / L[c][c] on its diagonal so that the
+// solves only multiply.  solve_ahead_body holds two panels and the right-hand
+// sides in LDS and lets steps of neighbouring panels run side by side;
+// solve_body needs one panel only and takes the larger systems.
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -34,6 +30,7 @@ namespace tdvmc {
 namespace {
 
 constexpr int kThreads = 1024;
+constexpr int kNB = 16, kLDP = kNB + 1;   // block width, LDS stride of a panel row
 
 typedef double double4v __attribute__((ext_vector_type(4)));
 
@@ -71,7 +68,6 @@ __device__ double block_reduce(double v, double* red)
     return s;
 }
 
-template <int NB>
 __device__ __forceinline__ void solve_body(const SolveArgs& a)
 {
     const int P = a.P, tid = threadIdx.x;
@@ -82,10 +78,10 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     double* sc = bI + P;
     double* dorig = sc + P;              // diagonal after scaling and the eps shift
     extern __shared__ __align__(16) unsigned char smem[];
-    double* pan = reinterpret_cast<double*>(smem);   // [rows below][NB + 1] panel; [NB][NB] blocks in the solves
+    double* pan = reinterpret_cast<double*>(smem);   // [rows below][kNB + 1] panel; [kNB][kNB] blocks in the solves
     __shared__ double red[kThreads / 64];
-    __shared__ double ipiv[NB];          // 1 / L[c][c]
-    __shared__ double ldc[NB * NB];      // diagonal block, column-major: ldc[c * NB + k] = L[k][c]
+    __shared__ double ipiv[kNB];          // 1 / L[c][c]
+    __shared__ double ldc[kNB * kNB];      // diagonal block, column-major: ldc[c * kNB + k] = L[k][c]
     __shared__ int nbad;
     const double* mO = a.mean;
     const double eR = a.mean[P], eI = a.mean[P + 1];
@@ -142,40 +138,39 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
 
     // ---------------------------------------------------------------- Cholesky
     // The rows below the diagonal block sit in LDS row-major with a padded
-    // stride (pan[rb * LDP + c], LDP = NB + 1): a thread's row is read with
+    // stride (pan[rb * kLDP + c]): a thread's row is read with
     // immediate offsets, and only threads rb and rb + 32 share a bank.  The
     // diagonal block is staged on its own, column-major and padded with the
-    // identity to NB x NB (ldc[c * NB + l] = A[l][c]): padded columns have
+    // identity to kNB x kNB (ldc[c * kNB + l] = A[l][c]): padded columns have
     // pivot 1 and zero off-diagonal entries and leave the real rows unchanged,
     // so no step below has a run-time bound on the block.  Only the last
     // block can be partial, and it has no rows below it.
-    constexpr int LDP = NB + 1;
-    for (int p0 = 0; p0 < P; p0 += NB) {
-        const int nb = min(NB, P - p0);
+    for (int p0 = 0; p0 < P; p0 += kNB) {
+        const int nb = min(kNB, P - p0);
         const int below = P - p0 - nb;
         if (below > 0) {
             Walk2 wk2(tid, below);
             for (int e = tid; e < nb * below; e += kThreads) {
-                pan[wk2.r * LDP + wk2.c] = Lm[(size_t)(p0 + wk2.c) * P + p0 + nb + wk2.r];
+                pan[wk2.r * kLDP + wk2.c] = Lm[(size_t)(p0 + wk2.c) * P + p0 + nb + wk2.r];
                 wk2.next();
             }
         }
-        for (int e = tid; e < NB * NB; e += kThreads) {
-            const int c = e / NB, l = e % NB;
+        for (int e = tid; e < kNB * kNB; e += kThreads) {
+            const int c = e / kNB, l = e % kNB;
             ldc[e] = (c < nb && l < nb) ? Lm[(size_t)(p0 + c) * P + p0 + l] : (c == l ? 1.0 : 0.0);
         }
         __syncthreads();
         // diagonal block by one wavefront in registers: lane l holds row
-        // l mod NB, column entries reach the other lanes by v_readlane.  Every
+        // l mod kNB, column entries reach the other lanes by v_readlane.  Every
         // lane updates its whole row (the entries above the diagonal are
         // never read), and the diagonal gets 1 / L[c][c] from ipiv at the end.
         if (wv == 0) {
-            const int l = lane & (NB - 1);
-            double av[NB];
+            const int l = lane & (kNB - 1);
+            double av[kNB];
 #pragma unroll
-            for (int k = 0; k < NB; k++) av[k] = ldc[k * NB + l];
+            for (int k = 0; k < kNB; k++) av[k] = ldc[k * kNB + l];
 #pragma unroll
-            for (int c = 0; c < NB; c++) {
+            for (int c = 0; c < kNB; c++) {
                 const double d = readlane_f(av[c], c);
                 double ipj;
                 if (d > 0.0) {
@@ -196,34 +191,34 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
                 av[c] *= ipj;
                 if (lane == 0) ipiv[c] = ipj;
 #pragma unroll
-                for (int k = c + 1; k < NB; k++) av[k] -= av[c] * readlane_f(av[c], k);
+                for (int k = c + 1; k < kNB; k++) av[k] -= av[c] * readlane_f(av[c], k);
                 // one column's lane reads at a time (scalar registers)
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (lane < NB) {
+            if (lane < kNB) {
 #pragma unroll
-                for (int k = 0; k < NB; k++) ldc[k * NB + lane] = av[k];
+                for (int k = 0; k < kNB; k++) ldc[k * kNB + lane] = av[k];
                 // the factor keeps 1 / L[c][c] on its diagonal: the triangular
                 // solves multiply by it (same wavefront, after the writes above
                 // and lane 0's ipiv writes)
-                ldc[lane * NB + lane] = ipiv[lane];
+                ldc[lane * kNB + lane] = ipiv[lane];
             }
         }
         __syncthreads();
         // rows below the block, one thread per row, right-looking within the
         // row: L[r][c] = v_c / L[c][c], then v_k -= L[r][c] L[k][c] for k > c
         for (int rb = tid; rb < below; rb += kThreads) {
-            double* pr = pan + rb * LDP;
-            double v[NB];
+            double* pr = pan + rb * kLDP;
+            double v[kNB];
 #pragma unroll
-            for (int k = 0; k < NB; k++) v[k] = pr[k];
+            for (int k = 0; k < kNB; k++) v[k] = pr[k];
 #pragma unroll
-            for (int c = 0; c < NB; c++) {
+            for (int c = 0; c < kNB; c++) {
                 const double xc = v[c] * ipiv[c];
                 pr[c] = xc;
-                const double* lcol = ldc + c * NB;   // L[k][c]
+                const double* lcol = ldc + c * kNB;   // L[k][c]
 #pragma unroll
-                for (int k = c + 1; k < NB; k++) v[k] -= xc * lcol[k];
+                for (int k = c + 1; k < kNB; k++) v[k] -= xc * lcol[k];
                 // keeps the 32 columns' table reads from being hoisted together (register spills)
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -234,7 +229,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
             for (int e = tid; e < nb * (nb + below); e += kThreads) {
                 const int c = wk3.c, r = wk3.r;
                 if (r >= c)
-                    Lm[(size_t)(p0 + c) * P + p0 + r] = r < nb ? ldc[c * NB + r] : pan[(r - nb) * LDP + c];
+                    Lm[(size_t)(p0 + c) * P + p0 + r] = r < nb ? ldc[c * kNB + r] : pan[(r - nb) * kLDP + c];
                 wk3.next();
             }
         }
@@ -265,11 +260,11 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
                     ok[v] = i < below && k <= i;
                     old[v] = ok[v] ? Lm[(q0 + k) * P + q0 + i] : 0.0;
                 }
-                const double* pa = pan + (16 * tk + pp) * LDP + kk;   // rows k
-                const double* pb = pan + (16 * ti + pp) * LDP + kk;   // rows i
+                const double* pa = pan + (16 * tk + pp) * kLDP + kk;   // rows k
+                const double* pb = pan + (16 * ti + pp) * kLDP + kk;   // rows i
                 double4v acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int s4 = 0; s4 < NB / 4; s4++)
+                for (int s4 = 0; s4 < kNB / 4; s4++)
                     acc = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[4 * s4], pb[4 * s4], acc, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
@@ -282,25 +277,25 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     }
 
     // ---------------------------------------------------------------- L t = b
-    for (int p0 = 0; p0 < P; p0 += NB) {
-        const int nb = min(NB, P - p0);
-        // diagonal block into LDS: pan[j * NB + l] = L[p0 + l][p0 + j]
+    for (int p0 = 0; p0 < P; p0 += kNB) {
+        const int nb = min(kNB, P - p0);
+        // diagonal block into LDS: pan[j * kNB + l] = L[p0 + l][p0 + j]
         for (int e = tid; e < nb * nb; e += kThreads) {
             const int j = e / nb, l = e % nb;
-            pan[j * NB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
+            pan[j * kNB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
         }
         __syncthreads();
         if (wv == 0) {
             // lane l owns row p0 + l; the diagonal holds 1 / L[j][j]
             double tR = lane < nb ? bR[p0 + lane] : 0.0, tI = lane < nb ? bI[p0 + lane] : 0.0;
             for (int j = 0; j < nb; j++) {
-                const double rjj = pan[j * NB + j];
+                const double rjj = pan[j * kNB + j];
                 const double xR = readlane_f(tR, j) * rjj, xI = readlane_f(tI, j) * rjj;
                 if (lane == j) {
                     tR = xR;
                     tI = xI;
                 } else if (lane > j && lane < nb) {
-                    const double l = pan[j * NB + lane];
+                    const double l = pan[j * kNB + lane];
                     tR -= l * xR;
                     tI -= l * xI;
                 }
@@ -326,9 +321,9 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     }
 
     // ---------------------------------------------------------------- L^T x = t
-    const int npan = (P + NB - 1) / NB;
+    const int npan = (P + kNB - 1) / kNB;
     for (int pb = npan - 1; pb >= 0; pb--) {
-        const int p0 = pb * NB, nb = min(NB, P - p0), pe = p0 + nb;
+        const int p0 = pb * kNB, nb = min(kNB, P - p0), pe = p0 + nb;
         // t_i -= sum_{j >= pe} L[j][i] x_j for the panel's rows (one wave per row group)
         for (int i = p0 + wv; i < pe; i += kThreads / 64) {
             double sR = 0.0, sI = 0.0;
@@ -346,22 +341,22 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
                 bI[i] -= sI;
             }
         }
-        // diagonal block into LDS: pan[j * NB + l] = L[p0 + l][p0 + j]
+        // diagonal block into LDS: pan[j * kNB + l] = L[p0 + l][p0 + j]
         for (int e = tid; e < nb * nb; e += kThreads) {
             const int j = e / nb, l = e % nb;
-            pan[j * NB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
+            pan[j * kNB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
         }
         __syncthreads();
         if (wv == 0) {
             double tR = lane < nb ? bR[p0 + lane] : 0.0, tI = lane < nb ? bI[p0 + lane] : 0.0;
             for (int j = nb - 1; j >= 0; j--) {
-                const double rjj = pan[j * NB + j];
+                const double rjj = pan[j * kNB + j];
                 const double xR = readlane_f(tR, j) * rjj, xI = readlane_f(tI, j) * rjj;
                 if (lane == j) {
                     tR = xR;
                     tI = xI;
                 } else if (lane < j) {
-                    const double l = pan[lane * NB + j];   // L[j][lane]
+                    const double l = pan[lane * kNB + j];   // L[j][lane]
                     tR -= l * xR;
                     tI -= l * xI;
                 }
@@ -385,6 +380,414 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     for (int i = tid; i < P; i += kThreads) {
         a.xdot[i] = bR[i] / sc[i];
         a.xdot[P + i] = bI[i] / sc[i];
+    }
+    if (tid == 0) {
+        if (a.imag_time == 0)
+            pi -= eR;
+        else
+            pr -= eR;
+        a.xdot[2 * P] = pr;
+        a.xdot[2 * P + 1] = pi;
+        if (a.status) a.status[0] += nbad;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The same solve where two panels and the right-hand sides fit the LDS.  One
+// workgroup's solve is a chain of short dependent steps, not of work (8.6
+// MFLOP at P = 296), so the steps that need not follow each other run side by
+// side:
+//   - the trailing update's first tile column goes straight into the LDS of
+//     the next panel (no store, reload and staging), then one wavefront
+//     factors the next diagonal block while the others update the rest;
+//   - the right-hand sides are two more rows under the matrix: L t = b is done
+//     with the factorisation;
+//   - in L^T x = t a wavefront has its row's entries of the factor loaded
+//     before the blocks that they meet are solved;
+//   - S is not copied: the first panel's update reads it in place.
+// The operations on each number and their order are solve_body's, so both give
+// the same bits.
+// At P = 32, 13 us against 27 without these; at P = 296, 152 against 373 us, of
+// which the matrix unit's work on one CU is about 35 us and the rest the
+// chains of the 19 diagonal blocks, row solves and back substitutions (about 5
+// us a block) and the trailing tiles' loads (two tiles' or four tiles' entries
+// under way instead of one: no faster).
+// rows of the first panel buffer: the rows below the first block, in whole
+// tiles (the second buffer holds a tile less); never less than the back
+// substitution's diagonal blocks need
+__host__ __device__ inline int ahead_rows(int P) { return P > 3 * kNB ? (P - kNB + 15) / 16 * 16 : 32; }
+
+template <int CTRL>
+__device__ __forceinline__ double row_dpp(double x)
+{
+    const int2 v = __builtin_bit_cast(int2, x);
+    int2 r;
+    r.x = __builtin_amdgcn_update_dpp(0, v.x, CTRL, 0xf, 0xf, true);
+    r.y = __builtin_amdgcn_update_dpp(0, v.y, CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, r);
+}
+// x of lane C of every 16 lanes (DPP row broadcast): the value stays in vector
+// registers, so there is no wait between the read and its use
+template <int C>
+__device__ __forceinline__ double row_bcast(double x) { return row_dpp<0x150 + C>(x); }
+// the sum over the wavefront, as a butterfly over 32, 16, .. 1 gives it (from 8
+// down the halves are alike, and rotating a row is the exchange)
+__device__ __forceinline__ double wave_sum(double x)
+{
+    x += __shfl_xor(x, 32, 64);
+    x += __shfl_xor(x, 16, 64);
+    x += row_dpp<0x128>(x);
+    x += row_dpp<0x124>(x);
+    x += row_dpp<0x122>(x);
+    return x + row_dpp<0x121>(x);
+}
+template <typename F, int... I>
+__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+// f(0), f(1), .. f(N - 1) with constant arguments
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F f) { each_of(f, std::make_integer_sequence<int, N>{}); }
+
+// Diagonal block d[c * 16 + l] = A[l][c] (l >= c; identity past the matrix)
+// factored in place by one wavefront (every 16 lanes alike), 1 / L[c][c] on the
+// diagonal; rd is the reciprocal of the lane's unreduced diagonal entry.  The
+// next column's pivot is worked out beside the rest of a column's updates.
+// Returns the number of non-positive pivots.
+__device__ __forceinline__ int factor_block(double* d, double rd, int lane)
+{
+    const int l = lane & (kNB - 1);
+    double av[kNB], own = 0.0;
+#pragma unroll
+    for (int k = 0; k < kNB; k++) av[k] = d[k * kNB + l];
+    int bad = 0;
+    auto pivot = [&](auto c) {
+        // 1 / sqrt(x) as in solve_body; where x is not positive the unreduced
+        // diagonal entry stands in as the pivot
+        const double x = row_bcast<c>(av[c]), hx = 0.5 * x, alt = row_bcast<c>(rd);
+        double y = __builtin_amdgcn_rsq(x);
+        y = y * (1.5 - hx * y * y);
+        y = y * (1.5 - hx * y * y);
+        bad += x > 0.0 ? 0 : 1;
+        return x > 0.0 ? y : alt;
+    };
+    double r = pivot(std::integral_constant<int, 0>{});
+    static_for<kNB>([&](auto c) {
+        av[c] *= r;
+        own = l == c ? r : own;
+        if constexpr (c + 1 < kNB) {
+            av[c + 1] -= av[c] * row_bcast<c + 1>(av[c]);
+            r = pivot(std::integral_constant<int, c + 1>{});
+        }
+        static_for<kNB>([&](auto k) {
+            if constexpr (k > c + 1) av[k] -= av[c] * row_bcast<k>(av[c]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    if (lane < kNB) {
+#pragma unroll
+        for (int k = 0; k < kNB; k++) d[k * kNB + lane] = av[k];
+        d[lane * kNB + lane] = own;
+    }
+    return bad;
+}
+
+// RHS_LDS: the right-hand sides in LDS, else in the work buffer.
+template <bool RHS_LDS>
+__device__ __forceinline__ void solve_ahead_body(const SolveArgs& a)
+{
+    const int P = a.P, tid = threadIdx.x;
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int NW = kThreads / 64;
+    static_assert(NW == kNB, "a wavefront per column of the first panel");
+    // Column-major with LD = P rounded up to whole tiles: Lm[j * LD + i] is
+    // A[i][j], later L[i][j].  No step of the update has an edge to look at;
+    // rows and columns past the matrix reach no other ones.
+    const int LD = (P + kNB - 1) / kNB * kNB;
+    double* Lm = a.work;
+    double* sc = a.work + (size_t)LD * LD;
+    double* rdiag = sc + LD;             // reciprocal of the diagonal after scaling and the eps shift
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int cap = ahead_rows(P);
+    double* pan0 = reinterpret_cast<double*>(smem);   // [cap][kLDP], [cap - 16][kLDP]
+    // [2][LD] right-hand sides, then t, then x
+    double* bl = RHS_LDS ? pan0 + (size_t)(2 * cap - kNB) * kLDP : rdiag + LD;
+    __shared__ double ldc[2][kNB * kNB];              // diagonal blocks, column-major
+    __shared__ double red[NW];
+    __shared__ int nbad;
+    const double* mO = a.mean;
+    const double eR = a.mean[P], eI = a.mean[P + 1];
+
+    if (tid == 0) nbad = 0;
+    for (int i = tid; i < LD; i += kThreads) {
+        double r = 0.0, m = 0.0;
+        if (i < P) {
+            const double sii = a.S[(size_t)i * P + i];
+            const double s = a.precondition ? sqrt(sii) : 1.0;
+            if (a.imag_time == 0) {
+                r = a.F[P + i];
+                m = -a.F[i];
+            } else {
+                r = -a.F[i];
+                m = -(a.F[P + i] + mO[i] * eI);
+            }
+            sc[i] = s;
+            if (a.precondition) {
+                r /= s;
+                m /= s;
+            }
+            rdiag[i] = 1.0 / ((a.precondition ? sii / (s * s) : sii) + a.eps);
+        }
+        bl[i] = r;
+        bl[LD + i] = m;
+    }
+    __syncthreads();
+    // entry of the scaled and shifted matrix, row r of column c <= r (S is
+    // symmetric: read along its row c)
+    auto entry = [&](double x, int r, int c) {
+        if (a.precondition) x /= (sc[r] * sc[c]);
+        return r == c ? x + a.eps : x;
+    };
+    {
+        const int c = min(wv, P - 1);
+        for (int r0 = lane; r0 < LD; r0 += 4 * 64) {
+            double v[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = a.S[(size_t)c * P + min(r0 + 64 * q, P - 1)];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = r0 + 64 * q;
+                if (r >= LD) continue;
+                const double x = entry(v[q], min(r, P - 1), c);
+                if (r < kNB)
+                    ldc[0][wv * kNB + r] = max(r, wv) < P ? x : r == wv ? 1.0 : 0.0;
+                else
+                    pan0[(r - kNB) * kLDP + wv] = x;
+            }
+        }
+    }
+    __syncthreads();
+    if (wv == 0) {
+        const int bad = factor_block(ldc[0], lane < P ? rdiag[lane & (kNB - 1)] : 1.0, lane);
+        if (lane == 0) nbad += bad;
+    }
+    __syncthreads();
+
+    // ---------------------------------------------------------------- Cholesky and L t = b
+    const int pp = lane & 15, kk = lane >> 4;
+    const unsigned loff = kk * LD + pp;
+    auto panel = [&](int p0, auto first) {
+        const int cur = (p0 / kNB) & 1, nxt = cur ^ 1;
+        double* pan = pan0 + (size_t)cur * cap * kLDP;
+        double* pann = pan0 + (size_t)nxt * cap * kLDP;
+        const double* blk = ldc[cur];
+        const int q0 = p0 + kNB;                 // first trailing row / column
+        const int below = max(P - q0, 0), n16 = (below + 15) / 16;
+        // rows below the block, and the right-hand sides, one thread each; a
+        // column of the block is read while the one before it is used
+        for (int rb = tid; rb < below + 2; rb += kThreads) {
+            double* pr = rb < below ? pan + rb * kLDP : bl + (rb - below) * LD + p0;
+            double v[kNB], lc[2][kNB];
+#pragma unroll
+            for (int k = 0; k < kNB; k++) v[k] = pr[k];
+#pragma unroll
+            for (int k = 0; k < kNB; k++) lc[0][k] = blk[k];
+#pragma unroll
+            for (int c = 0; c < kNB; c++) {
+#pragma unroll
+                for (int k = c + 1; k < kNB; k++) lc[(c + 1) & 1][k] = blk[(c + 1) * kNB + k];
+                const double xc = v[c] * lc[c & 1][c];
+                pr[c] = xc;
+#pragma unroll
+                for (int k = c + 1; k < kNB; k++) v[k] -= xc * lc[c & 1][k];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+        // Trailing update A[i][k] -= sum_c L[i][c] L[k][c] of tile (ti, tk):
+        // lane 16 kk + pp holds rows 16 tk + pp and 16 ti + pp, entry 4 s + kk;
+        // acc[v] sums row 16 ti + pp, column 16 tk + 4 v + kk (solve_body)
+        auto rows = [&](int tile, double* x) {
+            const double* q = pan + (16 * tile + pp) * kLDP + kk;
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++) x[s4] = q[4 * s4];
+        };
+        auto load_old = [&](int ti, int tk, double* o) {
+            if (first) {
+                const int i = min(q0 + 16 * ti + pp, P - 1);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int k = min(q0 + 16 * tk + 4 * v + kk, P - 1);
+                    o[v] = entry(a.S[(size_t)k * P + i], i, k);
+                }
+            } else {
+                const double* src = Lm + (size_t)(q0 + 16 * tk) * LD + q0 + 16 * ti;
+#pragma unroll
+                for (int v = 0; v < 4; v++) o[v] = (src + 4 * v * LD)[loff];
+            }
+        };
+        auto update = [&](const double* ra, const double* rb, double* o) {
+            double4v acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[s4], rb[s4], acc, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; v++) o[v] -= acc[v];
+        };
+        if (wv == 0) {
+            // the next diagonal block (identity past the matrix) and its factor
+            if (below > 0) {
+                double ra[4], o[4];
+                const double rd = q0 + pp < P ? rdiag[q0 + pp] : 1.0;
+                load_old(0, 0, o);
+                rows(0, ra);
+                update(ra, ra, o);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int k = 4 * v + kk;
+                    ldc[nxt][k * kNB + pp] = max(k, pp) < below ? o[v] : k == pp ? 1.0 : 0.0;
+                }
+                // the other wavefronts of its SIMD have the rest of the step to wait in
+                __builtin_amdgcn_s_setprio(3);
+                const int bad = factor_block(ldc[nxt], rd, lane);
+                __builtin_amdgcn_s_setprio(0);
+                if (lane == 0) nbad += bad;
+            }
+        } else {
+            // the other tiles of the triangle, row by row in equal shares
+            const int m = n16 * (n16 + 1) / 2 - 1;
+            int t = 1 + (wv - 1) * m / (NW - 1);
+            const int te = 1 + wv * m / (NW - 1);
+            if (t < te) {
+                int ti = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+                while (ti * (ti + 1) / 2 > t) ti--;
+                while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
+                ti = __builtin_amdgcn_readfirstlane(ti);
+                int tk = t - ti * (ti + 1) / 2;
+                double o[4], on[4], ra[4], rb[4];
+                load_old(ti, tk, o);
+                rows(ti, rb);
+                for (;;) {
+                    const int ni = tk == ti ? ti + 1 : ti, nk = tk == ti ? 0 : tk + 1;
+                    const bool more = t + 1 < te;
+                    if (more) load_old(ni, nk, on);
+                    rows(tk, ra);
+                    update(ra, rb, o);
+                    if (tk == 0) {
+                        double* dst = pann + (16 * (ti - 1) + pp) * kLDP + kk;
+#pragma unroll
+                        for (int v = 0; v < 4; v++) dst[4 * v] = o[v];
+                    } else {
+                        double* dst = Lm + (size_t)(q0 + 16 * tk) * LD + q0 + 16 * ti;
+#pragma unroll
+                        for (int v = 0; v < 4; v++) (dst + 4 * v * LD)[loff] = o[v];
+                    }
+                    if (!more) break;
+                    if (ni != ti) rows(ni, rb);
+                    ti = ni;
+                    tk = nk;
+                    t++;
+#pragma unroll
+                    for (int v = 0; v < 4; v++) o[v] = on[v];
+                }
+            }
+            // b -= L t of the rows below; the panel of the factor
+            for (int e = tid - 64; e < 2 * below; e += kThreads - 64) {
+                const int h = e >= below, i = h ? e - below : e;
+                const double* tb = bl + h * LD + p0;
+                double s = 0.0;
+#pragma unroll
+                for (int c = 0; c < kNB; c++) s += tb[c] * pan[i * kLDP + c];
+                bl[h * LD + q0 + i] -= s;
+            }
+            for (int i = tid - 64; i < kNB + below; i += kThreads - 64) {
+#pragma unroll
+                for (int c = 0; c < kNB; c++)
+                    (Lm + (size_t)(p0 + c) * LD + p0)[(unsigned)i] = i < kNB ? blk[c * kNB + i] : pan[(i - kNB) * kLDP + c];
+            }
+        }
+        __syncthreads();
+    };
+    panel(0, std::true_type{});
+    for (int p0 = kNB; p0 < P; p0 += kNB) panel(p0, std::false_type{});
+
+    // ---------------------------------------------------------------- L^T x = t
+    // Block by block from the last: each wavefront takes the solved part off
+    // one row, then the first one solves the block (lane l holds column l below
+    // the diagonal in f and 1 / L[l][l] in di; identity past the matrix), with
+    // the diagonal blocks in LDS (over the panels).
+    double* diag = pan0;   // [LD][kLDP]: L[p0 + j][c] of column c's block at c * kLDP + j
+    for (int e = tid; e < kNB * LD; e += kThreads) {
+        const int c = e / kNB, j = e % kNB;
+        diag[c * kLDP + j] = Lm[(size_t)c * LD + c / kNB * kNB + j];
+    }
+    constexpr int NQ = 10;   // 64 entries each: up to P = 656
+    double lr[NQ];
+    auto load_row = [&](int p0) {
+        const double* row = Lm + (size_t)(p0 + wv) * LD + p0 + kNB;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            if (p0 + kNB + 64 * q < P) lr[q] = row[(unsigned)min(64 * q + lane, P - 1 - kNB - p0)];
+        }
+    };
+    __syncthreads();
+    for (int p0 = LD - kNB; p0 >= 0; p0 -= kNB) {
+        const int pe = p0 + kNB;
+        if (pe < P) {
+            double sR = 0.0, sI = 0.0;
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                if (pe + 64 * q < P) {
+                    const int j = pe + 64 * q + lane;
+                    if (j < P) {
+                        sR += lr[q] * bl[j];
+                        sI += lr[q] * bl[LD + j];
+                    }
+                }
+            }
+            sR = wave_sum(sR);
+            sI = wave_sum(sI);
+            if (lane == 0) {
+                bl[p0 + wv] -= sR;
+                bl[LD + p0 + wv] -= sI;
+            }
+            __syncthreads();
+        }
+        if (p0 > 0) load_row(p0 - kNB);
+        if (wv == 0) {
+            const int i = p0 + pp;
+            double f[kNB];
+#pragma unroll
+            for (int j = 0; j < kNB; j++) f[j] = diag[i * kLDP + j];
+            const double di = diag[i * kLDP + pp];
+            double tR = bl[i], tI = bl[LD + i], xR = 0.0, xI = 0.0;
+            static_for<kNB>([&](auto jj) {
+                constexpr int j = kNB - 1 - jj;
+                const double uR = tR * di, uI = tI * di, fj = pp < j ? f[j] : 0.0;
+                xR = pp == j ? uR : xR;
+                xI = pp == j ? uI : xI;
+                tR -= fj * row_bcast<j>(uR);
+                tI -= fj * row_bcast<j>(uI);
+            });
+            if (lane < kNB) {
+                bl[i] = xR;
+                bl[LD + i] = xI;
+            }
+        }
+        __syncthreads();
+    }
+
+    // phi-dot on the (scaled) solution, then undo the scaling
+    double pr = 0.0, pi = 0.0;
+    for (int i = tid; i < P; i += kThreads) {
+        pr -= mO[i] * bl[i];
+        pi -= mO[i] * bl[LD + i];
+    }
+    pr = block_reduce(pr, red);
+    pi = block_reduce(pi, red);
+    for (int i = tid; i < P; i += kThreads) {
+        a.xdot[i] = bl[i] / sc[i];
+        a.xdot[P + i] = bl[LD + i] / sc[i];
     }
     if (tid == 0) {
         if (a.imag_time == 0)
@@ -650,70 +1053,69 @@ __device__ __forceinline__ void solve_qr_body(const SolveArgs& a)
     }
 }
 
-template <int NB>
-__global__ __launch_bounds__(kThreads) void solve_kernel(SolveArgs a)
-{
-    solve_body<NB>(a);
-}
+__global__ __launch_bounds__(kThreads) void solve_kernel(SolveArgs a) { solve_body(a); }
+template <bool RHS_LDS>
+__global__ __launch_bounds__(kThreads) void solve_ahead_kernel(SolveArgs a) { solve_ahead_body<RHS_LDS>(a); }
 __global__ __launch_bounds__(kThreads) void solve_qr_kernel(SolveArgs a)
 {
     solve_qr_body(a);
 }
 // one workgroup per system of a batch
-template <int NB>
+template <int FORM>
 __global__ __launch_bounds__(kThreads) void solve_batch_kernel(const SolveArgs* __restrict__ args)
 {
     const SolveArgs a = args[blockIdx.x];
     if (a.mean_sub)
         solve_qr_body(a);
+    else if constexpr (FORM > 0)
+        solve_ahead_body<FORM == 2>(a);
     else
-        solve_body<NB>(a);
+        solve_body(a);
 }
 
-// dynamic LDS of the Cholesky: the rows below a block at stride NB + 1 (also
-// holds the NB x NB blocks of the triangular solves)
-size_t solve_lds_bytes(int NB, int P) { return (size_t)(NB + 1) * std::max(P, NB) * sizeof(double); }
-constexpr size_t kMaxPanelLds = 150 * 1024;   // beside the static LDS (NB x NB block, reductions)
-// Block width: 16 up to P = 340, 32 above (measured crossover near P = 345:
-// at P = 296, 373 against 395 us; at P = 420, 738 against 705 us), 16 again
-// where the NB = 32 panel no longer fits in LDS
-constexpr int kNb16MaxP = 340;
-
-template <int NB>
-hipError_t launch_nb(const SolveArgs& a, hipStream_t st)
+// dynamic LDS of solve_body: the rows below a block at stride kLDP (also holds
+// the blocks of the triangular solves)
+size_t solve_lds_bytes(int P) { return (size_t)kLDP * std::max(P, kNB) * sizeof(double); }
+constexpr size_t kMaxPanelLds = 150 * 1024;   // beside the static LDS (blocks, reductions)
+// and of solve_ahead_body: both panel buffers and (rhs) the right-hand sides
+size_t solve_ahead_lds_bytes(int P, bool rhs)
 {
-    const size_t lds = solve_lds_bytes(NB, a.P);
-    auto kern = solve_kernel<NB>;
+    const size_t LD = ((size_t)P + kNB - 1) / kNB * kNB;
+    return ((size_t)(2 * ahead_rows(P) - kNB) * kLDP + (rhs ? 2 * LD : 0)) * sizeof(double);
+}
+// Form of the Cholesky: 2 (solve_ahead_body, right-hand sides in LDS) where the
+// buffers fit the 160 KB beside 4.5 KB of static LDS, P <= 560; 1 (right-hand
+// sides in the work buffer) where the panels alone do, P <= 608; 0 (solve_body)
+// above.  Whole call with its copies, solve_body against forms 2 and 1: 447 and
+// 229 us at P = 296, 1315 and 743 us at P = 560, 1640 and 938 us at P = 577.
+constexpr size_t kMaxAheadLds = 160 * 1024 - 4608;
+int solve_form(int P)
+{
+    return solve_ahead_lds_bytes(P, true) <= kMaxAheadLds ? 2 : solve_ahead_lds_bytes(P, false) <= kMaxAheadLds ? 1 : 0;
+}
+
+template <typename K, typename A>
+hipError_t launch_cholesky(K kern, int n, size_t lds, const A& args, hipStream_t st)
+{
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kern, dim3(1), dim3(kThreads), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(n), dim3(kThreads), lds, st, args);
     return hipGetLastError();
 }
 
 }  // namespace
 
-template <int NB>
-hipError_t launch_batch_nb(const SolveArgs* args_dev, int n, int P_max, hipStream_t st)
-{
-    // LDS: Cholesky panels or the QR transpositions (2 P ints)
-    const size_t lds = std::max(solve_lds_bytes(NB, P_max), 2 * (size_t)P_max * sizeof(int));
-    auto kern = solve_batch_kernel<NB>;
-    if (lds > 65536) {
-        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(kern, dim3(n), dim3(kThreads), lds, st, args_dev);
-    return hipGetLastError();
-}
-
 hipError_t launch_solve_batch(const SolveArgs* args_dev, int n, int P_max, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    if (P_max > kNb16MaxP && solve_lds_bytes(32, P_max) <= kMaxPanelLds)
-        return launch_batch_nb<32>(args_dev, n, P_max, st);
-    if (solve_lds_bytes(16, P_max) <= kMaxPanelLds) return launch_batch_nb<16>(args_dev, n, P_max, st);
+    const size_t qr = 2 * (size_t)P_max * sizeof(int);   // the QR's transpositions
+    const int form = solve_form(P_max);
+    const size_t lds = std::max(qr, form ? solve_ahead_lds_bytes(P_max, form == 2) : solve_lds_bytes(P_max));
+    if (form == 2) return launch_cholesky(solve_batch_kernel<2>, n, lds, args_dev, st);
+    if (form == 1) return launch_cholesky(solve_batch_kernel<1>, n, lds, args_dev, st);
+    if (lds <= kMaxPanelLds) return launch_cholesky(solve_batch_kernel<0>, n, lds, args_dev, st);
     return hipErrorInvalidValue;
 }
 
@@ -730,8 +1132,11 @@ hipError_t launch_solve(const SolveArgs& a, hipStream_t st)
         hipLaunchKernelGGL(solve_qr_kernel, dim3(1), dim3(kThreads), 2 * (size_t)a.P * sizeof(int), st, a);
         return hipGetLastError();
     }
-    if (a.P > kNb16MaxP && solve_lds_bytes(32, a.P) <= kMaxPanelLds) return launch_nb<32>(a, st);
-    if (solve_lds_bytes(16, a.P) <= kMaxPanelLds) return launch_nb<16>(a, st);
+    const int form = solve_form(a.P);
+    const size_t lds = form ? solve_ahead_lds_bytes(a.P, form == 2) : solve_lds_bytes(a.P);
+    if (form == 2) return launch_cholesky(solve_ahead_kernel<true>, 1, lds, a, st);
+    if (form == 1) return launch_cholesky(solve_ahead_kernel<false>, 1, lds, a, st);
+    if (lds <= kMaxPanelLds) return launch_cholesky(solve_kernel, 1, lds, a, st);
     return hipErrorInvalidValue;
 }
 
