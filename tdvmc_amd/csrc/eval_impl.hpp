@@ -306,19 +306,10 @@ __device__ __forceinline__ void eval_pairs(const KSys& sy, const typename Coord<
                         j = (int)x;
                         t = Prec<T>::fract_(x);
                     }
-                    // moments 1, t, t^2, t^3 of the pair's position in knot
-                    // interval j (FP64, the first an integer in the low half of
-                    // its slot: half the LDS traffic of a fourth FP64 add, mixed
-                    // measurement at N = 343 1.06 -> 1.04 ms (8192 walkers), 2-D
-                    // N = 400 3.86 -> 3.73 ms (16384)); the basis sums B_s are
-                    // rebuilt from them at the end
-                    const double td = (double)t, t2 = td * td, t3 = t2 * td;
-                    double* hb = hbase + j * (4 * HC);
-                    lds_add(reinterpret_cast<uint32_t*>(hb), 1u);
-                    lds_add(hb + HC, td);
-                    lds_add(hb + 2 * HC, t2);
-                    lds_add(hb + 3 * HC, t3);
-                    // u'(r), u''(r) per unit length on interval j
+                    // u'(r), u''(r) per unit length on interval j, read ahead of the
+                    // adds below, which the LDS takes in order (16384 walkers, the
+                    // other way round: mixed N = 343 1.59 -> 1.55 ms, 2-D N = 400
+                    // 3.73 -> 3.60; FP64 3.07 -> 2.97 and 5.71 -> 5.43)
                     const T* c = dsp + j * kDsplStride;
                     T c0, c1, c2, c3;
                     if constexpr (sizeof(T) == 4) {
@@ -334,6 +325,18 @@ __device__ __forceinline__ void eval_pairs(const KSys& sy, const typename Coord<
                         c2 = c[2];
                         c3 = c[3];
                     }
+                    // moments 1, t, t^2, t^3 of the pair's position in knot
+                    // interval j (FP64, the first an integer in the low half of
+                    // its slot: half the LDS traffic of a fourth FP64 add, mixed
+                    // measurement at N = 343 1.06 -> 1.04 ms (8192 walkers), 2-D
+                    // N = 400 3.86 -> 3.73 ms (16384)); the basis sums B_s are
+                    // rebuilt from them at the end
+                    const double td = (double)t, t2 = td * td, t3 = t2 * td;
+                    double* hb = hbase + j * (4 * HC);
+                    lds_add(reinterpret_cast<uint32_t*>(hb), 1u);
+                    lds_add(hb + HC, td);
+                    lds_add(hb + 2 * HC, t2);
+                    lds_add(hb + 3 * HC, t3);
                     const T upR = c0 + t * (c1 + t * c2);
                     const T fR = upR * rinv;
 #pragma unroll
