@@ -93,30 +93,67 @@ __device__ __forceinline__ double wave_rotate(double v)
     return *reinterpret_cast<double*>(&y);
 }
 
-// Sums of NV values over the WPW wavefronts of one walker: wave reductions,
-// then (WPW > 1) across the walker's waves through LDS.  With WPW = 1 no
-// barrier is needed.
+// Lane l's v of lane l ^ X within a row of 16 (X = 1, 2, 4, 8)
+template <int X>
+__device__ __forceinline__ double row_xor(double v)
+{
+    if constexpr (X == 1) return dpp_f<kDppXor1>(v);
+    if constexpr (X == 2) return dpp_f<kDppXor2>(v);
+    if constexpr (X == 8) return dpp_f<0x128>(v);   // row_ror:8
+    // row_shl:4 for the quads 0 and 2, row_shr:4 for 1 and 3
+    const int2 x = __builtin_bit_cast(int2, v);
+    int2 y;
+    y.x = __builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp(0, x.x, 0x104, 0xF, 0x5, false), x.x, 0x114, 0xF, 0xA, false);
+    y.y = __builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp(0, x.y, 0x104, 0xF, 0x5, false), x.y, 0x114, 0xF, 0xA, false);
+    return __builtin_bit_cast(double, y);
+}
+// One step of a sum over lanes l and l ^ X for n values that leaves (n + 1) / 2:
+// value 2 i for the lanes without bit X and 2 i + 1 for those with it
+template <int X, int NV>
+__device__ __forceinline__ void fold_sum(double (&v)[NV], int n, int lane)
+{
+    const bool odd = lane & X;
+#pragma unroll
+    for (int i = 0; i < n / 2; i++) {
+        const double keep = odd ? v[2 * i + 1] : v[2 * i], give = odd ? v[2 * i] : v[2 * i + 1];
+        v[i] = keep + row_xor<X>(give);
+    }
+    if (n & 1) v[n / 2] = v[n - 1] + row_xor<X>(v[n - 1]);
+}
+
+// Sums of NV <= 16 values over the WPW wavefronts of one walker, the same bits
+// as group_sum's tree.  The values share the lanes: after the four steps
+// within a row lane i holds value i, and one value's two steps across the rows
+// do for all (one tree per value was some 270 of a small walker's 900 vector
+// instructions: 16384 walkers, N = 64, FP64 144 -> 131 us, mixed 153 -> 135;
+// N = 343 mixed 1.55 -> 1.51 ms).  With WPW = 1 no barrier is needed.
 template <int WPW, int NV>
 __device__ __forceinline__ void walker_sum(double (&v)[NV], double* red, int wave, int lane)
 {
-    // wave sums by DPP steps and lane reads (no LDS round trips)
-#pragma unroll
-    for (int i = 0; i < NV; i++) v[i] = group_sum<64>(v[i]);
+    static_assert(NV <= 16, "a row of 16 lanes holds the sums");
+    fold_sum<1>(v, NV, lane);
+    fold_sum<2>(v, (NV + 1) / 2, lane);
+    fold_sum<4>(v, (NV + 3) / 4, lane);
+    fold_sum<8>(v, (NV + 7) / 8, lane);
+    // rows 0 and 1, 2 and 3, then both halves
+    auto halves = [](double x, auto swap) {
+        const uint2 u = __builtin_bit_cast(uint2, x);
+        const auto lo = swap(u.x), hi = swap(u.y);
+        return __builtin_bit_cast(double, make_uint2(lo[0], hi[0])) + __builtin_bit_cast(double, make_uint2(lo[1], hi[1]));
+    };
+    double s = halves(v[0], [](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    s = halves(s, [](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
     if constexpr (WPW > 1) {
         // (red is written only here, once per walker: no barrier before the writes)
-        if (lane == 0) {
-#pragma unroll
-            for (int i = 0; i < NV; i++) red[wave * NV + i] = v[i];
-        }
+        if (lane < NV) red[wave * NV + lane] = s;
         __syncthreads();
+        const int i = min(lane & 15, NV - 1);
+        s = 0.0;
 #pragma unroll
-        for (int i = 0; i < NV; i++) {
-            double s = 0.0;
-#pragma unroll
-            for (int w = 0; w < WPW; w++) s += red[w * NV + i];
-            v[i] = s;
-        }
+        for (int w = 0; w < WPW; w++) s += red[w * NV + i];
     }
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] = readlane_f(s, i);
 }
 constexpr int kRedDoubles = 40;   // >= 4 waves x 10 values
 
