@@ -706,11 +706,11 @@ KTables<T> tables_of(tdvmc_ctx* ctx, DevTables<T>& t)
 
 // packed: device parameters [2P + 2] to take (null: dUR, dUI), which then are in force
 template <typename T>
-int ensure_tables(tdvmc_ctx* ctx, DevTables<T>& t, bool force, const double* packed = nullptr)
+int ensure_tables(tdvmc_ctx* ctx, DevTables<T>& t, bool force, const double* packed = nullptr, int* zero = nullptr)
 {
     if (!t.dirty && !force) return TDVMC_OK;
     HIPC(launch_prep_tables<T>(ctx->sy, packed, ctx->dUR, ctx->dUI, ctx->dKmap, ctx->dKpos, t.kv, t.spl, t.dspl,
-                               t.alpha, t.kag, t.kagr, ctx->dNuBeta, ctx->stream));
+                               t.alpha, t.kag, t.kagr, ctx->dNuBeta, zero, ctx->stream));
     t.dirty = false;
     return TDVMC_OK;
 }
@@ -866,7 +866,8 @@ int resolve_precision(tdvmc_ctx* ctx, int precision, int* out)
     return TDVMC_OK;
 }
 
-int enqueue_sweep(tdvmc_ctx* ctx, int prec, int64_t n_moves, uint64_t seed, bool want_rho = false)
+// tick_later: the measurement enqueued next steps the epoch (enqueue_eval)
+int enqueue_sweep(tdvmc_ctx* ctx, int prec, int64_t n_moves, uint64_t seed, bool want_rho = false, bool tick_later = false)
 {
     if (n_moves <= 0) return TDVMC_OK;
     SweepArgs a;
@@ -888,15 +889,16 @@ int enqueue_sweep(tdvmc_ctx* ctx, int prec, int64_t n_moves, uint64_t seed, bool
     }
     rc = prof_end(ctx, "sweep", ev);
     if (rc) return rc;
-    HIPC(launch_add_u32(ctx->dEpoch, 1u, ctx->stream));
+    if (!tick_later) HIPC(launch_add_u32(ctx->dEpoch, 1u, ctx->stream));
     if (!ctx->in_capture) ctx->trials_total += n_moves * ctx->W;
     return TDVMC_OK;
 }
 
 // eval of the context walkers into sample rows [row0, row0 + W); use_rho:
 // take rho_k from the sweep that just ran instead of recomputing it
-int enqueue_eval(tdvmc_ctx* ctx, int prec, int64_t row0, bool use_rho = false, const double* R = nullptr)
+int enqueue_eval(tdvmc_ctx* ctx, int prec, int64_t row0, bool use_rho = false, const double* R = nullptr, bool tick = false)
 {
+    uint32_t* const epoch = tick ? ctx->dEpoch : nullptr;
     const bool rho = use_rho && ctx->sy.Kh > 0;
     if (!R) R = ctx->dR;
     const int P = P_of(ctx);
@@ -907,12 +909,13 @@ int enqueue_eval(tdvmc_ctx* ctx, int prec, int64_t row0, bool use_rho = false, c
         HIPC((launch_eval<float, float>(ctx->sy, tables_of(ctx, ctx->tf), R, ctx->W, ctx->dExpo + row0,
                                         ctx->dER + row0, ctx->dEI + row0, ctx->dO32 + row0 * P,
                                         ctx->dOther + row0 * 9, nullptr, nullptr, nullptr,
-                                        rho ? reinterpret_cast<const float*>(ctx->dRho) : nullptr, ctx->stream)));
+                                        rho ? reinterpret_cast<const float*>(ctx->dRho) : nullptr, ctx->stream, nullptr,
+                                        epoch)));
     } else {
         HIPC((launch_eval<double, double>(ctx->sy, tables_of(ctx, ctx->td), R, ctx->W, ctx->dExpo + row0,
                                           ctx->dER + row0, ctx->dEI + row0, ctx->dO64 + row0 * P,
                                           ctx->dOther + row0 * 9, nullptr, nullptr, nullptr,
-                                          rho ? ctx->dRho : nullptr, ctx->stream)));
+                                          rho ? ctx->dRho : nullptr, ctx->stream, nullptr, epoch)));
     }
     return prof_end(ctx, "eval", ev);
 }
@@ -1188,10 +1191,11 @@ int enqueue_stage_samples(tdvmc_ctx* ctx, int prec, uint64_t seed, bool keep = f
     if (rc) return rc;
     const size_t per = (size_t)ctx->W * ctx->sy.N * ctx->sy.D;
     for (int s = 0; s < ctx->spw; s++) {
-        rc = enqueue_sweep(ctx, prec, ctx->therm_moves, seed, true);
+        const bool tick = ctx->therm_moves > 0 && ctx->W > 0;
+        rc = enqueue_sweep(ctx, prec, ctx->therm_moves, seed, true, tick);
         if (rc) return rc;
         const bool swept = ctx->therm_moves > 0 || (s == 0 && ctx->init_moves > 0);
-        rc = enqueue_eval(ctx, prec, (int64_t)s * ctx->W, swept);
+        rc = enqueue_eval(ctx, prec, (int64_t)s * ctx->W, swept, nullptr, tick);
         if (rc) return rc;
         if (keep && ctx->spw > 1)
             HIPC(hipMemcpyAsync(ctx->dSamp + s * per, ctx->dR, per * sizeof(double), hipMemcpyDeviceToDevice,
@@ -1218,17 +1222,19 @@ int enqueue_reuse_samples(tdvmc_ctx* ctx, int prec)
     return enqueue_moments(ctx, prec, (int64_t)ctx->spw * ctx->W);
 }
 
-int enqueue_prep(tdvmc_ctx* ctx, int prec, const double* x)
+int enqueue_prep(tdvmc_ctx* ctx, int prec, const double* x, int* zero)
 {
-    if (prec == TDVMC_MIXED) return ensure_tables(ctx, ctx->tf, true, x);
-    return ensure_tables(ctx, ctx->td, true, x);
+    if (prec == TDVMC_MIXED) return ensure_tables(ctx, ctx->tf, true, x, zero);
+    return ensure_tables(ctx, ctx->td, true, x, zero);
 }
 
 // f(x): parameters x (packed, device) -> xdot.  reuse: evaluate the kept
-// samples instead of sampling; keep: keep this stage's samples for reuse
+// samples instead of sampling; keep: keep this stage's samples for reuse.  The
+// first stage of a step (xdot dK[0]) also clears dStatus, to which the step's
+// solves add their non-positive pivots.
 int enqueue_rhs(tdvmc_ctx* ctx, int prec, const double* x, double* xdot, bool reuse = false, bool keep = false)
 {
-    int rc = enqueue_prep(ctx, prec, x);
+    int rc = enqueue_prep(ctx, prec, x, xdot == ctx->dK[0] ? ctx->dStatus : nullptr);
     if (rc) return rc;
     rc = reuse ? enqueue_reuse_samples(ctx, prec) : enqueue_stage_samples(ctx, prec, ctx->seed, keep);
     if (rc) return rc;
@@ -1239,12 +1245,14 @@ int enqueue_tdvp_step(tdvmc_ctx* ctx, int prec, int ode, double dt)
 {
     const int P = P_of(ctx);
     int rc;
-    // the solves of this step add their non-positive pivots to dStatus
-    HIPC(launch_fill_u32(reinterpret_cast<uint32_t*>(ctx->dStatus), 0u, 1, ctx->stream));
+    // the last update also writes the tables' parameters, unless something follows it
+    const bool last = !ctx->normalize_wf && !ctx->adjust_params && (ode == 0 || ode == 2 || ode == 3);
+    double* const uR = last ? ctx->dUR : nullptr;
+    double* const uI = last ? ctx->dUI : nullptr;
     if (ode == 0) {
         rc = enqueue_rhs(ctx, prec, ctx->dX, ctx->dK[0]);
         if (rc) return rc;
-        HIPC(launch_axpy_params(P, ctx->dX, ctx->dK[0], dt, ctx->dX, ctx->stream));
+        HIPC(launch_axpy_params(P, ctx->dX, ctx->dK[0], dt, ctx->dX, ctx->stream, uR, uI));
     } else if (ode == 2) {
         rc = enqueue_rhs(ctx, prec, ctx->dX, ctx->dK[0]);
         if (rc) return rc;
@@ -1257,7 +1265,7 @@ int enqueue_tdvp_step(tdvmc_ctx* ctx, int prec, int ode, double dt)
         HIPC(launch_axpy_params(P, ctx->dX, ctx->dK[2], dt, ctx->dXtmp, ctx->stream));
         rc = enqueue_rhs(ctx, prec, ctx->dXtmp, ctx->dK[3]);
         if (rc) return rc;
-        HIPC(launch_rk4_combine(P, ctx->dX, ctx->dK[0], ctx->dK[1], ctx->dK[2], ctx->dK[3], dt, ctx->stream));
+        HIPC(launch_rk4_combine(P, ctx->dX, ctx->dK[0], ctx->dK[1], ctx->dK[2], ctx->dK[3], dt, ctx->stream, uR, uI));
     } else if (ode == 3) {
         // CalculateNextParametersRK4ReuseSamples (src/TDVMC.cpp:2037-2103):
         // fresh samples for k1, the same samples for k2..k4
@@ -1272,7 +1280,7 @@ int enqueue_tdvp_step(tdvmc_ctx* ctx, int prec, int ode, double dt)
         HIPC(launch_axpy_params(P, ctx->dX, ctx->dK[2], dt, ctx->dXtmp, ctx->stream));
         rc = enqueue_rhs(ctx, prec, ctx->dXtmp, ctx->dK[3], true);
         if (rc) return rc;
-        HIPC(launch_rk4_combine(P, ctx->dX, ctx->dK[0], ctx->dK[1], ctx->dK[2], ctx->dK[3], dt, ctx->stream));
+        HIPC(launch_rk4_combine(P, ctx->dX, ctx->dK[0], ctx->dK[1], ctx->dK[2], ctx->dK[3], dt, ctx->stream, uR, uI));
     } else if (ode == 1 || ode == 5) {
         // CalculateNextParametersPC (src/TDVMC.cpp:1855-1910): predictor
         // x + dt k1, one corrector x + dt/2 (k1 + k2) on fresh samples;
@@ -1300,7 +1308,7 @@ int enqueue_tdvp_step(tdvmc_ctx* ctx, int prec, int ode, double dt)
     if (ctx->normalize_wf || ctx->adjust_params)
         HIPC(launch_post_step(P, ctx->dX, ctx->dExpo + (int64_t)(ctx->spw - 1) * ctx->W, ctx->normalize_wf,
                               ctx->adjust_params, ctx->sy.off_pair, ctx->sy.P_s, ctx->stream));
-    HIPC(launch_unpack_params(P, ctx->dX, ctx->dUR, ctx->dUI, ctx->stream));
+    if (!last) HIPC(launch_unpack_params(P, ctx->dX, ctx->dUR, ctx->dUI, ctx->stream));
     return TDVMC_OK;
 }
 

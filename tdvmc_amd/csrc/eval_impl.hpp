@@ -63,6 +63,7 @@ struct EvalOut {
     double* lap;      // [W][N][2] or null (PP)
     double* outer;    // [W] count of pairs beyond the cutoff, or null
     double* bsum = nullptr;   // [W][P_s + 2] basis sums B_s before the BC map, or null
+    uint32_t* tick = nullptr; // counter to step (the sweep's epoch, which a launch of its own took 5 us for), or null
     __device__ __forceinline__ void O_store(int64_t w, int P, int k, double v) const { O[w * P + k] = (TO)v; }
 };
 
@@ -1228,6 +1229,7 @@ __global__ __launch_bounds__(kThreads, 4) void eval_kernel(KSys sy, KTables<T> t
 {
     constexpr int NS = 4 / WPW;
     const int slot = NS == 1 ? 0 : threadIdx.x / (64 * WPW);
+    if (out.tick && blockIdx.x == 0 && threadIdx.x == 0) *out.tick += 1;
     eval_body<T, D, PP, PER, TO, WPW>(sy, tb, Rg, W, out, rho_in, (int64_t)blockIdx.x * NS + slot, slot, slot_bytes);
 }
 

@@ -68,10 +68,10 @@ static hipError_t launch_eval_d(const KSys& sy, const KTables<T>& tb, const doub
 template <typename T, typename TO>
 hipError_t launch_eval(const KSys& sy, const KTables<T>& tb, const double* R, int64_t W, double* expo, double* ER,
                        double* EI, TO* O, double* other, double* grad, double* lap, double* outer,
-                       const T* rho_in, hipStream_t st, double* bsum)
+                       const T* rho_in, hipStream_t st, double* bsum, uint32_t* tick)
 {
     if (W <= 0) return hipSuccess;
-    EvalOut<TO> o{expo, ER, EI, O, other, grad, lap, outer, bsum};
+    EvalOut<TO> o{expo, ER, EI, O, other, grad, lap, outer, bsum, tick};
     const bool pp = grad != nullptr;
     switch (sy.D) {
     case 1: return launch_eval_d<T, 1, TO>(sy, tb, R, W, o, rho_in, pp, st);

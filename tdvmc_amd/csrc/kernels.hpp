@@ -9,22 +9,24 @@
 namespace tdvmc {
 
 // ---- parameter-derived tables (kernels_misc.hip)
-// packed: parameters [2P + 2] to take (and to copy to uR, uI first), or null: uR, uI as they are
+// packed: parameters [2P + 2] to take (and to copy to uR, uI first), or null: uR, uI as they are;
+// zero: a word to clear on the way, or null
 template <typename T>
 hipError_t launch_prep_tables(const KSys& sy, const double* packed, double* uR, double* uI, const int* kmap,
                               const int* kpos, const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr,
-                              const double* nubeta, hipStream_t st);
+                              const double* nubeta, int* zero, hipStream_t st);
 
 // ---- evaluation (kernels_eval.hip); grad/lap non-null selects the per-particle variant
 // LDS of one walker with wpw wavefronts (single contexts: 4)
 template <typename T>
 size_t eval_lds_bytes(const KSys& sy, bool per_particle, int wpw = 4);
 // rho_in: [W][K][2] rho_k of the walkers as left by the sweep (skips the
-// rho_k pass), or null to compute it from the coordinates
+// rho_k pass), or null to compute it from the coordinates; tick: a counter to
+// step by one, or null
 template <typename T, typename TO>
 hipError_t launch_eval(const KSys& sy, const KTables<T>& tb, const double* R, int64_t W, double* expo, double* ER,
                        double* EI, TO* O, double* other, double* grad, double* lap, double* outer,
-                       const T* rho_in, hipStream_t st, double* bsum = nullptr);
+                       const T* rho_in, hipStream_t st, double* bsum = nullptr, uint32_t* tick = nullptr);
 
 // ---- Metropolis sweeps (kernels_sweep.hip)
 struct SweepArgs {
@@ -193,10 +195,12 @@ hipError_t launch_moments_batch(const MomentsItem* items_dev, int n, int nchunk_
 hipError_t launch_post_step(int P, double* x, const double* expo, int normalize, int adjust, int off, int n,
                             hipStream_t st);
 // y = x0 + c * xdot  over the 2P+2 entries (alpha R, alpha I, phi R, phi I)
-hipError_t launch_axpy_params(int P, const double* x0, const double* xdot, double c, double* y, hipStream_t st);
+// (uR, uI: where given, the tables' copies are written too, as launch_unpack_params does)
+hipError_t launch_axpy_params(int P, const double* x0, const double* xdot, double c, double* y, hipStream_t st,
+                              double* uR = nullptr, double* uI = nullptr);
 // x += dt/6 (k1 + 2 k2 + 2 k3 + k4)
 hipError_t launch_rk4_combine(int P, double* x, const double* k1, const double* k2, const double* k3,
-                              const double* k4, double dt, hipStream_t st);
+                              const double* k4, double dt, hipStream_t st, double* uR = nullptr, double* uI = nullptr);
 // params (2P+2 packed) -> uR, uI arrays used by the tables
 // y = x + (k1 + k2) dt / 2 on the packed parameter vector [2P+2]
 hipError_t launch_pc_combine(int P, const double* x, const double* k1, const double* k2, double dt, double* y,

@@ -160,8 +160,9 @@ __global__ __launch_bounds__(64) void prep_tables_kernel(KSys sy, const double* 
                                                          const T* __restrict__ kv, T* __restrict__ spl,
                                                          T* __restrict__ dspl, T* __restrict__ alpha,
                                                          T* __restrict__ kag, T* __restrict__ kagr,
-                                                         const double* __restrict__ nubeta)
+                                                         const double* __restrict__ nubeta, int* __restrict__ zero)
 {
+    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
     extern __shared__ __align__(16) unsigned char smem[];
     prep_tables_body(sy, packed, uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta,
                      reinterpret_cast<double*>(smem), blockIdx.x, gridDim.x);
@@ -300,17 +301,34 @@ __global__ __launch_bounds__(256) void moments_reduce_kernel(const MomentsItem* 
     }
 }
 
-__global__ void axpy_params_kernel(int n, const double* x0, const double* xdot, double c, double* y)
+// Entry i of the packed parameters also to the tables' copy, where the step
+// ends with this update: a launch of its own is 4 us after a kernel this short
+__device__ __forceinline__ void put_param(double v, int i, int n, double* uR, double* uI)
 {
-    for (int i = threadIdx.x + blockIdx.x * blockDim.x; i < n; i += blockDim.x * gridDim.x)
+    const int P = n / 2 - 1;
+    if (!uR) return;
+    if (i < 2 * P)
+        (i < P ? uR + i : uI + i - P)[0] = v;
+    else
+        (i == 2 * P ? uR : uI)[P] = v;   // phi R, phi I
+}
+
+__global__ void axpy_params_kernel(int n, const double* x0, const double* xdot, double c, double* y, double* uR,
+                                   double* uI)
+{
+    for (int i = threadIdx.x + blockIdx.x * blockDim.x; i < n; i += blockDim.x * gridDim.x) {
         y[i] = x0[i] + c * xdot[i];
+        put_param(y[i], i, n, uR, uI);
+    }
 }
 
 __global__ void rk4_combine_kernel(int n, double* x, const double* k1, const double* k2, const double* k3,
-                                   const double* k4, double dt)
+                                   const double* k4, double dt, double* uR, double* uI)
 {
-    for (int i = threadIdx.x + blockIdx.x * blockDim.x; i < n; i += blockDim.x * gridDim.x)
+    for (int i = threadIdx.x + blockIdx.x * blockDim.x; i < n; i += blockDim.x * gridDim.x) {
         x[i] = x[i] + ((k1[i] + 2.0 * k2[i] + 2.0 * k3[i] + k4[i]) / 6.0) * dt;
+        put_param(x[i], i, n, uR, uI);
+    }
 }
 
 // predictor-corrector combination of src/TDVMC.cpp:1899-1902: y = x + (k1 + k2) dt/2
@@ -411,33 +429,33 @@ hipError_t launch_adjoint_outer(const double* outer, const double* gbar, int64_t
 template <typename T>
 hipError_t launch_prep_tables(const KSys& sy, const double* packed, double* uR, double* uI, const int* kmap,
                               const int* kpos, const T* kv, T* spl, T* dspl, T* alpha, T* kag, T* kagr,
-                              const double* nubeta, hipStream_t st)
+                              const double* nubeta, int* zero, hipStream_t st)
 {
     if (sy.nu && !nubeta) return hipErrorInvalidValue;
     const int n = 2 * (sy.P_s - 1) + sy.Kh;
     hipLaunchKernelGGL(prep_tables_kernel<T>, dim3((n + 63) / 64), dim3(64), 2 * sy.P_s * sizeof(double), st, sy, packed,
-                       uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta);
+                       uR, uI, kmap, kpos, kv, spl, dspl, alpha, kag, kagr, nubeta, zero);
     return hipGetLastError();
 }
 template hipError_t launch_prep_tables<float>(const KSys&, const double*, double*, double*, const int*, const int*,
-                                              const float*, float*, float*, float*, float*, float*, const double*,
-                                              hipStream_t);
+                                              const float*, float*, float*, float*, float*, float*, const double*, int*, hipStream_t);
 template hipError_t launch_prep_tables<double>(const KSys&, const double*, double*, double*, const int*, const int*,
                                                const double*, double*, double*, double*, double*, double*,
-                                               const double*, hipStream_t);
+                                               const double*, int*, hipStream_t);
 
-hipError_t launch_axpy_params(int P, const double* x0, const double* xdot, double c, double* y, hipStream_t st)
+hipError_t launch_axpy_params(int P, const double* x0, const double* xdot, double c, double* y, hipStream_t st,
+                              double* uR, double* uI)
 {
     const int n = 2 * P + 2;
-    hipLaunchKernelGGL(axpy_params_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, x0, xdot, c, y);
+    hipLaunchKernelGGL(axpy_params_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, x0, xdot, c, y, uR, uI);
     return hipGetLastError();
 }
 
 hipError_t launch_rk4_combine(int P, double* x, const double* k1, const double* k2, const double* k3,
-                              const double* k4, double dt, hipStream_t st)
+                              const double* k4, double dt, hipStream_t st, double* uR, double* uI)
 {
     const int n = 2 * P + 2;
-    hipLaunchKernelGGL(rk4_combine_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, x, k1, k2, k3, k4, dt);
+    hipLaunchKernelGGL(rk4_combine_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, x, k1, k2, k3, k4, dt, uR, uI);
     return hipGetLastError();
 }
 
