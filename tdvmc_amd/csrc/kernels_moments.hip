@@ -386,7 +386,7 @@ inline bool moments_small(int64_t W, int P, int mode)
 {
     // sums, means, packing, products and reduction are a launch each, 41 to
     // 62 us together at these sizes whatever the work; the two launches take
-    // 12 us (16 columns, 1024 walkers) to 25 us (34 columns, 16384 walkers).
+    // 9 us (16 columns, 1024 walkers) to 14 us (34 columns, 16384 walkers).
     // More columns or chunks would outgrow the LDS of the combination.
     return mode == 0 && P + 2 <= kSmallCols && W <= (int64_t)kSmallRows * kSmallChunks;
 }
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(1024) void small_combine_kernel(const double* __res
             const double m = red[tid] / (double)W;
             mt[tid] = m;
             // the diagonal tiles hold every column once
-            if (I == J && tid < 16 && col < Pa) {
+            if (I == J && blockIdx.y == 0 && tid < 16 && col < Pa) {
                 if (col >= P)
                     mean[P_full + (col - P)] = m;
                 else if (!outmap)
@@ -486,17 +486,21 @@ __global__ __launch_bounds__(1024) void small_combine_kernel(const double* __res
         }
         __syncthreads();
     }
-    // element (i, j) of the tile: chunks tid / 256, + 4, ..., then the four sums
-    const int e = tid & 255, i = e >> 4, j = e & 15;
+    // element (i, j) of the tile, 64 a workgroup: chunks tid / 64, + 16, ..., then
+    // the 16 sums (a workgroup for all 256 elements had four times the loads in a
+    // row: 16 against 8.6 us at 34 columns and 256 chunks)
+    const int e = blockIdx.y * 64 + (tid & 63), i = e >> 4, j = e & 15;
     const double mi = mt[i], mj = mt[16 + j];
     double s = 0.0;
 #pragma unroll 8
-    for (int k = tid >> 8; k < chunks; k += 4)
+    for (int k = tid >> 6; k < chunks; k += 16)
         s += part[((size_t)k * ntiles + t) * 256 + e] + rows(k) * (cm[k * 32 + i] - mi) * (cm[k * 32 + 16 + j] - mj);
     red[tid] = s;
     __syncthreads();
-    if (tid < 256 && !(I == J && i > j)) {
-        s = ((red[e] + red[256 + e]) + red[512 + e]) + red[768 + e];
+    if (tid < 64 && !(I == J && i > j)) {
+        s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) s += red[tid + 64 * q];
         store_cov(s * (1.0 / (double)W), 16 * I + i, 16 * J + j, P, outmap, P_full, S, F);
     }
 }
@@ -538,7 +542,7 @@ hipError_t launch_moments(const TO* O, const double* ER, const double* EI, int64
         double* tiles = static_cast<double*>(wk.xt);
         hipLaunchKernelGGL(small_partial_kernel<TO>, dim3(chunks), dim3(256), 0, st, O, ER, EI, W, Pc, cs, g.nb, wk.colsum,
                            tiles);
-        hipLaunchKernelGGL(small_combine_kernel, dim3(g.ntiles), dim3(1024), 0, st, wk.colsum, tiles, chunks, W, Pc, g.nb,
+        hipLaunchKernelGGL(small_combine_kernel, dim3(g.ntiles, 4), dim3(1024), 0, st, wk.colsum, tiles, chunks, W, Pc, g.nb,
                            wk.outmap, P, mean, S, F);
         return hipGetLastError();
     }
