@@ -48,7 +48,7 @@ struct DevTables {
     T* kv = nullptr;
     T* alpha = nullptr;
     T* kag = nullptr;
-    T* kagr = nullptr;   // FP64 only
+    T* kagr = nullptr;   // FP64 only, behind kag
     bool dirty = true;
 };
 
@@ -109,7 +109,7 @@ struct tdvmc_ctx {
     std::vector<double> kv_d;
     std::vector<int> kmap;            // [Kh][2] parameter slots of k and -k
     std::vector<int> kpos, krun;      // run order of the k-space terms (KTables)
-    int* dKmap = nullptr;
+    int* dKmap = nullptr;   // with dKpos and dKrun behind it
     int* dKpos = nullptr;
     int* dKrun = nullptr;
 
@@ -1440,17 +1440,15 @@ int alloc_ctx(tdvmc_ctx* ctx)
                         hipMemcpyHostToDevice, ctx->stream));
     HIPC(hipMemcpyAsync(ctx->dMomOut, ctx->mom_outmap.data(), ctx->mom_outmap.size() * sizeof(int),
                         hipMemcpyHostToDevice, ctx->stream));
-    HIPC(dalloc(&ctx->dKmap, ctx->kmap.size()));
-    HIPC(hipMemcpyAsync(ctx->dKmap, ctx->kmap.data(), ctx->kmap.size() * sizeof(int), hipMemcpyHostToDevice,
-                        ctx->stream));
+    // the k-space terms' integer tables in one buffer and one copy
+    std::vector<int> ktab = ctx->kmap;
+    ktab.insert(ktab.end(), ctx->kpos.begin(), ctx->kpos.end());
+    ktab.insert(ktab.end(), ctx->krun.begin(), ctx->krun.end());
+    HIPC(dalloc(&ctx->dKmap, ktab.size()));
+    HIPC(hipMemcpyAsync(ctx->dKmap, ktab.data(), ktab.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     if (ctx->sy.Kh > 0) {
-        HIPC(dalloc(&ctx->dKpos, ctx->kpos.size()));
-        HIPC(dalloc(&ctx->dKrun, ctx->krun.size()));
-        HIPC(dalloc(&ctx->td.kagr, 8 * (size_t)K));
-        HIPC(hipMemcpyAsync(ctx->dKpos, ctx->kpos.data(), ctx->kpos.size() * sizeof(int), hipMemcpyHostToDevice,
-                            ctx->stream));
-        HIPC(hipMemcpyAsync(ctx->dKrun, ctx->krun.data(), ctx->krun.size() * sizeof(int), hipMemcpyHostToDevice,
-                            ctx->stream));
+        ctx->dKpos = ctx->dKmap + ctx->kmap.size();
+        ctx->dKrun = ctx->dKpos + ctx->kpos.size();
     }
     HIPC(dalloc(&ctx->tf.spl, (size_t)Ps * 8));
     if (ctx->sy.nu) {
@@ -1469,7 +1467,8 @@ int alloc_ctx(tdvmc_ctx* ctx)
     HIPC(dalloc(&ctx->td.spl, (size_t)Ps * 8));
     HIPC(dalloc(&ctx->td.kv, 4 * (size_t)K));
     HIPC(dalloc(&ctx->td.alpha, 2 * (size_t)K));
-    HIPC(dalloc(&ctx->td.kag, 8 * (size_t)K));
+    HIPC(dalloc(&ctx->td.kag, 16 * (size_t)K));   // in term order, then in run order
+    if (ctx->sy.Kh > 0) ctx->td.kagr = ctx->td.kag + 8 * (size_t)K;
     HIPC(hipMemcpyAsync(ctx->tf.kv, ctx->kv_f.data(), ctx->kv_f.size() * sizeof(float), hipMemcpyHostToDevice,
                         ctx->stream));
     HIPC(hipMemcpyAsync(ctx->td.kv, ctx->kv_d.data(), ctx->kv_d.size() * sizeof(double), hipMemcpyHostToDevice,
@@ -1523,8 +1522,6 @@ void release(tdvmc_ctx* ctx)
     dfree(ctx->dMomOut);
     dfree(ctx->dMeanCols);
     dfree(ctx->dKmap);
-    dfree(ctx->dKpos);
-    dfree(ctx->dKrun);
     dfree(ctx->tf.dspl);
     dfree(ctx->td.dspl);
     dfree(ctx->tf.kv);
@@ -1534,7 +1531,6 @@ void release(tdvmc_ctx* ctx)
     dfree(ctx->td.kv);
     dfree(ctx->td.alpha);
     dfree(ctx->td.kag);
-    dfree(ctx->td.kagr);
     dfree(ctx->dO64);
     dfree(ctx->dO32);
     dfree(ctx->dER);
