@@ -21,8 +21,9 @@
 //   vectors' totals in order:
 //   S = (C^2 + S^2) / (N n_k).
 // FP64 form: distances by the reference's minimum image (src/Utils.cpp:266-281)
-// and FP64 division for the bin, powers by complex recurrence from one
-// sincospi.  Mixed form: FP32 distances from the wrapping difference of 32-bit
+// and the bin of the reference's FP64 division, powers by complex recurrence
+// from one sincospi; in 2-D and 3-D obs_mfma_kernel below takes S(k) as a matrix
+// product and the bins from thresholds of r^2.  Mixed form: FP32 distances from the wrapping difference of 32-bit
 // box fractions (exact minimum image), FP32 powers each from its own reduced
 // phase, FP32 sums per chunk added in FP64.
 

@@ -654,7 +654,7 @@ static hipError_t launch_sweep_l(const KSys& sy, const KTables<T>& tb, const Swe
         // slots of about 450 per trial in the FP32 form): every count has its
         // kernel, but 7, which no default lane count leads to (258 terms of a
         // 2-D system with 512 k on 64 lanes, 5 instead of 8: mixed sweep
-        // 35.2 -> 30.1 ms at 131072 walkers, N = 400)
+        // 35.2 -> 29.6 ms at 131072 walkers, N = 400)
         switch (kpl) {
         case 1: return launch_sweep_k<T, D, LPW, 1, PER>(sy, tb, a, st);
         case 2: return launch_sweep_k<T, D, LPW, 2, PER>(sy, tb, a, st);
