@@ -176,9 +176,35 @@ __host__ __device__ inline bool sweep_phase_table(const KSys& sy, int lpw)
     return sweep_base_lds<T>(sy, lpw) + (kThreads / lpw) * (size_t)sweep_phase_len(sy) * 2 * sizeof(T) <= kLdsMax;
 }
 
+// Spline rows of the mixed form 256 bytes apart, in 16 copies: the conversion of
+// r / h to an integer writes it into byte 1 of the row's LDS address, whose
+// other bytes stay (the lane's copy in byte 0, zeros above).  One instruction
+// instead of a conversion and a shift-add, for both distances of a pair's 41
+// issue slots, and no two of the 16 lanes that the LDS serves together share a
+// bank.  Same values, same bits.
+// Taken where five workgroups fit the LDS of a CU (the registers allow no
+// more); below that the wavefronts it costs take the gain back.  Sweep of
+// 16384 walkers in us, plain and wide: 2-D N = 400, 258 terms, 64 lanes (27 KB)
+// 3829 / 3680; 3-D, 32 lanes, N = 64 (24 KB) 112 / 109, N = 125 (30 KB) 370 / 362,
+// N = 160 (33 KB) 529 / 534, N = 260 (43 KB) 1240 / 1341, N = 343 (51 KB) 2478 /
+// 2485 (one workgroup of 1024 threads and one table for it: 2587).
+constexpr int kWide = 16;
+template <typename T>
+inline size_t sweep_wide_lds(const KSys& sy, int lpw)
+{
+    return sweep_base_lds<T>(sy, lpw) + (kWide - 1) * sizeof(T) * 4 * (size_t)sweep_table_len(sy);
+}
+template <typename T>
+inline bool sweep_wide(const KSys& sy, int lpw)
+{
+    // (32 KB hold at most 128 rows: a byte counts them)
+    return sizeof(T) == 4 && sy.periodic && !sy.nu && sweep_wide_lds<T>(sy, lpw) <= kLdsMax / 5;
+}
+typedef const __attribute__((address_space(3))) unsigned char* LdsBytes;
+
 // One workgroup's share of the sweep: walkers blk * WPB .. (blk + 1) * WPB - 1
-// of the system described by (sy, tb, a).  TAB: k-space terms from the phase
-// table (sweep_phase_table).
+// of the system described by (sy, tb, a).  TAB: FP64, k-space terms from the phase
+// table (sweep_phase_table); FP32, spline rows in the wide table (sweep_wide).
 template <typename T, int D, int LPW, int KPL, bool PER, bool NU = false, bool TAB = false>
 __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb, const SweepArgs& a, int64_t blk)
 {
@@ -194,11 +220,12 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
 
     extern __shared__ __align__(16) unsigned char smem[];
     Vec4<T>* spl = reinterpret_cast<Vec4<T>*>(smem);                       // NT x (A0..A3) of Re u
-    S* posb = reinterpret_cast<S*>(spl + NT);                                                    // WPB x N x D (particle-major)
+    constexpr bool WIDE = TAB && sizeof(T) == 4, PHASES = TAB && sizeof(T) == 8;
+    S* posb = reinterpret_cast<S*>(spl + NT * (WIDE ? kWide : 1));                                                    // WPB x N x D (particle-major)
     S* pos = posb + (size_t)grp * N * D;
-    const int km = sy.kmax, prow = 2 * km + 1;                             // TAB: rows per axis
+    const int km = sy.kmax, prow = 2 * km + 1;                             // PHASES: rows per axis
     Vec2<T>* ptab = reinterpret_cast<Vec2<T>*>(smem + sweep_base_lds<T>(sy, LPW)) +
-                    (size_t)grp * sweep_phase_len(sy);                     // TAB: [D][prow][2]
+                    (size_t)grp * sweep_phase_len(sy);                     // PHASES: [D][prow][2]
 
     const T u_out = (T)tb.uR[sy.outer_idx];
     // real length per coordinate-difference unit
@@ -216,12 +243,13 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
             spl[Ps + i] = Vec4<T>{(T)(e[0] / unit_len), (T)e[1], (T)(e[2] / unit_len), (T)(e[3] / unit_len)};
         }
     }
-    for (int i = NU ? NT : tid; i < NT; i += kThreads) {
+    for (int e = NU ? NT : tid; e < NT * (WIDE ? kWide : 1); e += kThreads) {
+        const int i = WIDE ? e / kWide : e;
         const T* q = tb.spl + 8 * i;
         if (i < Ps - 1)
-            spl[i] = Vec4<T>{q[0], q[1], q[2], q[3]};
+            spl[e] = Vec4<T>{q[0], q[1], q[2], q[3]};
         else
-            spl[i] = Vec4<T>{u_out, (T)0, (T)0, (T)0};
+            spl[e] = Vec4<T>{u_out, (T)0, (T)0, (T)0};
     }
     // lengths in box units when periodic (scale = 1/L), unscaled otherwise;
     // diff() and raw() return multiples of C::kUnit of that unit
@@ -235,8 +263,19 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
 
     const T hinv = (T)(sy.hinv / scale * C::kUnit), rc = (T)(sy.rc * scale / C::kUnit);
     const T cin = (T)(sy.cinv * unit_len), unitR = (T)unit_len;
-    auto uof = [&](T r) -> T {
-        if constexpr (NU)
+    // WIDE: LDS address of the lane's copy of a row, byte 1 the row (two, for the
+    // old and the new distance)
+    uint32_t row_at[2];
+    row_at[0] = row_at[1] = (uint32_t)(uintptr_t)(LdsBytes)smem + (tid & (kWide - 1)) * sizeof(Vec4<T>);
+    auto uof = [&](T r, int q = 0) -> T {
+        if constexpr (WIDE) {
+            const T x = r * hinv;
+            const T t = Prec<T>::fract_(x);
+            asm("v_cvt_u32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(row_at[q]) : "v"(x));
+            typedef float Row __attribute__((ext_vector_type(4)));   // 16-byte aligned: one LDS read
+            const Row cf = *(const __attribute__((address_space(3))) Row*)(LdsBytes)(uintptr_t)row_at[q];
+            return cf.x + t * (cf.y + t * (cf.z + t * cf.w));
+        } else if constexpr (NU)
             return pair_u_nu<T>(r, cin, sy.ncell - 1, unitR, Ps, spl);
         else
             return pair_u<T, PER>(r, rc, hinv, Ps, spl, u_out);
@@ -249,7 +288,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
     // 2 rho_k: scaling by 2 is exact, and it saves a multiply per k and trial)
     constexpr int KP = KPL > 0 ? KPL : 1;
     T sR[KP], sI[KP], qa[KP];
-    // TAB: the lane's rows in the phase table; otherwise revolutions per raw
+    // PHASES: the lane's rows in the phase table; otherwise revolutions per raw
     // coordinate unit
     T qx[KP], qy[KP], qz[KP];
     int rx[KP], ry[KP], rz[KP];
@@ -265,7 +304,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
         if (k < K) {
             const T* q = tb.kv + 4 * k;
             qa[m] = tb.alpha[2 * k];
-            if constexpr (TAB) {
+            if constexpr (PHASES) {
                 rx[m] = 2 * (km + (int)lattice(q[0]));
                 ry[m] = 2 * (prow + km + (int)lattice(q[1]));
                 if (D > 2) rz[m] = 2 * (2 * prow + km + (int)lattice(q[2]));
@@ -276,14 +315,14 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
             }
         }
     }
-    // TAB: lane gl computes the factors e = gl + j LPW of (position, axis, m =
+    // PHASES: lane gl computes the factors e = gl + j LPW of (position, axis, m =
     // 1 .. kmax): the coordinate's axis, the power, whether the position's
     // displacement is added (as a 0 / 1 weight per axis), the rows of m and -m
-    constexpr int NE = TAB ? 64 / LPW : 1;
+    constexpr int NE = PHASES ? 64 / LPW : 1;
     T ew[NE][3], em[NE];
     int ea[NE], eq[NE], eplus[NE], eminus[NE];
     const int ne = 2 * D * km;
-    if constexpr (TAB) {
+    if constexpr (PHASES) {
 #pragma unroll
         for (int j = 0; j < NE; j++) {
             const int e = gl + j * LPW;
@@ -326,7 +365,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    if constexpr (TAB) {
+    if constexpr (PHASES) {
         // rho_k of the walker, two particles per pass
         for (int n = 0; n < N; n += 2) {
             lds_order();
@@ -431,7 +470,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
                 dz[c] = bcast<LPW>(dl[c], tt);
                 nw[c] = C::add(old[c], dz[c]);
             }
-            if constexpr (TAB) {
+            if constexpr (PHASES) {
                 // phase factors of the old and the new position (read after the
                 // partner loop); a whole box added or taken off leaves them alone
 #pragma unroll
@@ -458,7 +497,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
                     rn2 += dNew * dNew;
                 }
                 const T uo = uof(Prec<T>::sqrt_r2(ro2));
-                const T un = uof(Prec<T>::sqrt_r2(rn2));
+                const T un = uof(Prec<T>::sqrt_r2(rn2), 1);
                 delta += un - uo;
             };
             // rounds in which every lane of the group has a partner run under a
@@ -479,7 +518,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
 #pragma unroll
             for (int m = 0; m < KPL; m++) {
                 T so, co, sn, cn;
-                if constexpr (TAB) {
+                if constexpr (PHASES) {
                     take(m, 0, &co, &so);
                     take(m, 1, &cn, &sn);
                 } else {
@@ -625,12 +664,18 @@ static int default_lanes(const KSys& sy, int64_t W)
 template <typename T, int D, int LPW, int KPL, bool PER>
 static hipError_t launch_sweep_k(const KSys& sy, const KTables<T>& tb, const SweepArgs& a, hipStream_t st)
 {
-    const size_t lds = sweep_lds_bytes<T>(sy, LPW);
+    size_t lds = sweep_lds_bytes<T>(sy, LPW);
     if (sy.nu && (!PER || !tb.nucell)) return hipErrorInvalidValue;
     auto kern = sy.nu ? sweep_kernel<T, D, LPW, KPL, PER, PER, false> : sweep_kernel<T, D, LPW, KPL, PER, false, false>;
     if constexpr (sizeof(T) == 8 && KPL > 0 && D > 1) {
         if (sweep_phase_table<T>(sy, LPW))
             kern = sy.nu ? sweep_kernel<T, D, LPW, KPL, PER, PER, true> : sweep_kernel<T, D, LPW, KPL, PER, false, true>;
+    }
+    if constexpr (sizeof(T) == 4 && PER) {
+        if (sweep_wide<T>(sy, LPW)) {
+            kern = sweep_kernel<T, D, LPW, KPL, PER, false, true>;
+            lds = sweep_wide_lds<T>(sy, LPW);
+        }
     }
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
