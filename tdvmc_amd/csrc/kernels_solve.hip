@@ -9,14 +9,14 @@
 // (phi-dot, computed on the scaled solution before the scaling is undone, as
 // in :1749-1758).  Solver type 1 is the full-pivot QR kernel further down.
 //
-// Blocked right-looking Cholesky in columns of kNB = 16: one wavefront factors
-// the 16 x 16 diagonal block in registers, one thread per row solves the rows
-// below it against that block in LDS (row-major at a padded stride), and the
-// trailing lower triangle is updated in 16 x 16 tiles on FP64 MFMA.  The factor
-// lives in the work buffer, with 1 / L[c][c] on its diagonal so that the
-// solves only multiply.  solve_ahead_body holds two panels and the right-hand
-// sides in LDS and lets steps of neighbouring panels run side by side;
-// solve_body needs one panel only and takes the larger systems.
+// Blocked right-looking Cholesky: one wavefront factors the NB x NB diagonal
+// block in registers, one thread per row solves the rows below it against that
+// block in LDS (row-major at a padded stride), and the trailing lower triangle
+// is updated in 16 x 16 tiles on FP64 MFMA.  The factor lives in the work
+// buffer, with 1 / L[c][c] on its diagonal so that the solves only multiply.
+// solve_ahead_body (NB = 16, the systems up to P = 340) holds two panels and
+// the right-hand sides in LDS and lets steps of neighbouring panels run side by
+// side; solve_body (NB = 32, or 16 for the largest) needs one panel only.
 
 #include <algorithm>
 #include <type_traits>
@@ -30,7 +30,7 @@ namespace tdvmc {
 namespace {
 
 constexpr int kThreads = 1024;
-constexpr int kNB = 16, kLDP = kNB + 1;   // block width, LDS stride of a panel row
+constexpr int kNB = 16, kLDP = kNB + 1;   // solve_ahead_body: block width, LDS stride of a panel row
 
 typedef double double4v __attribute__((ext_vector_type(4)));
 
@@ -68,6 +68,7 @@ __device__ double block_reduce(double v, double* red)
     return s;
 }
 
+template <int NB>
 __device__ __forceinline__ void solve_body(const SolveArgs& a)
 {
     const int P = a.P, tid = threadIdx.x;
@@ -78,10 +79,10 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     double* sc = bI + P;
     double* dorig = sc + P;              // diagonal after scaling and the eps shift
     extern __shared__ __align__(16) unsigned char smem[];
-    double* pan = reinterpret_cast<double*>(smem);   // [rows below][kNB + 1] panel; [kNB][kNB] blocks in the solves
+    double* pan = reinterpret_cast<double*>(smem);   // [rows below][NB + 1] panel; [NB][NB] blocks in the solves
     __shared__ double red[kThreads / 64];
-    __shared__ double ipiv[kNB];          // 1 / L[c][c]
-    __shared__ double ldc[kNB * kNB];      // diagonal block, column-major: ldc[c * kNB + k] = L[k][c]
+    __shared__ double ipiv[NB];          // 1 / L[c][c]
+    __shared__ double ldc[NB * NB];      // diagonal block, column-major: ldc[c * NB + k] = L[k][c]
     __shared__ int nbad;
     const double* mO = a.mean;
     const double eR = a.mean[P], eI = a.mean[P + 1];
@@ -138,39 +139,40 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
 
     // ---------------------------------------------------------------- Cholesky
     // The rows below the diagonal block sit in LDS row-major with a padded
-    // stride (pan[rb * kLDP + c]): a thread's row is read with
+    // stride (pan[rb * LDP + c], LDP = NB + 1): a thread's row is read with
     // immediate offsets, and only threads rb and rb + 32 share a bank.  The
     // diagonal block is staged on its own, column-major and padded with the
-    // identity to kNB x kNB (ldc[c * kNB + l] = A[l][c]): padded columns have
+    // identity to NB x NB (ldc[c * NB + l] = A[l][c]): padded columns have
     // pivot 1 and zero off-diagonal entries and leave the real rows unchanged,
     // so no step below has a run-time bound on the block.  Only the last
     // block can be partial, and it has no rows below it.
-    for (int p0 = 0; p0 < P; p0 += kNB) {
-        const int nb = min(kNB, P - p0);
+    constexpr int LDP = NB + 1;
+    for (int p0 = 0; p0 < P; p0 += NB) {
+        const int nb = min(NB, P - p0);
         const int below = P - p0 - nb;
         if (below > 0) {
             Walk2 wk2(tid, below);
             for (int e = tid; e < nb * below; e += kThreads) {
-                pan[wk2.r * kLDP + wk2.c] = Lm[(size_t)(p0 + wk2.c) * P + p0 + nb + wk2.r];
+                pan[wk2.r * LDP + wk2.c] = Lm[(size_t)(p0 + wk2.c) * P + p0 + nb + wk2.r];
                 wk2.next();
             }
         }
-        for (int e = tid; e < kNB * kNB; e += kThreads) {
-            const int c = e / kNB, l = e % kNB;
+        for (int e = tid; e < NB * NB; e += kThreads) {
+            const int c = e / NB, l = e % NB;
             ldc[e] = (c < nb && l < nb) ? Lm[(size_t)(p0 + c) * P + p0 + l] : (c == l ? 1.0 : 0.0);
         }
         __syncthreads();
         // diagonal block by one wavefront in registers: lane l holds row
-        // l mod kNB, column entries reach the other lanes by v_readlane.  Every
+        // l mod NB, column entries reach the other lanes by v_readlane.  Every
         // lane updates its whole row (the entries above the diagonal are
         // never read), and the diagonal gets 1 / L[c][c] from ipiv at the end.
         if (wv == 0) {
-            const int l = lane & (kNB - 1);
-            double av[kNB];
+            const int l = lane & (NB - 1);
+            double av[NB];
 #pragma unroll
-            for (int k = 0; k < kNB; k++) av[k] = ldc[k * kNB + l];
+            for (int k = 0; k < NB; k++) av[k] = ldc[k * NB + l];
 #pragma unroll
-            for (int c = 0; c < kNB; c++) {
+            for (int c = 0; c < NB; c++) {
                 const double d = readlane_f(av[c], c);
                 double ipj;
                 if (d > 0.0) {
@@ -191,34 +193,34 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
                 av[c] *= ipj;
                 if (lane == 0) ipiv[c] = ipj;
 #pragma unroll
-                for (int k = c + 1; k < kNB; k++) av[k] -= av[c] * readlane_f(av[c], k);
+                for (int k = c + 1; k < NB; k++) av[k] -= av[c] * readlane_f(av[c], k);
                 // one column's lane reads at a time (scalar registers)
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (lane < kNB) {
+            if (lane < NB) {
 #pragma unroll
-                for (int k = 0; k < kNB; k++) ldc[k * kNB + lane] = av[k];
+                for (int k = 0; k < NB; k++) ldc[k * NB + lane] = av[k];
                 // the factor keeps 1 / L[c][c] on its diagonal: the triangular
                 // solves multiply by it (same wavefront, after the writes above
                 // and lane 0's ipiv writes)
-                ldc[lane * kNB + lane] = ipiv[lane];
+                ldc[lane * NB + lane] = ipiv[lane];
             }
         }
         __syncthreads();
         // rows below the block, one thread per row, right-looking within the
         // row: L[r][c] = v_c / L[c][c], then v_k -= L[r][c] L[k][c] for k > c
         for (int rb = tid; rb < below; rb += kThreads) {
-            double* pr = pan + rb * kLDP;
-            double v[kNB];
+            double* pr = pan + rb * LDP;
+            double v[NB];
 #pragma unroll
-            for (int k = 0; k < kNB; k++) v[k] = pr[k];
+            for (int k = 0; k < NB; k++) v[k] = pr[k];
 #pragma unroll
-            for (int c = 0; c < kNB; c++) {
+            for (int c = 0; c < NB; c++) {
                 const double xc = v[c] * ipiv[c];
                 pr[c] = xc;
-                const double* lcol = ldc + c * kNB;   // L[k][c]
+                const double* lcol = ldc + c * NB;   // L[k][c]
 #pragma unroll
-                for (int k = c + 1; k < kNB; k++) v[k] -= xc * lcol[k];
+                for (int k = c + 1; k < NB; k++) v[k] -= xc * lcol[k];
                 // keeps the 32 columns' table reads from being hoisted together (register spills)
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -229,7 +231,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
             for (int e = tid; e < nb * (nb + below); e += kThreads) {
                 const int c = wk3.c, r = wk3.r;
                 if (r >= c)
-                    Lm[(size_t)(p0 + c) * P + p0 + r] = r < nb ? ldc[c * kNB + r] : pan[(r - nb) * kLDP + c];
+                    Lm[(size_t)(p0 + c) * P + p0 + r] = r < nb ? ldc[c * NB + r] : pan[(r - nb) * LDP + c];
                 wk3.next();
             }
         }
@@ -260,11 +262,11 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
                     ok[v] = i < below && k <= i;
                     old[v] = ok[v] ? Lm[(q0 + k) * P + q0 + i] : 0.0;
                 }
-                const double* pa = pan + (16 * tk + pp) * kLDP + kk;   // rows k
-                const double* pb = pan + (16 * ti + pp) * kLDP + kk;   // rows i
+                const double* pa = pan + (16 * tk + pp) * LDP + kk;   // rows k
+                const double* pb = pan + (16 * ti + pp) * LDP + kk;   // rows i
                 double4v acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int s4 = 0; s4 < kNB / 4; s4++)
+                for (int s4 = 0; s4 < NB / 4; s4++)
                     acc = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[4 * s4], pb[4 * s4], acc, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
@@ -277,25 +279,25 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     }
 
     // ---------------------------------------------------------------- L t = b
-    for (int p0 = 0; p0 < P; p0 += kNB) {
-        const int nb = min(kNB, P - p0);
-        // diagonal block into LDS: pan[j * kNB + l] = L[p0 + l][p0 + j]
+    for (int p0 = 0; p0 < P; p0 += NB) {
+        const int nb = min(NB, P - p0);
+        // diagonal block into LDS: pan[j * NB + l] = L[p0 + l][p0 + j]
         for (int e = tid; e < nb * nb; e += kThreads) {
             const int j = e / nb, l = e % nb;
-            pan[j * kNB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
+            pan[j * NB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
         }
         __syncthreads();
         if (wv == 0) {
             // lane l owns row p0 + l; the diagonal holds 1 / L[j][j]
             double tR = lane < nb ? bR[p0 + lane] : 0.0, tI = lane < nb ? bI[p0 + lane] : 0.0;
             for (int j = 0; j < nb; j++) {
-                const double rjj = pan[j * kNB + j];
+                const double rjj = pan[j * NB + j];
                 const double xR = readlane_f(tR, j) * rjj, xI = readlane_f(tI, j) * rjj;
                 if (lane == j) {
                     tR = xR;
                     tI = xI;
                 } else if (lane > j && lane < nb) {
-                    const double l = pan[j * kNB + lane];
+                    const double l = pan[j * NB + lane];
                     tR -= l * xR;
                     tI -= l * xI;
                 }
@@ -321,9 +323,9 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
     }
 
     // ---------------------------------------------------------------- L^T x = t
-    const int npan = (P + kNB - 1) / kNB;
+    const int npan = (P + NB - 1) / NB;
     for (int pb = npan - 1; pb >= 0; pb--) {
-        const int p0 = pb * kNB, nb = min(kNB, P - p0), pe = p0 + nb;
+        const int p0 = pb * NB, nb = min(NB, P - p0), pe = p0 + nb;
         // t_i -= sum_{j >= pe} L[j][i] x_j for the panel's rows (one wave per row group)
         for (int i = p0 + wv; i < pe; i += kThreads / 64) {
             double sR = 0.0, sI = 0.0;
@@ -341,22 +343,22 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
                 bI[i] -= sI;
             }
         }
-        // diagonal block into LDS: pan[j * kNB + l] = L[p0 + l][p0 + j]
+        // diagonal block into LDS: pan[j * NB + l] = L[p0 + l][p0 + j]
         for (int e = tid; e < nb * nb; e += kThreads) {
             const int j = e / nb, l = e % nb;
-            pan[j * kNB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
+            pan[j * NB + l] = Lm[(size_t)(p0 + j) * P + p0 + l];
         }
         __syncthreads();
         if (wv == 0) {
             double tR = lane < nb ? bR[p0 + lane] : 0.0, tI = lane < nb ? bI[p0 + lane] : 0.0;
             for (int j = nb - 1; j >= 0; j--) {
-                const double rjj = pan[j * kNB + j];
+                const double rjj = pan[j * NB + j];
                 const double xR = readlane_f(tR, j) * rjj, xI = readlane_f(tI, j) * rjj;
                 if (lane == j) {
                     tR = xR;
                     tI = xI;
                 } else if (lane < j) {
-                    const double l = pan[lane * kNB + j];   // L[j][lane]
+                    const double l = pan[lane * NB + j];   // L[j][lane]
                     tR -= l * xR;
                     tI -= l * xI;
                 }
@@ -405,8 +407,8 @@ __device__ __forceinline__ void solve_body(const SolveArgs& a)
 //   - in L^T x = t a wavefront has its row's entries of the factor loaded
 //     before the blocks that they meet are solved;
 //   - S is not copied: the first panel's update reads it in place.
-// The operations on each number and their order are solve_body's, so both give
-// the same bits.
+// The operations on each number and their order are those of solve_body with 16
+// columns, so both give the same bits.
 // At P = 32, 13 us against 27 without these; at P = 296, 152 against 373 us, of
 // which the matrix unit's work on one CU is about 35 us and the rest the
 // chains of the 19 diagonal blocks, row solves and back substitutions (about 5
@@ -493,8 +495,6 @@ __device__ __forceinline__ int factor_block(double* d, double rd, int lane)
     return bad;
 }
 
-// RHS_LDS: the right-hand sides in LDS, else in the work buffer.
-template <bool RHS_LDS>
 __device__ __forceinline__ void solve_ahead_body(const SolveArgs& a)
 {
     const int P = a.P, tid = threadIdx.x;
@@ -511,8 +511,7 @@ __device__ __forceinline__ void solve_ahead_body(const SolveArgs& a)
     extern __shared__ __align__(16) unsigned char smem[];
     const int cap = ahead_rows(P);
     double* pan0 = reinterpret_cast<double*>(smem);   // [cap][kLDP], [cap - 16][kLDP]
-    // [2][LD] right-hand sides, then t, then x
-    double* bl = RHS_LDS ? pan0 + (size_t)(2 * cap - kNB) * kLDP : rdiag + LD;
+    double* bl = pan0 + (size_t)(2 * cap - kNB) * kLDP;   // [2][LD] right-hand sides, then t, then x
     __shared__ double ldc[2][kNB * kNB];              // diagonal blocks, column-major
     __shared__ double red[NW];
     __shared__ int nbad;
@@ -721,7 +720,7 @@ __device__ __forceinline__ void solve_ahead_body(const SolveArgs& a)
         const int c = e / kNB, j = e % kNB;
         diag[c * kLDP + j] = Lm[(size_t)c * LD + c / kNB * kNB + j];
     }
-    constexpr int NQ = 10;   // 64 entries each: up to P = 656
+    constexpr int NQ = 6;   // 64 entries each: up to P = 400
     double lr[NQ];
     auto load_row = [&](int p0) {
         const double* row = Lm + (size_t)(p0 + wv) * LD + p0 + kNB;
@@ -1053,46 +1052,46 @@ __device__ __forceinline__ void solve_qr_body(const SolveArgs& a)
     }
 }
 
-__global__ __launch_bounds__(kThreads) void solve_kernel(SolveArgs a) { solve_body(a); }
-template <bool RHS_LDS>
-__global__ __launch_bounds__(kThreads) void solve_ahead_kernel(SolveArgs a) { solve_ahead_body<RHS_LDS>(a); }
+template <int NB>
+__global__ __launch_bounds__(kThreads) void solve_kernel(SolveArgs a)
+{
+    solve_body<NB>(a);
+}
+__global__ __launch_bounds__(kThreads) void solve_ahead_kernel(SolveArgs a) { solve_ahead_body(a); }
 __global__ __launch_bounds__(kThreads) void solve_qr_kernel(SolveArgs a)
 {
     solve_qr_body(a);
 }
-// one workgroup per system of a batch
-template <int FORM>
+// one workgroup per system of a batch; NB = 0: solve_ahead_body
+template <int NB>
 __global__ __launch_bounds__(kThreads) void solve_batch_kernel(const SolveArgs* __restrict__ args)
 {
     const SolveArgs a = args[blockIdx.x];
     if (a.mean_sub)
         solve_qr_body(a);
-    else if constexpr (FORM > 0)
-        solve_ahead_body<FORM == 2>(a);
+    else if constexpr (NB == 0)
+        solve_ahead_body(a);
     else
-        solve_body(a);
+        solve_body<NB>(a);
 }
 
-// dynamic LDS of solve_body: the rows below a block at stride kLDP (also holds
-// the blocks of the triangular solves)
-size_t solve_lds_bytes(int P) { return (size_t)kLDP * std::max(P, kNB) * sizeof(double); }
-constexpr size_t kMaxPanelLds = 150 * 1024;   // beside the static LDS (blocks, reductions)
-// and of solve_ahead_body: both panel buffers and (rhs) the right-hand sides
-size_t solve_ahead_lds_bytes(int P, bool rhs)
+constexpr size_t kMaxPanelLds = 150 * 1024;   // beside the static LDS (NB x NB block, reductions)
+// Block width of the Cholesky; 0: solve_ahead_body, for the systems up to P =
+// 340 (at P = 296 the whole call with its copies takes 229 us, with solve_body
+// 447).  Above, 32 columns (fewer panels and barriers: at P = 420, 705 against
+// 738 us with 16), and 16 again where the panel of 32 no longer fits in LDS.
+// solve_ahead_body would be the faster one up to P = 608 (P = 560: 743 against
+// 1315 us) but with 16 columns its sums are grouped otherwise than with 32: a
+// nearly singular S of a few hundred parameters turns such a last-bit change
+// into 1e-9 of the stepped parameters, so those sizes keep their 32 columns.
+constexpr int kAheadMaxP = 340;
+size_t solve_lds_bytes(int NB, int P)
 {
-    const size_t LD = ((size_t)P + kNB - 1) / kNB * kNB;
-    return ((size_t)(2 * ahead_rows(P) - kNB) * kLDP + (rhs ? 2 * LD : 0)) * sizeof(double);
+    if (NB == 0) return ((size_t)(2 * ahead_rows(P) - kNB) * kLDP + 2 * (size_t)((P + kNB - 1) / kNB * kNB)) * sizeof(double);
+    // the rows below a block at stride NB + 1 (also holds the blocks of the triangular solves)
+    return (size_t)(NB + 1) * std::max(P, NB) * sizeof(double);
 }
-// Form of the Cholesky: 2 (solve_ahead_body, right-hand sides in LDS) where the
-// buffers fit the 160 KB beside 4.5 KB of static LDS, P <= 560; 1 (right-hand
-// sides in the work buffer) where the panels alone do, P <= 608; 0 (solve_body)
-// above.  Whole call with its copies, solve_body against forms 2 and 1: 447 and
-// 229 us at P = 296, 1315 and 743 us at P = 560, 1640 and 938 us at P = 577.
-constexpr size_t kMaxAheadLds = 160 * 1024 - 4608;
-int solve_form(int P)
-{
-    return solve_ahead_lds_bytes(P, true) <= kMaxAheadLds ? 2 : solve_ahead_lds_bytes(P, false) <= kMaxAheadLds ? 1 : 0;
-}
+int solve_width(int P) { return P <= kAheadMaxP ? 0 : solve_lds_bytes(32, P) <= kMaxPanelLds ? 32 : 16; }
 
 template <typename K, typename A>
 hipError_t launch_cholesky(K kern, int n, size_t lds, const A& args, hipStream_t st)
@@ -1111,11 +1110,11 @@ hipError_t launch_solve_batch(const SolveArgs* args_dev, int n, int P_max, hipSt
 {
     if (n <= 0) return hipSuccess;
     const size_t qr = 2 * (size_t)P_max * sizeof(int);   // the QR's transpositions
-    const int form = solve_form(P_max);
-    const size_t lds = std::max(qr, form ? solve_ahead_lds_bytes(P_max, form == 2) : solve_lds_bytes(P_max));
-    if (form == 2) return launch_cholesky(solve_batch_kernel<2>, n, lds, args_dev, st);
-    if (form == 1) return launch_cholesky(solve_batch_kernel<1>, n, lds, args_dev, st);
-    if (lds <= kMaxPanelLds) return launch_cholesky(solve_batch_kernel<0>, n, lds, args_dev, st);
+    const int nb = solve_width(P_max);
+    const size_t lds = std::max(qr, solve_lds_bytes(nb, P_max));
+    if (nb == 0) return launch_cholesky(solve_batch_kernel<0>, n, lds, args_dev, st);
+    if (nb == 32) return launch_cholesky(solve_batch_kernel<32>, n, lds, args_dev, st);
+    if (lds <= kMaxPanelLds) return launch_cholesky(solve_batch_kernel<16>, n, lds, args_dev, st);
     return hipErrorInvalidValue;
 }
 
@@ -1132,11 +1131,11 @@ hipError_t launch_solve(const SolveArgs& a, hipStream_t st)
         hipLaunchKernelGGL(solve_qr_kernel, dim3(1), dim3(kThreads), 2 * (size_t)a.P * sizeof(int), st, a);
         return hipGetLastError();
     }
-    const int form = solve_form(a.P);
-    const size_t lds = form ? solve_ahead_lds_bytes(a.P, form == 2) : solve_lds_bytes(a.P);
-    if (form == 2) return launch_cholesky(solve_ahead_kernel<true>, 1, lds, a, st);
-    if (form == 1) return launch_cholesky(solve_ahead_kernel<false>, 1, lds, a, st);
-    if (lds <= kMaxPanelLds) return launch_cholesky(solve_kernel, 1, lds, a, st);
+    const int nb = solve_width(a.P);
+    const size_t lds = solve_lds_bytes(nb, a.P);
+    if (nb == 0) return launch_cholesky(solve_ahead_kernel, 1, lds, a, st);
+    if (nb == 32) return launch_cholesky(solve_kernel<32>, 1, lds, a, st);
+    if (lds <= kMaxPanelLds) return launch_cholesky(solve_kernel<16>, 1, lds, a, st);
     return hipErrorInvalidValue;
 }
 

@@ -1,6 +1,7 @@
 """The Cholesky solve at the sizes where its kernels change over or a block is
 partial: one block, a block and a row, the smallest panel buffers, the last
-sizes whose right-hand sides (P = 560) and whose panels (P = 608) fit the LDS.
+size of the kernel that factors ahead (P = 340) and of the 32-column blocks
+(P = 581), and both sides of them.
 Against the oracle's restatement, with the tolerance of the solver's other
 tests; a repeated call gives the same bits (no race between the steps that run
 side by side)."""
@@ -44,7 +45,7 @@ def _check(m, bad, pre):
 
 
 @pytest.mark.parametrize("pre", [0, 1])
-@pytest.mark.parametrize("P", [1, 2, 15, 16, 17, 31, 32, 47, 48, 49, 64, 65, 561, 576, 577, 608, 609])
+@pytest.mark.parametrize("P", [1, 2, 15, 16, 17, 31, 32, 47, 48, 49, 64, 65, 336, 337, 340, 341, 561, 576, 577, 581, 582, 609])
 def test_solve_edges(P, pre):
     print("solve", P, pre, flush=True)
     _check(_moments(P), 0, pre)
@@ -52,7 +53,7 @@ def test_solve_edges(P, pre):
 
 # non-positive pivots in the first block, on both sides of a block's edge, in a
 # block factored ahead and in a partial last one
-@pytest.mark.parametrize("P,bad", [(16, (0,)), (33, (15, 16, 32)), (50, (3, 31, 49)), (577, (0, 300, 576))])
+@pytest.mark.parametrize("P,bad", [(16, (0,)), (33, (15, 16, 32)), (50, (3, 31, 49)), (340, (0, 177, 339)), (577, (0, 300, 576))])
 def test_solve_pivots(P, bad):
     print("solve", P, bad, flush=True)
     _check(_moments(P, bad), len(bad), 0)
