@@ -107,6 +107,16 @@ def build_cpp_check(verbose: bool = True) -> str:
         raise RuntimeError(f"SplinedFunction check build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     if verbose:
         print("built", sc)
+    # the launch rules, which the kernels' sources share with the host
+    for name in ("sweep_rules_check",):
+        rc = os.path.join(os.path.dirname(CPP_CHECK_BIN), name)
+        cmd = [HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1",
+               os.path.join(ROOT, "tests", "cpp", name + ".cpp"), "-o", rc]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"launch rules check build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+        if verbose:
+            print("built", rc)
     return CPP_CHECK_BIN
 
 
