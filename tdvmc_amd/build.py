@@ -108,7 +108,7 @@ def build_cpp_check(verbose: bool = True) -> str:
     if verbose:
         print("built", sc)
     # the launch rules, which the kernels' sources share with the host
-    for name in ("sweep_rules_check",):
+    for name in ("sweep_rules_check", "eval_rules_check"):
         rc = os.path.join(os.path.dirname(CPP_CHECK_BIN), name)
         cmd = [HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1",
                os.path.join(ROOT, "tests", "cpp", name + ".cpp"), "-o", rc]

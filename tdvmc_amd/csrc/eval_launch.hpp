@@ -25,21 +25,30 @@ static hipError_t launch_eval_w(const KSys& sy, const KTables<T>& tb, const doub
 // Wavefronts per walker.  Four share the set-up, the histogram's clearing and
 // reduction and the assembly of one walker, which is most of a small walker's
 // time; with one or two, four or two walkers do theirs side by side (one
-// pair tile leaves four wavefronts N / 8 steps each).  FP64, us with 1 / 2 / 4:
-//   N = 8 (3-D, 16384 walkers) 55 / 85 / 141; N = 25 (2-D, 16 terms, 4099) 67 / 66 / 136;
-//   N = 33 (8192) 67 / 74 / 99; N = 64 (16384) 154 / 147 / 181; N = 96 (8192) 196 / 154 / 160;
-//   N = 128 (8192) 267 / 191 / 180; with per-particle output N = 33 74 / 81 / 92, N = 64 193 / 180 / 174.
-// Few walkers need more wavefronts each to reach every SIMD: N = 20, 1024
-// walkers 18.7 / 16.4 / 16.6; N = 64 24 / 23 / 21 with 1024, 32 / 30 / 34 with
-// 2048.  The mixed form keeps four: its FP32 sums are added up per wavefront.
+// pair tile leaves four wavefronts N / 8 steps each).  Fewer are taken where that
+// leaves the chip full:
+//   - two wavefronts for every one of the 1024 SIMDs: N = 20, 1024 walkers 18.7 /
+//     16.4 / 16.6 us with 1 / 2 / 4; N = 19, 101 terms, 588 walkers 48 / 32 / 25;
+//   - the LDS of three workgroups (one each) or four (two each) in a CU: N = 27
+//     (2-D), 48 knots, 64 terms, 2610 walkers 61 / 48 / 56 (two, four and four
+//     workgroups); N = 15 (2-D), 48 knots, 258 terms, 3164 walkers 267 / 157 / 127;
+//   - at most 64 and 200 k-space terms, which a walker's wavefronts go through one
+//     after the other: N = 14, 206 terms, 48 knots, 1328 walkers 158 / 70 / 63; N = 27,
+//     101 terms, 2291 walkers 77 / 67 / 61, N = 16, 101 terms, 11568 walkers 173 /
+//     173 / 208, N = 20, 206 terms, 2063 walkers 176 / 106 / 87.
+// Where all hold: N = 8 (16384 walkers) 55 / 85 / 141; N = 25 (2-D, 16 terms, 4099)
+// 67 / 66 / 136; N = 38 (2-D, 64 terms, 7876) 107 / 114 / 137; N = 64 (16384) 154 / 147 /
+// 181; N = 96 (8192) 196 / 154 / 160; N = 128 (8192) 267 / 191 / 180; with per-particle
+// output N = 33 (8192) 74 / 81 / 92, N = 64 193 / 180 / 174.  The mixed form keeps
+// four: its FP32 sums are added up per wavefront.
 template <typename T>
 static int eval_waves(const KSys& sy, bool pp, int64_t W)
 {
     if (sizeof(T) == 4 || sy.N > (pp ? 48 : 100)) return 4;
-    int wpw = sy.N <= 48 ? 1 : 2;
-    const int64_t least = sy.N <= 48 ? 1025 : 4096;   // wavefronts
-    while (wpw < 4 && (W * wpw < least || (4 / wpw) * eval_lds_bytes<T>(sy, pp, wpw) > 160 * 1024)) wpw *= 2;
-    return wpw;
+    auto workgroups = [&](int wpw) { return 160 * 1024 / ((4 / wpw) * eval_lds_bytes<T>(sy, pp, wpw)); };
+    if (sy.N <= 48 && W >= 2048 && sy.Kh <= 64 && workgroups(1) >= 3) return 1;
+    if (W >= 1024 && sy.Kh <= 200 && workgroups(2) >= 4) return 2;
+    return 4;
 }
 
 template <typename T, int D, bool PP, bool PER, typename TO>
