@@ -629,9 +629,18 @@ __device__ __forceinline__ void eval_kgrad(const KSys& sy, const KTables<T>& tb,
 // last axis.  16384 walkers, whole measurement: N = 343, 128 terms (rho_k
 // handed over) 3.23 -> 2.97 ms; 2-D, N = 400, 258 terms 6.86 -> 5.73 ms.
 // Below kRunTerms terms per wavefront the D sincos of the particle and the
-// chain of a run's dependent products cost more than they save: the direct
-// form runs there (N = 25, 16 terms, 4 a wavefront: 61 against 65 us).
-constexpr int kRunTerms = 8;
+// chain of a run's dependent products cost more than they save, and the start
+// of a run costs up to D products: the direct form runs there, and for at most 32
+// particles (which it spreads over both half-waves) where a run holds fewer than
+// kRunLength terms on average, as in 3-D.  Direct and run form, us: N = 25 (2-D),
+// 16 terms, 4 a wavefront 61 / 65; N = 14 (3-D), 206 terms in 68 runs, 1328
+// walkers, two wavefronts 74 / 70, four 63 / 66; N = 5 (3-D), 101 terms in 41 runs,
+// 481 walkers 20.5 / 22.1.
+constexpr int kRunTerms = 12, kRunLength = 4;
+__host__ __device__ inline bool eval_use_runs(const KSys& sy, int wpw)
+{
+    return sy.Kh >= kRunTerms * wpw && (sy.N > 32 || sy.Kh >= kRunLength * sy.nrun);
+}
 struct Cplx {
     double x, y;
 };
@@ -777,7 +786,30 @@ __device__ __forceinline__ void eval_kgrad_runs(const KSys& sy, const KTables<do
 // thread multiplies D of them per particle for its term; the particles are
 // split over G threads per term where there are more threads than terms.
 // scratch: `bytes` of LDS that nothing else holds yet.  Returns false, with
-// nothing done, where the table does not fit.
+// nothing done, where the table is not taken (rho_table_particles).
+//
+// Particles per pass for nt threads (0: a thread computes its terms' sincos).
+// Small walkers keep the direct sums, whose few sincos cost less than the
+// table's barriers: N = 16 (2-D), 16 terms, 276 walkers 18.3 us, with the table
+// 25.7; N = 32 (3-D), 9 terms, 7196 walkers 143 and 265 (four wavefronts), 110 and
+// 114 (two).  So do walkers whose LDS holds less than an eighth of their
+// particles (or of 64): N = 86 (2-D), 8 knots, 64 terms, 525 walkers 45 and 81.
+struct RhoTable {
+    int particles, G;
+};
+__host__ __device__ inline RhoTable rho_table_particles(const KSys& sy, size_t bytes, int nt)
+{
+    const int K = sy.Kh, terms = nt == 256 ? 2 : (nt == 128 ? 3 : 5);   // terms per thread
+    if (sy.D < 2 || sy.N < 48 || K < 8 || K > terms * nt) return RhoTable{0, 0};
+    const size_t cx = 2 * sizeof(double), row = cx * sy.D * (2 * sy.kmax + 1);
+    int G = nt > K ? nt / K : 1;
+    while (G > 1 && cx * G * K + row > bytes) G--;
+    const size_t parts = G > 1 ? cx * G * K : 0;
+    if (parts + row > bytes) return RhoTable{0, 0};
+    const size_t fit = (bytes - parts) / row;
+    const int nb = fit < 64 ? (int)fit : 64;
+    return 8 * nb < (sy.N < 64 ? sy.N : 64) ? RhoTable{0, 0} : RhoTable{nb, G};
+}
 template <int D, int NT>
 __device__ __forceinline__ bool eval_rho_table(const KSys& sy, const KTables<double>& tb, const double* pos,
                                                double* rho, double* scratch, size_t bytes, int tid,
@@ -785,14 +817,11 @@ __device__ __forceinline__ bool eval_rho_table(const KSys& sy, const KTables<dou
 {
     const int N = sy.N, K = sy.Kh, km = sy.kmax, prow = 2 * km + 1;
     constexpr int KR = NT == 256 ? 2 : (NT == 128 ? 3 : 5);   // terms per thread
-    int G = max(1, NT / K);
-    const size_t row = sizeof(Cplx) * D * prow;
-    while (G > 1 && sizeof(Cplx) * G * K + row > bytes) G--;
-    const size_t parts = G > 1 ? sizeof(Cplx) * G * K : 0;
-    if (parts + row > bytes || K > KR * NT) return false;
-    const int nb = (int)min((size_t)64, (bytes - parts) / row);   // particles per pass
+    const RhoTable rt = rho_table_particles(sy, bytes, NT);
+    if (rt.particles == 0) return false;
+    const int G = rt.G, nb = rt.particles;
     Cplx* part = reinterpret_cast<Cplx*>(scratch);
-    Cplx* tab = part + parts / sizeof(Cplx);
+    Cplx* tab = part + (G > 1 ? G * K : 0);
     int q[KR][D];
     Cplx acc[KR];
     const int g = G > 1 ? tid / K : 0;
@@ -984,7 +1013,7 @@ __device__ __forceinline__ void eval_body(const KSys& sy, const KTables<T>& tb, 
     // ------------------------------------------------------------ rho_k
     // phase in revolutions = kq . raw coordinate, |phase| <= sum_a |n_a| / 2
     double ex_k = 0.0;
-    const bool use_runs = sizeof(T) == 8 && K >= kRunTerms * WPW;   // rho in run order, for eval_kgrad_runs
+    const bool use_runs = sizeof(T) == 8 && eval_use_runs(sy, WPW);   // rho in run order, for eval_kgrad_runs
     bool ready = false;                                              // rho holds every term
     if constexpr (sizeof(T) == 8 && D > 1 && PER) {
         if (K > 0 && !rho_in) {

@@ -43,7 +43,7 @@ def test_one_and_two_wavefronts_per_walker(waves, D, N, K, P_s, W, real):
         Kh = ctx.info.K_terms
         ctx.set_params(uR, uI)
         for per_particle in (False, True):
-            used = subprocess.run([CHECK], input="%d %d %d %d %d %d" % (D, N, P_s, Kh, W, per_particle), capture_output=True, text=True,
+            used = subprocess.run([CHECK], input="%d %d %d %d %d %d 1 1" % (D, N, P_s, Kh, W, per_particle), capture_output=True, text=True,
                                   check=True).stdout.split()[0]
             if per_particle and N > 48:
                 assert used == "4"
