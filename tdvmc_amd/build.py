@@ -107,6 +107,15 @@ def build_cpp_check(verbose: bool = True) -> str:
         raise RuntimeError(f"SplinedFunction check build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     if verbose:
         print("built", sc)
+    # HIP calls a test looks at or refuses (loaded before libtdvmc.so)
+    sh = os.path.join(os.path.dirname(CPP_CHECK_BIN), "libhip_shim.so")
+    cmd = ["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", os.path.join(ROOT, "tests", "cpp", "hip_shim.cpp"), "-Wl,--no-as-needed",
+           "-L" + os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib"), "-lamdhip64", "-ldl", "-o", sh]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"HIP shim build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    if verbose:
+        print("built", sh)
     # the launch rules, which the kernels' sources share with the host
     for name in ("sweep_rules_check", "eval_rules_check"):
         rc = os.path.join(os.path.dirname(CPP_CHECK_BIN), name)

@@ -268,9 +268,15 @@ public:
             if (ctx->ws_pin) (void)hipHostFree(ctx->ws_pin);
             ctx->ws_pin = nullptr;
             ctx->ws_pin_cap = 0;
-            e = hipHostMalloc(reinterpret_cast<void**>(&ctx->ws_pin), total * sizeof(double), hipHostMallocDefault);
-            if (e != hipSuccess) return e;
-            ctx->ws_pin_cap = total;
+            if (hipHostMalloc(reinterpret_cast<void**>(&ctx->ws_pin), total * sizeof(double), hipHostMallocDefault) ==
+                hipSuccess) {
+                ctx->ws_pin_cap = total;
+            } else {
+                // no pinned memory to be had: the arrays travel from and to the caller's
+                ctx->ws_pin = nullptr;
+                pinned = false;
+                (void)hipGetLastError();
+            }
         }
         return hipSuccess;
     }
