@@ -1604,7 +1604,7 @@ struct tdvmc_batch {
     double* dK[4] = {nullptr, nullptr, nullptr, nullptr};
     uint32_t* dEpoch = nullptr;
     int64_t sweep_blocks = 0, eval_blocks = 0;
-    size_t sweep_lds = 0, eval_lds_f = 0, eval_lds_d = 0;
+    size_t sweep_lds_f = 0, sweep_lds_d = 0, eval_lds_f = 0, eval_lds_d = 0;
     hipGraphExec_t graph = nullptr;
     hipGraph_t graph_src = nullptr;
     std::string graph_key;
@@ -1700,7 +1700,7 @@ int batch_upload(tdvmc_batch* b, int64_t n_moves, uint64_t seed, bool want_rho)
     std::vector<MomentsItem> mi(n);
     std::vector<SolveArgs> sv[4];
     int64_t sb = 0, eb = 0, part_len = 0;
-    size_t slds = 0, elf = 0, eld = 0;
+    size_t slf = 0, sld = 0, elf = 0, eld = 0;
     for (int s = 0; s < n; s++) {
         tdvmc_ctx* c = b->sys[s];
         sy[s] = c->sy;
@@ -1719,7 +1719,8 @@ int batch_upload(tdvmc_batch* b, int64_t n_moves, uint64_t seed, bool want_rho)
         const size_t slot_d = eval_lds_bytes<double>(c->sy, false, wpw);
         estart[s] = eb;
         eb += (c->W + 4 / wpw - 1) / (4 / wpw);
-        slds = std::max(slds, std::max(sweep_lds_bytes<float>(c->sy, lanes), sweep_lds_bytes<double>(c->sy, lanes)));
+        slf = std::max(slf, sweep_lds_bytes<float>(c->sy, lanes));
+        sld = std::max(sld, sweep_lds_bytes<double>(c->sy, lanes));
         elf = std::max(elf, (size_t)(4 / wpw) * slot_f);
         eld = std::max(eld, (size_t)(4 / wpw) * slot_d);
         SweepArgs& a = sa[s];
@@ -1774,7 +1775,8 @@ int batch_upload(tdvmc_batch* b, int64_t n_moves, uint64_t seed, bool want_rho)
     }
     b->sweep_blocks = sb;
     b->eval_blocks = eb;
-    b->sweep_lds = slds;
+    b->sweep_lds_f = slf;
+    b->sweep_lds_d = sld;
     b->eval_lds_f = elf;
     b->eval_lds_d = eld;
     int rc;
@@ -1799,11 +1801,11 @@ int batch_sweep_launch(tdvmc_batch* b, int prec)
     const int lanes = batch_lanes(b);
     if (prec == TDVMC_MIXED) {
         SweepBatch<float> bt{n, b->dSweepStart, b->dSys, b->dTabF, b->dSweepArgs};
-        BHIPC(launch_sweep_batch<float>(bt, b->D, b->periodic, lanes, b->kh_max, b->sweep_blocks, b->sweep_lds,
+        BHIPC(launch_sweep_batch<float>(bt, b->D, b->periodic, lanes, b->kh_max, b->sweep_blocks, b->sweep_lds_f,
                                         b->stream));
     } else {
         SweepBatch<double> bt{n, b->dSweepStart, b->dSys, b->dTabD, b->dSweepArgs};
-        BHIPC(launch_sweep_batch<double>(bt, b->D, b->periodic, lanes, b->kh_max, b->sweep_blocks, b->sweep_lds,
+        BHIPC(launch_sweep_batch<double>(bt, b->D, b->periodic, lanes, b->kh_max, b->sweep_blocks, b->sweep_lds_d,
                                          b->stream));
     }
     BHIPC(launch_add_u32(b->dEpoch, 1u, b->stream));

@@ -3,10 +3,15 @@
 #include <dlfcn.h>
 #include <stddef.h>
 
+struct ShimDim3 {
+    unsigned x, y, z;
+};
+
 extern "C" {
 
 int shim_refuse_pinned = 0;    // hipHostMalloc returns hipErrorOutOfMemory
 int shim_refused = 0;          // how often it did
+size_t shim_most_lds = 0;      // largest dynamic LDS of the launches since it was cleared
 
 int hipHostMalloc(void** ptr, size_t size, unsigned flags)
 {
@@ -18,6 +23,15 @@ int hipHostMalloc(void** ptr, size_t size, unsigned flags)
     using F = int (*)(void**, size_t, unsigned);
     static const F next = reinterpret_cast<F>(dlsym(RTLD_NEXT, "hipHostMalloc"));
     return next(ptr, size, flags);
+}
+
+// what every kernel<<<>>> launch passes its shape through
+unsigned __hipPushCallConfiguration(ShimDim3 grid, ShimDim3 block, size_t lds, void* stream)
+{
+    if (lds > shim_most_lds) shim_most_lds = lds;
+    using F = unsigned (*)(ShimDim3, ShimDim3, size_t, void*);
+    static const F next = reinterpret_cast<F>(dlsym(RTLD_NEXT, "__hipPushCallConfiguration"));
+    return next(grid, block, lds, stream);
 }
 
 }
