@@ -1250,9 +1250,11 @@ __device__ __forceinline__ void eval_body(const KSys& sy, const KTables<T>& tb, 
 }
 
 // WPW wavefronts per walker, 4 / WPW walkers per workgroup (slot_bytes of LDS
-// each)
+// each).  The mixed form without per-particle output is held to the registers of
+// five wavefronts per SIMD: in 3-D the compiler's choice was one more than that
+// (129 terms, N = 72, 1194 walkers 34 -> 40 us with four).
 template <typename T, int D, bool PP, bool PER, typename TO, int WPW>
-__global__ __launch_bounds__(kThreads, 4) void eval_kernel(KSys sy, KTables<T> tb, const double* __restrict__ Rg,
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 && !PP ? 5 : 4) void eval_kernel(KSys sy, KTables<T> tb, const double* __restrict__ Rg,
                                                          int64_t W, EvalOut<TO> out, const T* __restrict__ rho_in,
                                                          size_t slot_bytes)
 {
