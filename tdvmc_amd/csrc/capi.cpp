@@ -984,16 +984,18 @@ constexpr int kObsShells = 50;
 constexpr int kObsMaxBins = 8192;
 
 // Segments per row of g(r)'s pair loop: enough work items for the workgroup's
-// 256 threads twice, and the count whose last round of items and last partner
-// of a segment are fullest (N = 343: 8 segments keep 95 % of the lanes busy, the
-// 2 that 512 items need 89 %).
-int gr_segments(int N)
+// 256 threads twice, and (fullest) the count whose last round of items and last
+// partner of a segment are fullest (N = 343: 8 segments keep 95 % of the lanes
+// busy, the 2 that 512 items need 89 %).  Not in the mixed form in 3-D, whose reads
+// of the partners decide (N = 142: 4 segments 161 us, 9 173; N = 214: 3 and 7, 137 and
+// 145).
+int gr_segments(int N, bool fullest)
 {
     const int M = N / 2;   // partners of a row
     const int least = std::max(1, std::min(M, (512 + N - 1) / N));
     int best = least;
     double eff = 0.0;
-    for (int s = least; s <= std::min(M, least + 10); s++) {
+    for (int s = least; fullest && s <= std::min(M, least + 10); s++) {
         const double items = (double)N * s;
         const double e = items / (256.0 * std::ceil(items / 256.0)) * M / (s * std::ceil((double)M / s));
         if (e > eff + 0.01) {
@@ -1138,8 +1140,9 @@ int enqueue_obs(tdvmc_ctx* ctx, int prec, const double* dR, int64_t W, double* g
     // FP64 in 2-D and 3-D: the matrix-product form where its LDS fits (and the
     // squared distances fit an FP32 guess)
     const size_t mfma = f32 || o.gmax < 1e-12 || o.gmax > 1e12 ? 0 : obs_mfma_lds_bytes(N, D, chunk, o.nmax, o.count, o.npair);
-    const bool use_mfma = mfma > 0 && mfma <= 65536;
-    const size_t lds = use_mfma ? mfma : obs_lds_bytes(N, D, o.V, chunk, o.nmax, o.count, f32);
+    const size_t direct = obs_lds_bytes(N, D, o.V, chunk, o.nmax, o.count, f32);
+    const bool use_mfma = mfma > 0 && mfma <= 65536 && (direct > 65536 || obs_mfma_pays(N, o.count, W, gr_w != nullptr));
+    const size_t lds = use_mfma ? mfma : direct;
     if (lds > 65536) {
         ctx->err = "g(r) / S(k) need " + std::to_string(lds) + " bytes of LDS per walker (at most 65536)";
         return TDVMC_ERR_BAD_ARG;
@@ -1165,7 +1168,7 @@ int enqueue_obs(tdvmc_ctx* ctx, int prec, const double* dR, int64_t W, double* g
     a.nshell = o.nshell;
     a.nmax = o.nmax;
     a.chunk = chunk;
-    a.gr_segs = gr_segments(N);
+    a.gr_segs = gr_segments(N, !f32 || D < 3);
     a.sk_w = sk_w;
     hipEvent_t ev{};
     int rc = prof_begin(ctx, "observables", &ev);

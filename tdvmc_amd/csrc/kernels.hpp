@@ -244,6 +244,8 @@ size_t obs_lds_bytes(int N, int D, int V, int chunk, int nmax, int count, bool f
 // FP64 in 2-D and 3-D: S(k) as a matrix product, bins from thresholds; its LDS,
 // or 0 where it does not take the shape
 size_t obs_mfma_lds_bytes(int N, int D, int chunk, int nmax, int count, int npair);
+// whether it is the faster form (per_walker: each walker's g(r) is asked for)
+bool obs_mfma_pays(int N, int count, int64_t W, bool per_walker);
 hipError_t launch_obs_mfma(const ObsArgs& a, int D, size_t lds, hipStream_t st);
 template <typename T>
 hipError_t launch_obs(const ObsArgs& a, int D, size_t lds, hipStream_t st);

@@ -27,6 +27,7 @@
 // box fractions (exact minimum image), FP32 powers each from its own reduced
 // phase, FP32 sums per chunk added in FP64.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -82,10 +83,20 @@ __device__ __forceinline__ void add_counts(const ObsArgs& a, const unsigned* cnt
     }
 }
 
+// the workgroup's pair counts [count], behind the walker's LDS
 template <typename T, int D>
-__global__ __launch_bounds__(kObsThreads) void obs_kernel(ObsArgs a)
+__device__ __forceinline__ unsigned* obs_counts(const ObsArgs& a, unsigned char* smem)
 {
-    extern __shared__ __align__(16) unsigned char smem[];
+    const int R = a.V >> 8, Vr = a.V & 255, G = Vr ? kObsThreads / Vr : 1;
+    return reinterpret_cast<unsigned*>(smem + ((size_t)4 * a.N + 2 * (size_t)(256 * R + Vr * G)) * sizeof(double) +
+                                       (sizeof(T) == 4 ? (size_t)a.N * sizeof(uint4) : 0) +
+                                       (size_t)D * (a.nmax + 1) * (a.chunk + 1) * sizeof(Cx<T>));
+}
+
+// One walker w.  SHARED: the workgroup goes through several (obs_grid)
+template <typename T, int D, bool SHARED>
+__device__ __forceinline__ void obs_walker(const ObsArgs& a, int64_t w, unsigned char* smem)
+{
     const int tid = threadIdx.x;
     const int N = a.N;
     const int nm = a.nmax + 1;
@@ -98,224 +109,245 @@ __global__ __launch_bounds__(kObsThreads) void obs_kernel(ObsArgs a)
     double* part = reinterpret_cast<double*>(fix + (sizeof(T) == 4 ? N : 0));   // [256 R + Vr G][2] totals
     // phase tables [D][nm][chunk + 1]: the particle index runs fastest, and the
     // padded row keeps the rows of different powers in different banks
-    const int CS = a.chunk + 1;
+    int CS = a.chunk + 1;
     Cx<T>* tab = reinterpret_cast<Cx<T>*>(part + 2 * (size_t)(256 * R + Vr * G));
     unsigned* cnt = reinterpret_cast<unsigned*>(tab + (size_t)D * nm * CS);   // [count]
-
-    for (int b = tid; b < a.count; b += kObsThreads) cnt[b] = 0u;
-    for (int64_t w = blockIdx.x; w < a.W; w += gridDim.x) {
-        const double* Rw = a.R + w * (int64_t)N * D;
-        for (int e = tid; e < N * 4; e += kObsThreads) {
-            const int i = e >> 2, c = e & 3;
-            pos[e] = c < D ? Rw[i * D + c] : 0.0;
-        }
-        if constexpr (sizeof(T) == 4) {
-            // 32-bit fractions of the box: the wrapping difference is the minimum image
-            for (int i = tid; i < N; i += kObsThreads) {
-                unsigned u[3] = {0u, 0u, 0u};
+    const int* kvec = a.kvec;
+    // a thread's vectors and table rows stay the walker's own: kept in registers over
+    // all walkers they took 30 to 60 more
+    if constexpr (SHARED) asm volatile("" : "+s"(CS), "+s"(kvec));
+    if constexpr (!SHARED)
+        for (int b = tid; b < a.count; b += kObsThreads) cnt[b] = 0u;
+    const double* Rw = a.R + w * (int64_t)N * D;
+    for (int e = tid; e < N * 4; e += kObsThreads) {
+        const int i = e >> 2, c = e & 3;
+        pos[e] = c < D ? Rw[i * D + c] : 0.0;
+    }
+    if constexpr (sizeof(T) == 4) {
+        // 32-bit fractions of the box: the wrapping difference is the minimum image
+        for (int i = tid; i < N; i += kObsThreads) {
+            unsigned u[3] = {0u, 0u, 0u};
 #pragma unroll
-                for (int c = 0; c < D; c++) {
-                    double f = Rw[i * D + c] * a.Lr;
-                    f -= __builtin_floor(f);
-                    u[c] = (unsigned)(unsigned long long)(f * 4294967296.0);
+            for (int c = 0; c < D; c++) {
+                double f = Rw[i * D + c] * a.Lr;
+                f -= __builtin_floor(f);
+                u[c] = (unsigned)(unsigned long long)(f * 4294967296.0);
+            }
+            fix[i] = make_uint4(u[0], u[1], u[2], 0u);
+        }
+    }
+    __syncthreads();
+
+    // ------------------------------------------------------------ g(r)
+    // Work item (row i, segment): particle i stays in registers and meets the
+    // partners j = i + 1 + o (mod N) for the segment's offsets o.  Every row
+    // has M = (N-1)/2 offsets, rows i < N/2 one more (o = N/2 - 1, j = i + N/2)
+    // when N is even, so every unordered pair occurs once.  Consecutive
+    // threads hold consecutive segments of a row: with the same segment of
+    // consecutive rows the lanes of a wavefront meet their neighbours at one
+    // distance where the particles are in order, and their additions to one bin
+    // wait for each other (1-D, N = 208, 702 walkers 85 us, this way 57).
+    {
+        const int M = (N - 1) / 2;
+        const int even = (N % 2 == 0) ? 1 : 0;
+        const int S = a.gr_segs;
+        const int seg = (M + even + S - 1) / S;
+        const float sc = (float)(a.L * (1.0 / 4294967296.0));
+        for (int t = tid; t < N * S; t += kObsThreads) {
+            const int i = t / S, sg = t - i * S;
+            const int Mi = M + ((even && i < N / 2) ? 1 : 0);
+            const int o0 = sg * seg, o1 = min(Mi, o0 + seg);
+            int j = i + 1 + o0;
+            if (j >= N) j -= N;
+            if constexpr (sizeof(T) == 8) {
+                // the reference's minimum image and sum of squares, without fused multiply-adds
+#pragma clang fp contract(off)
+                const double4 ri = *reinterpret_cast<const double4*>(pos + 4 * i);
+                for (int o = o0; o < o1; o++) {
+                    const double4 rj = *reinterpret_cast<const double4*>(pos + 4 * j);
+                    double d = nic_coord_ref(ri.x - rj.x, a.L, a.Lr);
+                    double s = d * d;
+                    if constexpr (D > 1) {
+                        d = nic_coord_ref(ri.y - rj.y, a.L, a.Lr);
+                        s += d * d;
+                    }
+                    if constexpr (D > 2) {
+                        d = nic_coord_ref(ri.z - rj.z, a.L, a.Lr);
+                        s += d * d;
+                    }
+                    const double r = __builtin_sqrt(s);
+                    if (r < a.gmax) {
+                        const int bin = (int)__builtin_floor(r / a.spacing);
+                        if (bin < a.count) atomicAdd(cnt + bin, 1u);
+                    }
+                    if (++j == N) j = 0;
                 }
-                fix[i] = make_uint4(u[0], u[1], u[2], 0u);
+            } else {
+                const uint4 ui = fix[i];
+                const float gmax = (float)a.gmax, isp = (float)(1.0 / a.spacing);
+                for (int o = o0; o < o1; o++) {
+                    const uint4 uj = fix[j];
+                    float d = (float)(int)(ui.x - uj.x);
+                    float s = d * d;
+                    if constexpr (D > 1) {
+                        d = (float)(int)(ui.y - uj.y);
+                        s += d * d;
+                    }
+                    if constexpr (D > 2) {
+                        d = (float)(int)(ui.z - uj.z);
+                        s += d * d;
+                    }
+                    const float r = __builtin_amdgcn_sqrtf(s) * sc;
+                    if (r < gmax) {
+                        const int bin = (int)(r * isp);
+                        if (bin < a.count) atomicAdd(cnt + bin, 1u);
+                    }
+                    if (++j == N) j = 0;
+                }
+            }
+        }
+    }
+
+    // ------------------------------------------------------------ S(k)
+    // Vectors v < 256 R (R = V / 256) go one per thread and round over all
+    // particles.  The Vr = V mod 256 left over are split by particle residue:
+    // item (r, g), g < G = 256 / Vr, sums vector 256 R + r over the particles
+    // i = g mod G, so every thread has at most one such item.  Per-vector and
+    // per-item totals meet in LDS and are added per shell in a fixed order.
+    constexpr int kRounds = 4;
+    const bool has_item = tid < Vr * G;
+    const int ir = has_item ? tid % Vr : 0, ig = has_item ? tid / Vr : 0;
+    int nv[kRounds + 1][3];
+    double accR[kRounds + 1], accI[kRounds + 1];
+#pragma unroll
+    for (int q = 0; q <= kRounds; q++) {
+        const int v = q < kRounds ? tid + q * kObsThreads : 256 * R + ir;
+        const bool ok = q < kRounds ? q < R : has_item;
+#pragma unroll
+        for (int c = 0; c < 3; c++) nv[q][c] = (ok && c < D) ? kvec[v * 4 + c] : 0;
+        accR[q] = accI[q] = 0.0;
+    }
+    // this thread's table rows: power n[c] of axis c, all particles of the chunk
+    auto rows = [&](const int* n, const Cx<T>** r) {
+#pragma unroll
+        for (int c = 0; c < D; c++) r[c] = tab + ((size_t)c * nm + n[c]) * CS;
+    };
+    auto term = [&](const Cx<T>* const* r, int il) {
+        Cx<T> z = r[0][il];
+        if constexpr (D > 1) z = cmul(z, r[1][il]);
+        if constexpr (D > 2) z = cmul(z, r[2][il]);
+        return z;
+    };
+    for (int c0 = 0; c0 < N; c0 += a.chunk) {
+        const int nc = min(a.chunk, N - c0);
+        __syncthreads();   // previous chunk's table reads are done
+        for (int e = tid; e < nc * D; e += kObsThreads) {
+            const int il = e / D, c = e - il * D;
+            double t = pos[(c0 + il) * 4 + c] * a.Lr;
+            t -= __builtin_floor(t);
+            Cx<T>* col = tab + (size_t)c * nm * CS + il;   // power m at col[m * CS]
+            if constexpr (sizeof(T) == 8) {
+                double sn, cs;
+                sincospi(2.0 * t, &sn, &cs);
+                const Cx<T> e1{cs, sn};
+                Cx<T> pw{1.0, 0.0};
+                for (int m = 0; m < nm; m++) {
+                    col[(size_t)m * CS] = pw;
+                    pw = cmul(pw, e1);
+                }
+            } else {
+                for (int m = 0; m < nm; m++) {
+                    double u = (double)m * t;
+                    u -= __builtin_floor(u);
+                    float sn, cs;
+                    Prec<float>::sincos_small((float)u, &sn, &cs);
+                    col[(size_t)m * CS] = Cx<T>{cs, sn};
+                }
             }
         }
         __syncthreads();
-
-        // ------------------------------------------------------------ g(r)
-        // Work item (row i, segment): particle i stays in registers and meets the
-        // partners j = i + 1 + o (mod N) for the segment's offsets o.  Every row
-        // has M = (N-1)/2 offsets, rows i < N/2 one more (o = N/2 - 1, j = i + N/2)
-        // when N is even, so every unordered pair occurs once.  Consecutive
-        // threads hold consecutive rows and read consecutive partners.
-        {
-            const int M = (N - 1) / 2;
-            const int even = (N % 2 == 0) ? 1 : 0;
-            const int S = a.gr_segs;
-            const int seg = (M + even + S - 1) / S;
-            const float sc = (float)(a.L * (1.0 / 4294967296.0));
-            for (int t = tid; t < N * S; t += kObsThreads) {
-                const int sg = t / N, i = t - sg * N;
-                const int Mi = M + ((even && i < N / 2) ? 1 : 0);
-                const int o0 = sg * seg, o1 = min(Mi, o0 + seg);
-                int j = i + 1 + o0;
-                if (j >= N) j -= N;
-                if constexpr (sizeof(T) == 8) {
-                    // the reference's minimum image and sum of squares, without fused multiply-adds
-#pragma clang fp contract(off)
-                    const double4 ri = *reinterpret_cast<const double4*>(pos + 4 * i);
-                    for (int o = o0; o < o1; o++) {
-                        const double4 rj = *reinterpret_cast<const double4*>(pos + 4 * j);
-                        double d = nic_coord_ref(ri.x - rj.x, a.L, a.Lr);
-                        double s = d * d;
-                        if constexpr (D > 1) {
-                            d = nic_coord_ref(ri.y - rj.y, a.L, a.Lr);
-                            s += d * d;
-                        }
-                        if constexpr (D > 2) {
-                            d = nic_coord_ref(ri.z - rj.z, a.L, a.Lr);
-                            s += d * d;
-                        }
-                        const double r = __builtin_sqrt(s);
-                        if (r < a.gmax) {
-                            const int bin = (int)__builtin_floor(r / a.spacing);
-                            if (bin < a.count) atomicAdd(cnt + bin, 1u);
-                        }
-                        if (++j == N) j = 0;
-                    }
-                } else {
-                    const uint4 ui = fix[i];
-                    const float gmax = (float)a.gmax, isp = (float)(1.0 / a.spacing);
-                    for (int o = o0; o < o1; o++) {
-                        const uint4 uj = fix[j];
-                        float d = (float)(int)(ui.x - uj.x);
-                        float s = d * d;
-                        if constexpr (D > 1) {
-                            d = (float)(int)(ui.y - uj.y);
-                            s += d * d;
-                        }
-                        if constexpr (D > 2) {
-                            d = (float)(int)(ui.z - uj.z);
-                            s += d * d;
-                        }
-                        const float r = __builtin_amdgcn_sqrtf(s) * sc;
-                        if (r < gmax) {
-                            const int bin = (int)(r * isp);
-                            if (bin < a.count) atomicAdd(cnt + bin, 1u);
-                        }
-                        if (++j == N) j = 0;
-                    }
-                }
-            }
-        }
-
-        // ------------------------------------------------------------ S(k)
-        // Vectors v < 256 R (R = V / 256) go one per thread and round over all
-        // particles.  The Vr = V mod 256 left over are split by particle residue:
-        // item (r, g), g < G = 256 / Vr, sums vector 256 R + r over the particles
-        // i = g mod G, so every thread has at most one such item.  Per-vector and
-        // per-item totals meet in LDS and are added per shell in a fixed order.
-        constexpr int kRounds = 4;
-        const bool has_item = tid < Vr * G;
-        const int ir = has_item ? tid % Vr : 0, ig = has_item ? tid / Vr : 0;
-        int nv[kRounds + 1][3];
-        double accR[kRounds + 1], accI[kRounds + 1];
-#pragma unroll
-        for (int q = 0; q <= kRounds; q++) {
-            const int v = q < kRounds ? tid + q * kObsThreads : 256 * R + ir;
-            const bool ok = q < kRounds ? q < R : has_item;
-#pragma unroll
-            for (int c = 0; c < 3; c++) nv[q][c] = (ok && c < D) ? a.kvec[v * 4 + c] : 0;
-            accR[q] = accI[q] = 0.0;
-        }
-        // this thread's table rows: power n[c] of axis c, all particles of the chunk
-        auto rows = [&](const int* n, const Cx<T>** r) {
-#pragma unroll
-            for (int c = 0; c < D; c++) r[c] = tab + ((size_t)c * nm + n[c]) * CS;
-        };
-        auto term = [&](const Cx<T>* const* r, int il) {
-            Cx<T> z = r[0][il];
-            if constexpr (D > 1) z = cmul(z, r[1][il]);
-            if constexpr (D > 2) z = cmul(z, r[2][il]);
-            return z;
-        };
-        for (int c0 = 0; c0 < N; c0 += a.chunk) {
-            const int nc = min(a.chunk, N - c0);
-            __syncthreads();   // previous chunk's table reads are done
-            for (int e = tid; e < nc * D; e += kObsThreads) {
-                const int il = e / D, c = e - il * D;
-                double t = pos[(c0 + il) * 4 + c] * a.Lr;
-                t -= __builtin_floor(t);
-                Cx<T>* col = tab + (size_t)c * nm * CS + il;   // power m at col[m * CS]
-                if constexpr (sizeof(T) == 8) {
-                    double sn, cs;
-                    sincospi(2.0 * t, &sn, &cs);
-                    const Cx<T> e1{cs, sn};
-                    Cx<T> pw{1.0, 0.0};
-                    for (int m = 0; m < nm; m++) {
-                        col[(size_t)m * CS] = pw;
-                        pw = cmul(pw, e1);
-                    }
-                } else {
-                    for (int m = 0; m < nm; m++) {
-                        double u = (double)m * t;
-                        u -= __builtin_floor(u);
-                        float sn, cs;
-                        Prec<float>::sincos_small((float)u, &sn, &cs);
-                        col[(size_t)m * CS] = Cx<T>{cs, sn};
-                    }
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < kRounds; q++) {
-                if (q >= R) break;
-                const Cx<T>* r[D];
-                rows(nv[q], r);
-                T sr = (T)0, si = (T)0;
-#pragma unroll 4
-                for (int il = 0; il < nc; il++) {
-                    const Cx<T> z = term(r, il);
-                    sr += z.re;
-                    si += z.im;
-                }
-                accR[q] += (double)sr;
-                accI[q] += (double)si;
-            }
-            if (has_item) {
-                const Cx<T>* r[D];
-                rows(nv[kRounds], r);
-                T sr = (T)0, si = (T)0;
-                for (int il = (ig - c0 % G + G) % G; il < nc; il += G) {
-                    const Cx<T> z = term(r, il);
-                    sr += z.re;
-                    si += z.im;
-                }
-                accR[kRounds] += (double)sr;
-                accI[kRounds] += (double)si;
-            }
-        }
 #pragma unroll
         for (int q = 0; q < kRounds; q++) {
-            if (q < R) {
-                const int v = tid + q * kObsThreads;
-                part[2 * v] = accR[q];
-                part[2 * v + 1] = accI[q];
+            if (q >= R) break;
+            const Cx<T>* r[D];
+            rows(nv[q], r);
+            T sr = (T)0, si = (T)0;
+#pragma unroll 4
+            for (int il = 0; il < nc; il++) {
+                const Cx<T> z = term(r, il);
+                sr += z.re;
+                si += z.im;
             }
+            accR[q] += (double)sr;
+            accI[q] += (double)si;
         }
-        double* rest = part + 2 * 256 * R;   // [Vr][G][2]
         if (has_item) {
-            rest[2 * (ir * G + ig)] = accR[kRounds];
-            rest[2 * (ir * G + ig) + 1] = accI[kRounds];
-        }
-        __syncthreads();
-        for (int s = tid; s < a.nshell; s += kObsThreads) {
-            double cs = 0.0, sn = 0.0;
-            const int v0 = a.shell_off[s], v1 = a.shell_off[s + 1];
-            for (int v = v0; v < v1; v++) {
-                if (v < 256 * R) {
-                    cs += part[2 * v];
-                    sn += part[2 * v + 1];
-                } else {
-                    const double* p = rest + 2 * (v - 256 * R) * G;
-                    double pc = 0.0, ps = 0.0;
-                    for (int g = 0; g < G; g++) {
-                        pc += p[2 * g];
-                        ps += p[2 * g + 1];
-                    }
-                    cs += pc;
-                    sn += ps;
-                }
+            const Cx<T>* r[D];
+            rows(nv[kRounds], r);
+            T sr = (T)0, si = (T)0;
+            for (int il = (ig - c0 % G + G) % G; il < nc; il += G) {
+                const Cx<T> z = term(r, il);
+                sr += z.re;
+                si += z.im;
             }
-            a.sk_w[w * a.nshell + s] = (cs * cs + sn * sn) / ((double)N * (double)(v1 - v0));
+            accR[kRounds] += (double)sr;
+            accI[kRounds] += (double)si;
         }
-        if (a.gr_w)
-            for (int b = tid; b < a.count; b += kObsThreads) a.gr_w[w * a.count + b] = (double)cnt[b] * a.scale[b];
-        __syncthreads();   // the walker's LDS is free for the next one
     }
-    add_counts(a, cnt, tid);
+#pragma unroll
+    for (int q = 0; q < kRounds; q++) {
+        if (q < R) {
+            const int v = tid + q * kObsThreads;
+            part[2 * v] = accR[q];
+            part[2 * v + 1] = accI[q];
+        }
+    }
+    double* rest = part + 2 * 256 * R;   // [Vr][G][2]
+    if (has_item) {
+        rest[2 * (ir * G + ig)] = accR[kRounds];
+        rest[2 * (ir * G + ig) + 1] = accI[kRounds];
+    }
+    __syncthreads();
+    for (int s = tid; s < a.nshell; s += kObsThreads) {
+        double cs = 0.0, sn = 0.0;
+        const int v0 = a.shell_off[s], v1 = a.shell_off[s + 1];
+        for (int v = v0; v < v1; v++) {
+            if (v < 256 * R) {
+                cs += part[2 * v];
+                sn += part[2 * v + 1];
+            } else {
+                const double* p = rest + 2 * (v - 256 * R) * G;
+                double pc = 0.0, ps = 0.0;
+                for (int g = 0; g < G; g++) {
+                    pc += p[2 * g];
+                    ps += p[2 * g + 1];
+                }
+                cs += pc;
+                sn += ps;
+            }
+        }
+        a.sk_w[w * a.nshell + s] = (cs * cs + sn * sn) / ((double)N * (double)(v1 - v0));
+    }
+    if (a.gr_w)
+        for (int b = tid; b < a.count; b += kObsThreads) a.gr_w[w * a.count + b] = (double)cnt[b] * a.scale[b];
+    if constexpr (!SHARED) add_counts(a, cnt, tid);
+}
+
+template <typename T, int D, bool SHARED>
+__global__ __launch_bounds__(kObsThreads) void obs_kernel(ObsArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    if constexpr (SHARED) {
+        unsigned* cnt = obs_counts<T, D>(a, smem);
+        for (int b = threadIdx.x; b < a.count; b += kObsThreads) cnt[b] = 0u;
+        for (int64_t w = blockIdx.x; w < a.W; w += gridDim.x) {
+            obs_walker<T, D, true>(a, w, smem);
+            __syncthreads();   // the walker's LDS is free for the next one
+        }
+        add_counts(a, cnt, threadIdx.x);
+    } else {
+        obs_walker<T, D, false>(a, blockIdx.x, smem);
+    }
 }
 
 // FP64 form in 2-D and 3-D.
@@ -547,16 +579,27 @@ size_t obs_lds_bytes(int N, int D, int V, int chunk, int nmax, int count, bool f
            (size_t)(chunk + 1) * D * (nmax + 1) * cx + (size_t)count * sizeof(unsigned);
 }
 
-// Workgroups.  One walker each from N = 200 on (or where each walker's g(r) is
+// Workgroups.  One walker each from N = alone on (or where each walker's g(r) is
 // asked for): the pair loop hides the additions to the totals, and the last
 // workgroups leave no CU waiting (N = 343, 16384 walkers: 1774 us, 1960 with 16
-// walkers each).  Smaller walkers: 1024 workgroups, at most 1024 walkers each
-// (their counts have 32 bits).
-static unsigned obs_grid(const ObsArgs& a)
+// walkers each; the 1-D FP64 form from N = 100: N = 166, 10615 walkers 452 us, 537
+// shared), and of fewer than 1536 walkers (which wait for the workgroups that have
+// two: N = 7, 1129 walkers 24 us, 28 shared).  Otherwise 1024 workgroups, at most
+// 1024 walkers each (their counts have 32 bits).
+static unsigned obs_grid(int N, int64_t W, bool per_walker, int alone)
 {
-    if (a.gr_w || a.N >= 200) return (unsigned)a.W;
-    const int64_t least = (a.W + 1023) / 1024, most = a.W < 1024 ? a.W : 1024;
-    return (unsigned)(least > most ? least : most);
+    if (per_walker || N >= alone || W < 1536) return (unsigned)W;
+    return (unsigned)std::max<int64_t>(1024, (W + 1023) / 1024);
+}
+constexpr int kMfmaAlone = 200;
+
+// A workgroup of one walker with few pairs spends more on staging the bins'
+// thresholds than its pairs save: N = 12, 1000 bins, 192 walkers 11.7 us without,
+// 13.8 with them; N = 5, 808 walkers 17.4 and 20.4; N = 19 (1000 bins) and N = 5 (50
+// bins) are even.
+bool obs_mfma_pays(int N, int count, int64_t W, bool per_walker)
+{
+    return (int64_t)obs_grid(N, W, per_walker, kMfmaAlone) < W || 3LL * N * (N - 1) >= count;
 }
 
 size_t obs_mfma_lds_bytes(int N, int D, int chunk, int nmax, int count, int npair)
@@ -571,7 +614,7 @@ size_t obs_mfma_lds_bytes(int N, int D, int chunk, int nmax, int count, int npai
 hipError_t launch_obs_mfma(const ObsArgs& a, int D, size_t lds, hipStream_t st)
 {
     if (a.W <= 0) return hipSuccess;
-    const dim3 grid(obs_grid(a)), block(kObsThreads);
+    const dim3 grid(obs_grid(a.N, a.W, a.gr_w, kMfmaAlone)), block(kObsThreads);
     if (D == 2)
         hipLaunchKernelGGL(obs_mfma_kernel<2>, grid, block, lds, st, a);
     else
@@ -579,15 +622,23 @@ hipError_t launch_obs_mfma(const ObsArgs& a, int D, size_t lds, hipStream_t st)
     return hipGetLastError();
 }
 
+template <typename T, int D>
+static void launch_obs_d(const ObsArgs& a, size_t lds, hipStream_t st)
+{
+    const unsigned grid = obs_grid(a.N, a.W, a.gr_w, sizeof(T) == 8 ? 100 : 200);
+    if (grid < a.W)
+        hipLaunchKernelGGL((obs_kernel<T, D, true>), dim3(grid), dim3(kObsThreads), lds, st, a);
+    else
+        hipLaunchKernelGGL((obs_kernel<T, D, false>), dim3(grid), dim3(kObsThreads), lds, st, a);
+}
 template <typename T>
 hipError_t launch_obs(const ObsArgs& a, int D, size_t lds, hipStream_t st)
 {
     if (a.W <= 0) return hipSuccess;
-    const dim3 grid(obs_grid(a)), block(kObsThreads);
     switch (D) {
-    case 1: hipLaunchKernelGGL((obs_kernel<T, 1>), grid, block, lds, st, a); break;
-    case 2: hipLaunchKernelGGL((obs_kernel<T, 2>), grid, block, lds, st, a); break;
-    default: hipLaunchKernelGGL((obs_kernel<T, 3>), grid, block, lds, st, a); break;
+    case 1: launch_obs_d<T, 1>(a, lds, st); break;
+    case 2: launch_obs_d<T, 2>(a, lds, st); break;
+    default: launch_obs_d<T, 3>(a, lds, st); break;
     }
     return hipGetLastError();
 }
