@@ -200,7 +200,10 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
     const T hinv = (T)(sy.hinv / scale * C::kUnit), rc = (T)(sy.rc * scale / C::kUnit);
     const T cin = (T)(sy.cinv * unit_len), unitR = (T)unit_len;
     // WIDE: LDS address of the lane's copy of a row, byte 1 the row (two, for the
-    // old and the new distance)
+    // old and the new distance).  Right only while the table starts at LDS address
+    // 0, that is while the kernel has no static LDS (tests/test_kernel_registers_cpu.py
+    // reads that from the built kernels); adding the start to each address instead
+    // is two more instructions a pair
     uint32_t row_at[2];
     row_at[0] = row_at[1] = (uint32_t)(uintptr_t)(LdsBytes)smem + (tid & (kWide - 1)) * sizeof(Vec4<T>);
     auto uof = [&](T r, int q = 0) -> T {

@@ -33,3 +33,11 @@ def test_mixed_observables_keep_eight_wavefronts(built):
     assert len(found) == 3
     for name, v in found:
         assert v["vgpr_count"] <= 64 and v["vgpr_spill_count"] == 0, (name, v)
+
+
+def test_wide_spline_table_starts_at_lds_address_zero(built):
+    # its rows' addresses are made by writing the row into byte 1 (kernels_sweep.hip): static LDS would come first
+    found = [(k, v) for k, v in built.items() if re.search(r"sweep_kernel<float, \d, \d+, \d, true, false, true>", k)]
+    assert len(found) == 72
+    for name, v in found:
+        assert v["group_segment_fixed_size"] == 0, (name, v)
