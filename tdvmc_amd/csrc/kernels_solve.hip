@@ -30,7 +30,10 @@ namespace tdvmc {
 namespace {
 
 constexpr int kThreads = 1024;
-constexpr int kNB = 16, kLDP = kNB + 1;   // solve_ahead_body: block width, LDS stride of a panel row
+// solve_ahead_body: block width, LDS stride of a panel row, 64-entry pieces of a
+// row that the back substitution loads ahead, the largest system it is used for
+constexpr int kNB = 16, kLDP = kNB + 1, kRowPieces = 6, kAheadMaxP = 340;
+static_assert(kAheadMaxP <= 64 * kRowPieces + kNB, "the back substitution holds a whole row");
 
 typedef double double4v __attribute__((ext_vector_type(4)));
 
@@ -720,7 +723,7 @@ __device__ __forceinline__ void solve_ahead_body(const SolveArgs& a)
         const int c = e / kNB, j = e % kNB;
         diag[c * kLDP + j] = Lm[(size_t)c * LD + c / kNB * kNB + j];
     }
-    constexpr int NQ = 6;   // 64 entries each: up to P = 400
+    constexpr int NQ = kRowPieces;
     double lr[NQ];
     auto load_row = [&](int p0) {
         const double* row = Lm + (size_t)(p0 + wv) * LD + p0 + kNB;
@@ -1080,11 +1083,12 @@ constexpr size_t kMaxPanelLds = 150 * 1024;   // beside the static LDS (NB x NB 
 // 340 (at P = 296 the whole call with its copies takes 229 us, with solve_body
 // 447).  Above, 32 columns (fewer panels and barriers: at P = 420, 705 against
 // 738 us with 16), and 16 again where the panel of 32 no longer fits in LDS.
-// solve_ahead_body would be the faster one up to P = 608 (P = 560: 743 against
-// 1315 us) but with 16 columns its sums are grouped otherwise than with 32: a
-// nearly singular S of a few hundred parameters turns such a last-bit change
-// into 1e-9 of the stepped parameters, so those sizes keep their 32 columns.
-constexpr int kAheadMaxP = 340;
+// With more pieces of a row held ahead (kRowPieces; as it stands it takes up to P
+// = 400) solve_ahead_body was the faster one up to P = 608, where its panels no
+// longer fit the LDS (P = 560: 743 against 1315 us).  Up to 581 its 16 columns group
+// the sums otherwise than 32 do: a nearly singular S of a few hundred parameters
+// turns such a last-bit change into 1e-9 of the stepped parameters, so those
+// sizes keep their 32 columns; 582 to 608 are left with solve_body's 16.
 size_t solve_lds_bytes(int NB, int P)
 {
     if (NB == 0) return ((size_t)(2 * ahead_rows(P) - kNB) * kLDP + 2 * (size_t)((P + kNB - 1) / kNB * kNB)) * sizeof(double);
