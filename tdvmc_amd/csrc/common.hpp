@@ -121,7 +121,7 @@ __device__ __forceinline__ double u01d(uint32_t hi, uint32_t lo)
 template <typename T> struct Prec;
 
 template <> struct Prec<float> {
-    // start value of a sum of squares handed to sqrt_r2 / r_and_rinv
+    // start value of a sum of squares handed to sqrt_r2
     static constexpr float kR2Floor = 0.0f;
     __device__ static __forceinline__ float sqrt_r2(float x) { return __builtin_amdgcn_sqrtf(x); }
     __device__ static __forceinline__ float rint_(float x) { return __builtin_rintf(x); }
@@ -162,9 +162,10 @@ template <> struct Prec<double> {
     // x^(-1/2) / 2 to 2^-46, the remainder x - g^2 (exact in an FMA) then
     // x^(1/2) rounded as the general square root rounds it (but for results
     // within 2^-92 of a tie), 8 instructions in all, and two more x^(-1/2)
-    // within an ulp.  Sums of squares start at kR2Floor, which no sum of a
-    // nonzero displacement notices: coincident particles get r = 2^-500 (the
-    // knot position of r = 0) and 1/r = infinity, and a NaN stays one.
+    // within an ulp.  A NaN stays one.
+    // sqrt_r2: sums of squares start at kR2Floor, so that coincident particles get
+    // r = 2^-500 (the knot position of r = 0; so do displacements below about that),
+    // and a sum that overflows gives a NaN, which no cutoff test lets pass.
     static constexpr double kR2Floor = 0x1p-1000;
     __device__ static __forceinline__ void rsq_step(double x, double* g, double* h)
     {
@@ -190,10 +191,18 @@ template <> struct Prec<double> {
         double h;
         rsq_step(r2, r, &h);
         h += h;
-        h = __builtin_fma(h, __builtin_fma(-*r, h, 1.0), h);
-        // h is 2^500 here for coincident particles: infinity with its exponent raised
-        const int hi = __double2hiint(h);
-        *rinv = __hiloint2double(r2 <= 0x1p-990 ? 0x7ff00000 : hi, __double2loint(h));
+        *rinv = __builtin_fma(h, __builtin_fma(-*r, h, 1.0), h);
+        // below 2^-999 and from 2^1023 on (0 and infinity among them) the step's
+        // products leave the range
+        const bool odd = (unsigned)__double2hiint(r2) - 0x01800000u >= 0x7fe00000u - 0x01800000u;
+        if (__builtin_amdgcn_ballot_w64(odd)) {
+            // behind a branch that hardly any wave takes
+            asm volatile("" ::: "memory");
+            if (odd) {
+                *r = __builtin_sqrt(r2);
+                *rinv = 1.0 / *r;
+            }
+        }
     }
     // Quarter turn q = rint(4 t), the remainder f = t - q / 4 in [-1/8, 1/8]
     // (exact), the Taylor series of sin and cos in 2 pi f (truncated below

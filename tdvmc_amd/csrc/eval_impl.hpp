@@ -295,13 +295,14 @@ __device__ __forceinline__ void eval_pairs(const KSys& sy, const typename Coord<
 
             auto pair = [&]() {
                 T d[D];
-                T r2 = Prec<T>::kR2Floor;
+                T r2 = (T)0;
 #pragma unroll
                 for (int a = 0; a < D; a++) {
                     d[a] = C::diff(rn[a], cp[a]);
                     r2 += d[a] * d[a];
                 }
-                // FP32: one v_rsq gives 1/r, and r = r^2 / r; FP64: sqrt and a divide
+                // FP32: one v_rsq gives 1/r, and r = r^2 / r; FP64: r and 1/r from v_rsq_f64 and
+                // one coupled step
                 T r, rinv;
                 Prec<T>::r_and_rinv(r2, &r, &rinv);
                 if constexpr (!PER && POT != 0) vs += pair_pot<T, POT>(pc, r, r2, rinv);
