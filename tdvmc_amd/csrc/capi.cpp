@@ -130,6 +130,7 @@ struct tdvmc_ctx {
     double* ws_dev = nullptr;
     double* ws_pin = nullptr;
     size_t ws_dev_cap = 0, ws_pin_cap = 0;   // doubles
+    size_t ws_asked = 0;                     // the largest call so far that a pinned block could serve
     tdvmc_batch* batch = nullptr;            // the batch this context is a member of
     bool params_in_batch = false;            // the parameters are those of the batch's last step (and host_params_stale)
     MomentsWork mw{};
@@ -225,7 +226,10 @@ void dfree(T*& p)
 // all) travel through a pinned buffer, the results in one copy: an
 // allocation and release per array and a copy per result were most of a small
 // call (16 configurations of 64 particles: 107 us, 15 of them in the kernel).
-constexpr size_t kWsDevice = (size_t)64 << 20, kWsPinned = (size_t)1 << 20;
+// A pinned block above kWsPinnedAtOnce is first allocated by a context's second
+// call of that size: where the process has none yet it costs up to 0.7 ms (768 KB:
+// 868 us instead of 176 for that call, 88 instead of 129 for each after it).
+constexpr size_t kWsDevice = (size_t)64 << 20, kWsPinned = (size_t)1 << 20, kWsPinnedAtOnce = (size_t)64 << 10;
 class Arena {
 public:
     explicit Arena(tdvmc_ctx* c) : ctx(c) {}
@@ -264,6 +268,10 @@ public:
             own = true;
         }
         pinned = total * sizeof(double) <= kWsPinned;
+        if (pinned && ctx->ws_pin_cap < total && total * sizeof(double) > kWsPinnedAtOnce && ctx->ws_asked < total) {
+            pinned = false;
+            ctx->ws_asked = total;
+        }
         if (pinned && ctx->ws_pin_cap < total) {
             if (ctx->ws_pin) (void)hipHostFree(ctx->ws_pin);
             ctx->ws_pin = nullptr;

@@ -11,10 +11,12 @@ extern "C" {
 
 int shim_refuse_pinned = 0;    // hipHostMalloc returns hipErrorOutOfMemory
 int shim_refused = 0;          // how often it did
+size_t shim_pinned = 0;        // bytes asked of hipHostMalloc
 size_t shim_most_lds = 0;      // largest dynamic LDS of the launches since it was cleared
 
 int hipHostMalloc(void** ptr, size_t size, unsigned flags)
 {
+    shim_pinned += size;
     if (shim_refuse_pinned) {
         shim_refused++;
         *ptr = nullptr;
