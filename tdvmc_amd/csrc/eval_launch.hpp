@@ -36,17 +36,22 @@ static hipError_t launch_eval_w(const KSys& sy, const KTables<T>& tb, const doub
 //     after the other: N = 14, 206 terms, 48 knots, 1328 walkers 158 / 70 / 63; N = 27,
 //     101 terms, 2291 walkers 77 / 67 / 61, N = 16, 101 terms, 11568 walkers 173 /
 //     173 / 208, N = 20, 206 terms, 2063 walkers 176 / 106 / 87.
-// Where all hold: N = 8 (16384 walkers) 55 / 85 / 141; N = 25 (2-D, 16 terms, 4099)
-// 67 / 66 / 136; N = 38 (2-D, 64 terms, 7876) 107 / 114 / 137; N = 64 (16384) 154 / 147 /
-// 181; N = 96 (8192) 196 / 154 / 160; N = 128 (8192) 267 / 191 / 180; with per-particle
-// output N = 33 (8192) 74 / 81 / 92, N = 64 193 / 180 / 174.  The mixed form keeps
-// four: its FP32 sums are added up per wavefront.
+// Where all hold, up to N = 32 one, to 64 two (with per-particle output, whose
+// sums per particle the wavefronts share: 16 and 36).  1 / 2 / 4, us: N = 8 (16384
+// walkers) 55 / 85 / 141; N = 25 (2-D, 16 terms, 4099) 67 / 66 / 136; N = 30 (2-D trap,
+// 8 knots, complex, 2100) 32 / 30 / 32; N = 38 (2-D, 64 terms, 7876) 107 / 114 / 137;
+// N = 48 (2-D trap, 48 knots, 3200) 60 / 48 / 47; N = 64 (16384) 154 / 147 / 181;
+// N = 90 (2-D trap, 24 knots, 2100) 105 / 74 / 58; N = 96 (8192) 196 / 154 / 160; N = 128
+// (8192) 267 / 191 / 180; with per-particle output N = 33 (8192) 74 / 81 / 92, N = 40
+// (2-D trap, 48 knots, 2100) 46 / 40 / 34, N = 48 (same) 53 / 44 / 37.  The mixed form
+// keeps four: its FP32 sums are added up per wavefront.
 template <typename T>
 static int eval_waves(const KSys& sy, bool pp, int64_t W)
 {
-    if (sizeof(T) == 4 || sy.N > (pp ? 48 : 100)) return 4;
+    const int one = pp ? 16 : 32, two = pp ? 36 : 64;   // particles
+    if (sizeof(T) == 4 || sy.N > two) return 4;
     auto workgroups = [&](int wpw) { return 160 * 1024 / ((4 / wpw) * eval_lds_bytes<T>(sy, pp, wpw)); };
-    if (sy.N <= 48 && W >= 2048 && sy.Kh <= 64 && workgroups(1) >= 3) return 1;
+    if (sy.N <= one && W >= 2048 && sy.Kh <= 64 && workgroups(1) >= 3) return 1;
     if (W >= 1024 && sy.Kh <= 200 && workgroups(2) >= 4) return 2;
     return 4;
 }

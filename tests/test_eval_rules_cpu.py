@@ -43,6 +43,10 @@ def test_fewer_wavefronts_leave_the_chip_full(D, pp):
     ((3, 5, 48, 257, 5915, 0), 4),
     # 588 walkers, 101 terms: 25 us with four, 32 with two
     ((3, 19, 24, 101, 588, 0), 4),
+    # 3200 walkers in a 2-D trap, 48 knots: 60 us with one, 48 with two; per-particle output 69, 58 and 48 with four
+    ((2, 48, 48, 0, 3200, 0), 2),
+    ((2, 48, 48, 0, 3200, 1), 4),
+    ((2, 90, 24, 0, 2100, 0), 4),
     # the sizes the fewer wavefronts were measured at
     ((2, 25, 12, 16, 4099, 0), 1),
     ((3, 64, 32, 0, 16384, 0), 2),
