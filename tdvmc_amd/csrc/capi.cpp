@@ -994,10 +994,9 @@ constexpr int kObsMaxBins = 8192;
 // Segments per row of g(r)'s pair loop: enough work items for the workgroup's
 // 256 threads twice, and (fullest) the count whose last round of items and last
 // partner of a segment are fullest (N = 343: 8 segments keep 95 % of the lanes
-// busy, the 2 that 512 items need 89 %).  Not in the mixed form in 3-D from N = 120
-// to 220, where the banks of the partners' reads decide (N = 142: 4 segments 161 us,
-// 9 173; N = 192: 3 and 4, 134 and 140; N = 214: 3 and 7, 137 and 145; outside, N = 110:
-// 5 and 11, 141 and 138; N = 300: 2 and 5, 91 and 85).
+// busy, the 2 that 512 items need 89 %).  Not in the mixed form in 3-D, whose reads
+// of the partners decide (N = 142: 4 segments 161 us, 9 173; N = 214: 3 and 7, 137 and
+// 145).
 int gr_segments(int N, bool fullest)
 {
     const int M = N / 2;   // partners of a row
@@ -1177,7 +1176,7 @@ int enqueue_obs(tdvmc_ctx* ctx, int prec, const double* dR, int64_t W, double* g
     a.nshell = o.nshell;
     a.nmax = o.nmax;
     a.chunk = chunk;
-    a.gr_segs = gr_segments(N, !f32 || D < 3 || N < 120 || N > 220);
+    a.gr_segs = gr_segments(N, !f32 || D < 3);
     a.sk_w = sk_w;
     hipEvent_t ev{};
     int rc = prof_begin(ctx, "observables", &ev);
