@@ -629,18 +629,18 @@ __device__ __forceinline__ void eval_kgrad(const KSys& sy, const KTables<T>& tb,
 // e_a = e^{2 pi i x_a}, leaves 4 for the term that follows another along the
 // last axis.  16384 walkers, whole measurement: N = 343, 128 terms (rho_k
 // handed over) 3.23 -> 2.97 ms; 2-D, N = 400, 258 terms 6.86 -> 5.73 ms.
-// Below kRunTerms terms per wavefront the D sincos of the particle and the
-// chain of a run's dependent products cost more than they save, and the start
-// of a run costs up to D products: the direct form runs there, and for at most 32
-// particles (which it spreads over both half-waves) where a run holds fewer than
-// kRunLength terms on average, as in 3-D.  Direct and run form, us: N = 25 (2-D),
-// 16 terms, 4 a wavefront 61 / 65; N = 14 (3-D), 206 terms in 68 runs, 1328
+// Below 12 terms per wavefront (8 in long runs, as in 1-D) the D sincos of the
+// particle and the chain of a run's dependent products cost more than they save,
+// and the start of a run costs up to D products: the direct form runs there, and
+// for at most 32 particles (which it spreads over both half-waves) where a run
+// holds fewer than 4 terms on average, as in 3-D.  Direct and run form, us: N = 25
+// (2-D), 16 terms, 4 a wavefront 61 / 65; N = 14 (3-D), 206 terms in 68 runs, 1328
 // walkers, two wavefronts 74 / 70, four 63 / 66; N = 5 (3-D), 101 terms in 41 runs,
-// 481 walkers 20.5 / 22.1.
-constexpr int kRunTerms = 12, kRunLength = 4;
+// 481 walkers 20.5 / 22.1; N = 108 (1-D), 40 terms, 6570 walkers, four wavefronts, the
+// whole call with its moments 448 / 395.
 __host__ __device__ inline bool eval_use_runs(const KSys& sy, int wpw)
 {
-    return sy.Kh >= kRunTerms * wpw && (sy.N > 32 || sy.Kh >= kRunLength * sy.nrun);
+    return sy.Kh >= (sy.Kh >= 8 * sy.nrun ? 8 : 12) * wpw && sy.Kh > 0 && (sy.N > 32 || sy.Kh >= 4 * sy.nrun);
 }
 struct Cplx {
     double x, y;
@@ -792,7 +792,7 @@ __device__ __forceinline__ void eval_kgrad_runs(const KSys& sy, const KTables<do
 // Particles per pass for nt threads (0: a thread computes its terms' sincos).
 // Small walkers keep the direct sums, whose few sincos cost less than the
 // table's barriers: N = 16 (2-D), 16 terms, 276 walkers 18.3 us, with the table
-// 25.7; N = 32 (3-D), 9 terms, 7196 walkers 143 and 265 (four wavefronts), 110 and
+// 25.7 (N = 180, 3 terms, 3 walkers, the whole call: 85 and 67); N = 32 (3-D), 9 terms, 7196 walkers 143 and 265 (four wavefronts), 110 and
 // 114 (two).  So do walkers whose LDS holds less than an eighth of their
 // particles (or of 64): N = 86 (2-D), 8 knots, 64 terms, 525 walkers 45 and 81.
 struct RhoTable {
@@ -801,7 +801,7 @@ struct RhoTable {
 __host__ __device__ inline RhoTable rho_table_particles(const KSys& sy, size_t bytes, int nt)
 {
     const int K = sy.Kh, terms = nt == 256 ? 2 : (nt == 128 ? 3 : 5);   // terms per thread
-    if (sy.D < 2 || sy.N < 48 || K < 8 || K > terms * nt) return RhoTable{0, 0};
+    if (sy.D < 2 || sy.N < 48 || K < 1 || K > terms * nt) return RhoTable{0, 0};
     const size_t cx = 2 * sizeof(double), row = cx * sy.D * (2 * sy.kmax + 1);
     int G = nt > K ? nt / K : 1;
     while (G > 1 && cx * G * K + row > bytes) G--;

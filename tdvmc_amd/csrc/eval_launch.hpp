@@ -36,7 +36,8 @@ static hipError_t launch_eval_w(const KSys& sy, const KTables<T>& tb, const doub
 //     after the other: N = 14, 206 terms, 48 knots, 1328 walkers 158 / 70 / 63; N = 27,
 //     101 terms, 2291 walkers 77 / 67 / 61, N = 16, 101 terms, 11568 walkers 173 /
 //     173 / 208, N = 20, 206 terms, 2063 walkers 176 / 106 / 87.
-// Where all hold, up to N = 32 one, to 64 two (with per-particle output, whose
+// Where all hold, up to N = 32 one, to 80 two (64 in open space, where most pairs
+// fall into a few of the histogram's intervals; with per-particle output, whose
 // sums per particle the wavefronts share: 16 and 36).  1 / 2 / 4, us: N = 8 (16384
 // walkers) 55 / 85 / 141; N = 25 (2-D, 16 terms, 4099) 67 / 66 / 136; N = 30 (2-D trap,
 // 8 knots, complex, 2100) 32 / 30 / 32; N = 38 (2-D, 64 terms, 7876) 107 / 114 / 137;
@@ -48,7 +49,7 @@ static hipError_t launch_eval_w(const KSys& sy, const KTables<T>& tb, const doub
 template <typename T>
 static int eval_waves(const KSys& sy, bool pp, int64_t W)
 {
-    const int one = pp ? 16 : 32, two = pp ? 36 : 64;   // particles
+    const int one = pp ? 16 : 32, two = pp ? 36 : (sy.periodic ? 80 : 64);   // particles
     if (sizeof(T) == 4 || sy.N > two) return 4;
     auto workgroups = [&](int wpw) { return 160 * 1024 / ((4 / wpw) * eval_lds_bytes<T>(sy, pp, wpw)); };
     if (sy.N <= one && W >= 2048 && sy.Kh <= 64 && workgroups(1) >= 3) return 1;

@@ -47,6 +47,7 @@ def test_fewer_wavefronts_leave_the_chip_full(D, pp):
     ((2, 48, 48, 0, 3200, 0), 2),
     ((2, 48, 48, 0, 3200, 1), 4),
     ((2, 90, 24, 0, 2100, 0), 4),
+    ((1, 70, 29, 5, 12357, 0), 2),
     # the sizes the fewer wavefronts were measured at
     ((2, 25, 12, 16, 4099, 0), 1),
     ((3, 64, 32, 0, 16384, 0), 2),
@@ -62,7 +63,10 @@ def test_measured_sizes(row, waves):
     (3, 5, 24, 101, 41, 3, (0, 0, 0), 0),
     (2, 25, 12, 16, 5, 3, (0, 0, 0), 0),            # few terms
     (2, 25, 8, 50, 11, 5, (1, 1, 1), 0),
-    (1, 20, 8, 11, 1, 11, (0, 0, 0), 0),
+    (1, 20, 8, 7, 1, 7, (0, 0, 0), 0),
+    (1, 20, 8, 11, 1, 11, (1, 0, 0), 0),
+    (1, 108, 47, 40, 1, 40, (1, 1, 1), 0),
+    (3, 180, 12, 3, 3, 1, (0, 0, 0), 1),
     (1, 20, 8, 24, 1, 24, (1, 1, 0), 0),
     (3, 33, 24, 32, 18, 2, (1, 1, 0), 0),
     (3, 47, 24, 128, 47, 4, (1, 1, 1), 0),

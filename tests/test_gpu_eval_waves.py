@@ -23,7 +23,7 @@ CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "build",
 CASES = [(1, 1, 1, 5, 20, 6, 2049), (1, 1, 1, 16, 127, 8, 2050), (1, 1, 2, 2, 10, 4, 2051), (1, 2, 2, 25, 30, 12, 4099), (1, 1, 2, 16, 126, 16, 2049),
          (1, 1, 3, 7, 0, 24, 2050), (1, 2, 3, 32, 60, 10, 2051), (1, 1, 3, 13, 122, 8, 2049), (1, 2, 2, 31, 126, 8, 2049), (2, 2, 1, 30, 300, 6, 1025),
          (2, 2, 2, 9, 64, 8, 1025), (2, 2, 2, 33, 374, 8, 2049), (2, 2, 3, 16, 200, 8, 1027), (2, 2, 3, 36, 26, 24, 1025), (2, 4, 3, 48, 256, 10, 1025),
-         (2, 4, 2, 64, 100, 24, 1025), (2, 4, 3, 63, 131, 10, 1025), (2, 4, 3, 50, 66, 16, 1025), (4, 4, 3, 65, 131, 10, 1025)]
+         (2, 4, 2, 64, 100, 24, 1025), (2, 4, 3, 63, 131, 10, 1025), (2, 4, 3, 50, 66, 16, 1025), (2, 4, 3, 80, 66, 10, 1025), (4, 4, 3, 81, 66, 10, 1025)]
 
 
 @pytest.mark.parametrize("real", [True, False])
