@@ -1251,13 +1251,15 @@ __device__ __forceinline__ void eval_body(const KSys& sy, const KTables<T>& tb, 
 }
 
 // WPW wavefronts per walker, 4 / WPW walkers per workgroup (slot_bytes of LDS
-// each).  The mixed form without per-particle output is held to the registers of
-// five wavefronts per SIMD: in 3-D the compiler's choice was one more than that
-// (129 terms, N = 72, 1194 walkers 34 -> 40 us with four).
+// each).  The mixed 3-D form without per-particle output is held to the
+// registers of five wavefronts per SIMD: the compiler's choice was one more than
+// that (129 terms, N = 72, 1194 walkers 34 -> 40 us with four).  1-D and 2-D fit
+// by themselves, and the bound only made a slower order of the same registers
+// (2-D, N = 400, 512 terms, 32768 walkers 7.05 -> 7.26 ms).
 template <typename T, int D, bool PP, bool PER, typename TO, int WPW>
-__global__ __launch_bounds__(kThreads, sizeof(T) == 4 && !PP ? 5 : 4) void eval_kernel(KSys sy, KTables<T> tb, const double* __restrict__ Rg,
-                                                         int64_t W, EvalOut<TO> out, const T* __restrict__ rho_in,
-                                                         size_t slot_bytes)
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 && D == 3 && !PP ? 5 : 4) void eval_kernel(
+    KSys sy, KTables<T> tb, const double* __restrict__ Rg, int64_t W, EvalOut<TO> out, const T* __restrict__ rho_in,
+    size_t slot_bytes)
 {
     constexpr int NS = 4 / WPW;
     const int slot = NS == 1 ? 0 : threadIdx.x / (64 * WPW);
