@@ -22,6 +22,10 @@
  *   - one context owns its device buffers and one HIP stream; calls on one
  *     context are not thread-safe, distinct contexts may be used concurrently;
  *     calls returning host data synchronise the context's stream;
+ *   - a context keeps the workspace of its largest call on host arrays so far, at
+ *     most 64 MiB of device and 1 MiB of pinned host memory, until it is
+ *     destroyed; larger calls give theirs back, and where the system refuses
+ *     pinned memory a call does without;
  *   - precision: TDVMC_FP64 (plain form) or TDVMC_MIXED (FP32 pair / spline /
  *     phase arithmetic, split-bf16 (bf16x6) MFMA moments, FP64 solve); TDVMC_PRECISION_DEFAULT
  *     selects the context's configured precision.

@@ -1,6 +1,7 @@
 // Wavefunction evaluation of walker configurations: ln psi, O_k = d ln psi /
 // d alpha_k, local energy E_L, and (optionally) the per-particle gradient and
-// Laplacian of ln psi.  One workgroup of 4 wavefronts evaluates one walker.
+// Laplacian of ln psi.  A workgroup of 4 wavefronts evaluates one walker, or two or
+// four with 2 or 1 wavefronts each (FP64 form and batches).
 //
 // Restates src/PhysicalSystems/BosonsBulk.cpp:179-218 (basis sums O_k and the
 // outer-pair count), :220-336 (pair potential, gradient and Laplacian pieces),

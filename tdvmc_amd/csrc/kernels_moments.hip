@@ -397,8 +397,9 @@ __global__ __launch_bounds__(256) void small_partial_kernel(const TO* __restrict
                                                             const double* __restrict__ EI, int64_t W, int P, ColSrc cs,
                                                             int nb, double* __restrict__ mean, double* __restrict__ part)
 {
-    // rows 16 doubles apart from a multiple of 32 banks' width: the 4 rows of
-    // an MFMA operand sit in different banks
+    // 68 doubles a row: the rows of an MFMA operand (16 doubles each) start 8 banks
+    // apart, so two that are read together share 24 of 32 banks, where 64 doubles
+    // would put them in the same ones
     constexpr int LD = kSmallCols + 4;
     __shared__ double X[kSmallRows * LD];
     __shared__ double m[4][kSmallCols];

@@ -23,9 +23,9 @@
 // FP64 form: distances by the reference's minimum image (src/Utils.cpp:266-281)
 // and the bin of the reference's FP64 division, powers by complex recurrence
 // from one sincospi; in 2-D and 3-D obs_mfma_kernel below takes S(k) as a matrix
-// product and the bins from thresholds of r^2.  Mixed form: FP32 distances from the wrapping difference of 32-bit
-// box fractions (exact minimum image), FP32 powers each from its own reduced
-// phase, FP32 sums per chunk added in FP64.
+// product and the bins from thresholds of r^2.  Mixed form: FP32 distances from
+// the wrapping difference of 32-bit box fractions (exact minimum image), FP32
+// powers each from its own reduced phase, FP32 sums per chunk added in FP64.
 
 #include <algorithm>
 #include <type_traits>
@@ -362,8 +362,8 @@ __global__ __launch_bounds__(kObsThreads) void obs_kernel(ObsArgs a)
 //   g(r): the bin is a monotone function of the squared distance s, so its
 //   boundaries in s (the exact ones, found on the host by the same square root
 //   and division) decide it; an FP32 guess of the bin is it or the one below.  The
-//   same bins as floor(sqrt(s) / spacing), without the 30-odd instructions of
-//   the FP64 square root and division per pair.
+//   bins of the same s are those of floor(sqrt(s) / spacing), without the 30-odd
+//   instructions of the FP64 square root and division per pair.
 // N = 343 3-D, 16384 walkers, 200 bins: 3.81 -> 1.77 ms; N = 400 2-D, 8192
 // walkers: 1.71 -> 0.83 ms.
 typedef double double4v __attribute__((ext_vector_type(4)));
@@ -371,7 +371,9 @@ constexpr int kObsTiles = 2;   // tiles per wavefront
 
 // nic_coord_ref where the displacement is not within 1e-6 of half the box of
 // its image (there the rounding of x / L + 1/2 and the nudge decide: near is
-// set, and the caller takes nic_coord_ref)
+// set, and the caller takes nic_coord_ref).  One multiply-add, as the compiler
+// makes of nic_coord_ref's x - k L: past one box it rounds once, and a pair whose
+// r / spacing is then an integer to the last bit can fall to either side of it.
 __device__ __forceinline__ double nic_coord_fast(double x, double L, double Lr, double near_half, bool* near)
 {
     const double res = __builtin_fma(-__builtin_rint(x * Lr), L, x);

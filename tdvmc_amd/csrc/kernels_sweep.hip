@@ -283,7 +283,7 @@ __device__ __forceinline__ void sweep_body(const KSys& sy, const KTables<T>& tb,
             const int q = on ? e / (D * km) : 0, f = on ? e - q * (D * km) : 0;
             ea[j] = km ? f / km : 0;
             eq[j] = q;
-            const int m = on ? f - ea[j] * km + 1 : 0;   // 0: an idle lane, writes the entry 1 of m = 0
+            const int m = on ? f - ea[j] * km + 1 : 0;   // 0: an idle lane, whose put is left out
             em[j] = (T)m;
             eplus[j] = 2 * (ea[j] * prow + km + m) + q;
             eminus[j] = 2 * (ea[j] * prow + km - m) + q;
@@ -613,9 +613,9 @@ static hipError_t launch_sweep_l(const KSys& sy, const KTables<T>& tb, const Swe
     } else {
         // a term past the lane's last costs what a real one does (31 issue
         // slots of about 450 per trial in the FP32 form): every count has its
-        // kernel, but 7, which no default lane count leads to (258 terms of a
-        // 2-D system with 512 k on 64 lanes, 5 instead of 8: mixed sweep
-        // 35.2 -> 29.6 ms at 131072 walkers, N = 400)
+        // kernel (258 terms of a 2-D system with 512 k on 64 lanes, 5 instead of
+        // 8: mixed sweep 35.2 -> 29.6 ms at 131072 walkers, N = 400), but 7,
+        // which runs in the kernel of 8 with one empty term
         switch (kpl) {
         case 1: return launch_sweep_k<T, D, LPW, 1, PER>(sy, tb, a, st);
         case 2: return launch_sweep_k<T, D, LPW, 2, PER>(sy, tb, a, st);

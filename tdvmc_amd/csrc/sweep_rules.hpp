@@ -56,9 +56,9 @@ __host__ __device__ inline bool sweep_phase_table(const KSys& sy, int lpw)
 // Spline rows of the mixed form 256 bytes apart, in 16 copies: the conversion of
 // r / h to an integer writes it into byte 1 of the row's LDS address, whose
 // other bytes stay (the lane's copy in byte 0, zeros above).  One instruction
-// instead of a conversion and a shift-add, for both distances of a pair's 41
-// issue slots, and no two of the 16 lanes that the LDS serves together share a
-// bank.  Same values, same bits.
+// instead of a conversion and a shift-add, for both distances of a pair's 37
+// vector instructions and 4 LDS reads, and no two of the 16 lanes that the LDS
+// serves together share a bank.  Same values, same bits.
 // Taken where five workgroups fit the LDS of a CU (the registers allow no
 // more); below that the wavefronts it costs take the gain back.  Sweep of
 // 16384 walkers in us, plain and wide: 2-D N = 400, 258 terms, 64 lanes (27 KB)
