@@ -992,18 +992,16 @@ constexpr int kObsShells = 50;
 constexpr int kObsMaxBins = 8192;
 
 // Segments per row of g(r)'s pair loop: enough work items for the workgroup's
-// 256 threads twice, and (fullest) the count whose last round of items and last
-// partner of a segment are fullest (N = 343: 8 segments keep 95 % of the lanes
-// busy, the 2 that 512 items need 89 %).  Not in the mixed form in 3-D, whose reads
-// of the partners decide (N = 142: 4 segments 161 us, 9 173; N = 214: 3 and 7, 137 and
-// 145).
-int gr_segments(int N, bool fullest)
+// 256 threads twice, and the count whose last round of items and last partner of a
+// segment are fullest (N = 343: 8 segments keep 95 % of the lanes busy, the 2 that
+// 512 items need 89 %).
+int gr_segments(int N)
 {
     const int M = N / 2;   // partners of a row
     const int least = std::max(1, std::min(M, (512 + N - 1) / N));
     int best = least;
     double eff = 0.0;
-    for (int s = least; fullest && s <= std::min(M, least + 10); s++) {
+    for (int s = least; s <= std::min(M, least + 10); s++) {
         const double items = (double)N * s;
         const double e = items / (256.0 * std::ceil(items / 256.0)) * M / (s * std::ceil((double)M / s));
         if (e > eff + 0.01) {
@@ -1176,7 +1174,7 @@ int enqueue_obs(tdvmc_ctx* ctx, int prec, const double* dR, int64_t W, double* g
     a.nshell = o.nshell;
     a.nmax = o.nmax;
     a.chunk = chunk;
-    a.gr_segs = gr_segments(N, !f32 || D < 3);
+    a.gr_segs = gr_segments(N);
     a.sk_w = sk_w;
     hipEvent_t ev{};
     int rc = prof_begin(ctx, "observables", &ev);

@@ -146,7 +146,11 @@ __device__ __forceinline__ void obs_walker(const ObsArgs& a, int64_t w, unsigned
     // threads hold consecutive segments of a row: with the same segment of
     // consecutive rows the lanes of a wavefront meet their neighbours at one
     // distance where the particles are in order, and their additions to one bin
-    // wait for each other (1-D, N = 208, 702 walkers 85 us, this way 57).
+    // wait for each other (1-D, N = 208, 702 walkers 85 us, this way 57; 2-D, N = 343,
+    // 4000 walkers 369 and 259).  In the mixed 3-D form, where order matters less, the
+    // reads decide: consecutive rows read consecutive partners, segments of a row
+    // can all start in the same banks (4000 walkers, N = 214 215 us, segments first
+    // 255; N = 343 381 and 389; N = 400 461 and 580).
     {
         const int M = (N - 1) / 2;
         const int even = (N % 2 == 0) ? 1 : 0;
@@ -154,7 +158,9 @@ __device__ __forceinline__ void obs_walker(const ObsArgs& a, int64_t w, unsigned
         const int seg = (M + even + S - 1) / S;
         const float sc = (float)(a.L * (1.0 / 4294967296.0));
         for (int t = tid; t < N * S; t += kObsThreads) {
-            const int i = t / S, sg = t - i * S;
+            constexpr bool ROWS = sizeof(T) == 4 && D == 3;
+            const int hi = t / (ROWS ? N : S), lo = t - hi * (ROWS ? N : S);
+            const int i = ROWS ? lo : hi, sg = ROWS ? hi : lo;
             const int Mi = M + ((even && i < N / 2) ? 1 : 0);
             const int o0 = sg * seg, o1 = min(Mi, o0 + seg);
             int j = i + 1 + o0;
