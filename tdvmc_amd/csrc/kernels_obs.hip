@@ -591,15 +591,19 @@ size_t obs_lds_bytes(int N, int D, int V, int chunk, int nmax, int count, bool f
 // asked for): the pair loop hides the additions to the totals, and the last
 // workgroups leave no CU waiting (N = 343, 16384 walkers: 1774 us, 1960 with 16
 // walkers each; the 1-D FP64 form from N = 100: N = 166, 10615 walkers 452 us, 537
-// shared), and of fewer than 1536 walkers (which wait for the workgroups that have
-// two: N = 7, 1129 walkers 24 us, 28 shared).  Otherwise 1024 workgroups, at most
-// 1024 walkers each (their counts have 32 bits).
-static unsigned obs_grid(int N, int64_t W, bool per_walker, int alone)
+// shared), and of few walkers, which would wait for the workgroups that have
+// two: up to 1024 in FP64 and, for the more registers of its shared kernel, up to
+// 1152 and 1280 in the 2-D and 3-D mixed form.  Shared and single, us: FP64 3-D, N = 8,
+// 1060 walkers 22.8 / 26.4; mixed 1-D, N = 50, 1060 walkers 24.3 / 29.7; 2-D, N = 50,
+// 1060 walkers 28.0 / 27.1, 1200 walkers 27.6 / 29.4; 3-D, N = 24, 1060 walkers 34.0 /
+// 29.0, 1280 walkers 32.8 / 32.1, 1400 walkers 31.2 / 34.1.  Otherwise 1024
+// workgroups, at most 1024 walkers each (their counts have 32 bits).
+static unsigned obs_grid(int N, int64_t W, bool per_walker, int alone, int few)
 {
-    if (per_walker || N >= alone || W < 1536) return (unsigned)W;
+    if (per_walker || N >= alone || W <= few) return (unsigned)W;
     return (unsigned)std::max<int64_t>(1024, (W + 1023) / 1024);
 }
-constexpr int kMfmaAlone = 200;
+constexpr int kMfmaAlone = 200, kMfmaFew = 1024;
 
 // A workgroup of one walker with few pairs spends more on staging the bins'
 // thresholds than its pairs save: N = 12, 1000 bins, 192 walkers 11.7 us without,
@@ -607,7 +611,7 @@ constexpr int kMfmaAlone = 200;
 // bins) are even.
 bool obs_mfma_pays(int N, int count, int64_t W, bool per_walker)
 {
-    return (int64_t)obs_grid(N, W, per_walker, kMfmaAlone) < W || 3LL * N * (N - 1) >= count;
+    return (int64_t)obs_grid(N, W, per_walker, kMfmaAlone, kMfmaFew) < W || 3LL * N * (N - 1) >= count;
 }
 
 size_t obs_mfma_lds_bytes(int N, int D, int chunk, int nmax, int count, int npair)
@@ -622,7 +626,7 @@ size_t obs_mfma_lds_bytes(int N, int D, int chunk, int nmax, int count, int npai
 hipError_t launch_obs_mfma(const ObsArgs& a, int D, size_t lds, hipStream_t st)
 {
     if (a.W <= 0) return hipSuccess;
-    const dim3 grid(obs_grid(a.N, a.W, a.gr_w, kMfmaAlone)), block(kObsThreads);
+    const dim3 grid(obs_grid(a.N, a.W, a.gr_w, kMfmaAlone, kMfmaFew)), block(kObsThreads);
     if (D == 2)
         hipLaunchKernelGGL(obs_mfma_kernel<2>, grid, block, lds, st, a);
     else
@@ -633,7 +637,8 @@ hipError_t launch_obs_mfma(const ObsArgs& a, int D, size_t lds, hipStream_t st)
 template <typename T, int D>
 static void launch_obs_d(const ObsArgs& a, size_t lds, hipStream_t st)
 {
-    const unsigned grid = obs_grid(a.N, a.W, a.gr_w, sizeof(T) == 8 ? 100 : 200);
+    constexpr bool f32 = sizeof(T) == 4;
+    const unsigned grid = obs_grid(a.N, a.W, a.gr_w, f32 ? 200 : 100, f32 ? 1024 + 128 * (D - 1) : 1024);
     if (grid < a.W)
         hipLaunchKernelGGL((obs_kernel<T, D, true>), dim3(grid), dim3(kObsThreads), lds, st, a);
     else
